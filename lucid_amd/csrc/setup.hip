@@ -142,9 +142,16 @@ __device__ void store_tri(const FrameConst &c, const FrameBufs &b, uint32_t t, u
 	b.tri_scan[2 * (size_t)tri_rec(b, t) + 1] = make_uint4(f2bits(step[0]), f2bits(step[1]), f2bits(step[2]), signs);
 }
 
+// Quads that pass the culling tests: corners, cull bits of the two triangles and their pixel
+// row ranges, from which the triangles' records are made.
+struct QuadSetup {
+	V3 p[4];
+	uint32_t cull_flags, y_aabb[2];
+};
+
 // Returns 0 small, 1 large, 2 + rejection type when rejected.
-__device__ int process_quad(const FrameConst &c, const FrameBufs &b, uint32_t q, uint32_t inst,
-							uint32_t flags, const uint32_t vi[4]) {
+__device__ int process_quad(const FrameConst &c, const FrameBufs &b, uint32_t q,
+							const uint32_t vi[4], QuadSetup &qs) {
 	bool cull0 = vi[0] == vi[1] || vi[1] == vi[2] || vi[2] == vi[0];
 	bool cull1 = vi[0] == vi[2] || vi[2] == vi[3] || vi[3] == vi[0];
 	if(cull0 && cull1)
@@ -227,34 +234,51 @@ __device__ int process_quad(const FrameConst &c, const FrameBufs &b, uint32_t q,
 		bb[i] = f2u(box[i]) >> kBinShift;
 	uint32_t enc = encode_aabb28(bb[0], bb[1], bb[2], bb[3]) | (cull_flags << 30);
 	uint32_t area = (bb[2] - bb[0] + 1u) * (bb[3] - bb[1] + 1u);
-	uint32_t y_aabb[2] = {f2u(a0[1]) | (f2u(a0[3]) << 16), f2u(a1[1]) | (f2u(a1[3]) << 16)};
 	b.quad_aabb[q] = enc;
-
-	uint32_t flags_id = flags | (inst << 16);
-	V3 o = ld3(c.origin);
-	const uint32_t vq[4] = {vi[0], vi[1], vi[2], vi[3]};
+	qs.y_aabb[0] = f2u(a0[1]) | (f2u(a0[3]) << 16);
+	qs.y_aabb[1] = f2u(a1[1]) | (f2u(a1[3]) << 16);
+	qs.cull_flags = cull_flags;
 #pragma unroll
-	for(int s = 0; s < 2; s++) {
-		if((cull_flags >> s) & 1u)
-			continue; // no record is read for a culled triangle
-		const uint32_t t = 2 * q + s;
+	for(int i = 0; i < 4; i++)
+		qs.p[i] = p[i];
+	return area <= 4u ? 0 : 1;
+}
+
+// Records of triangle s of the wave's quads (lanes with `have`; q0 is the quad of lane 0), for
+// the whole wave at once. Setup is bound by its record writes (176 bytes per triangle). The
+// 128-byte shading records go through LDS: stored straight from the lanes, each of a record's
+// seven 16-byte stores touches 64 lines per wave, and the unwritten eighth word leaves every
+// line partial; from LDS a store instruction writes eight whole lines, the eighth word zero.
+// 5.2 M triangles (a 2.6 M quad mesh): 338 us stored from the lanes, 356 us staged without the
+// eighth word, 252 us as here (4.2 TB/s); 1 M soup triangles 77 -> 69 us. Staging 32 records at
+// a time (16 KB per work-group) keeps eight work-groups on a CU (all 64: 273 us).
+constexpr int kStageRows = 32;
+
+__device__ __forceinline__ void store_wave_records(const FrameConst &c, const FrameBufs &b,
+												   uint32_t q0, int s, bool have,
+												   const QuadSetup &qs, uint32_t flags,
+												   uint32_t inst, const uint32_t (&vq)[4],
+												   uint4 *s_rec) {
+	const uint64_t mask = ballot(have);
+	if(!mask)
+		return; // no record is read for a culled triangle
+	const int lane = lane_id();
+	const uint32_t t = 2 * (q0 + lane) + s;
+	uint4 rec[kRecQuads];
+	if(have) {
+		const V3 o = ld3(c.origin);
 		uint4 d, b0, b1;
 		uint32_t nrm;
-		store_tri(c, b, t, flags_id, sub3(p[0], o), sub3(p[1 + s], o), sub3(p[2 + s], o),
-				  y_aabb[s], d, b0, b1, nrm);
+		store_tri(c, b, t, flags | (inst << 16), sub3(qs.p[0], o), sub3(s ? qs.p[2] : qs.p[1], o),
+				  sub3(s ? qs.p[3] : qs.p[2], o), s ? qs.y_aabb[1] : qs.y_aabb[0], d, b0, b1, nrm);
 		// shading record: depth and barycentric planes, colours (storeQuad,
 		// quad_setup.glsl:256-272) and lighting, one 128-byte line
-		uint4 rec[kRecQuads];
 		make_shading_record(c, b, t, d, b0, b1, nrm, vq, rec);
-		uint4 *dst = b.tri_shade + (size_t)kRecStride * tri_rec(b, t);
-#pragma unroll
-		for(int j = 0; j < kRecQuads; j++)
-			dst[j] = rec[j];
 		if(c.has_textures && (flags & LUCID_INST_HAS_ALBEDO_TEXTURE)) {
 			// texture coordinates of the triangle's corners, relative to corner 0
 			// (storeQuad, quad_setup.glsl:265-271)
 			const float *tc = b.tex_coords;
-			const uint32_t w0 = vq[0], w1 = vq[1 + s], w2 = vq[2 + s];
+			const uint32_t w0 = vq[0], w1 = s ? vq[2] : vq[1], w2 = s ? vq[3] : vq[2];
 			const float t0x = tc[2 * (size_t)w0], t0y = tc[2 * (size_t)w0 + 1];
 			const float d1x = tc[2 * (size_t)w1] - t0x, d1y = tc[2 * (size_t)w1 + 1] - t0y;
 			const float d2x = tc[2 * (size_t)w2] - t0x, d2y = tc[2 * (size_t)w2 + 1] - t0y;
@@ -263,7 +287,28 @@ __device__ int process_quad(const FrameConst &c, const FrameBufs &b, uint32_t q,
 			tt[1] = make_uint4(f2bits(d2x), f2bits(d2y), 0u, 0u);
 		}
 	}
-	return area <= 4u ? 0 : 1;
+	static_assert(kRecStride == 8, "eight lanes store a record");
+	uint4 *dst = b.tri_shade + (size_t)kRecStride * tri_rec(b, 2 * q0 + s);
+#pragma unroll
+	for(int h = 0; h < 64 / kStageRows; h++) {
+		const int row_l = lane - h * kStageRows;
+		if(have && (uint32_t)row_l < (uint32_t)kStageRows) {
+			// word j of a record at column j ^ (row & 7): no bank conflicts either way
+#pragma unroll
+			for(int j = 0; j < kRecStride; j++)
+				s_rec[row_l * kRecStride + (j ^ (row_l & 7))] =
+					j < kRecQuads ? rec[j < kRecQuads ? j : 0] : make_uint4(0u, 0u, 0u, 0u);
+		}
+		wave_sync_lds();
+#pragma unroll
+		for(int k = 0; k < kStageRows / 8; k++) {
+			const int row = k * 8 + (lane >> 3), col = lane & 7;
+			if((mask >> (h * kStageRows + row)) & 1ull)
+				dst[(h * kStageRows + k * 8) * kRecStride + lane] =
+					s_rec[row * kRecStride + (col ^ (row & 7))];
+		}
+		wave_sync_lds(); // the staging is used again
+	}
 }
 
 // Instance of quad q: the last instance whose first quad (inst_prefix) is at most q
@@ -280,18 +325,38 @@ __device__ __forceinline__ int find_instance(const FrameConst &c, const FrameBuf
 	return lo;
 }
 
+// The same by a whole wave: each step probes 64 positions at once, so that a table of 977
+// instances (1 M quads) takes two dependent loads instead of ten.
+__device__ __forceinline__ int find_instance_wave(const FrameConst &c, const FrameBufs &b, uint32_t q) {
+	int lo = 0, n = c.num_instances; // the answer is one of lo .. lo + n - 1
+	while(n > 1) {
+		const int step = (n + 63) >> 6, at = lane_id() * step;
+		// the prefixes do not decrease: the lanes at or before q are the lowest ones (lane 0
+		// always is: prefix[lo] <= q)
+		const bool le = at < n && (lane_id() == 0 || (uint32_t)b.inst_prefix[lo + at] <= q);
+		const int last = (__popcll(ballot(le)) - 1) * step;
+		lo += last;
+		n = min(step, n - last);
+	}
+	return lo;
+}
+
 __device__ __forceinline__ void setup_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
 	__shared__ uint32_t s_counts[6]; // small, large, rejected x4
 	__shared__ int s_inst[2];         // instances of the work-group's first and last quads
 	__shared__ uint32_t s_prefix[kSetupThreads]; // their prefixes, when they span few instances
+	__shared__ uint4 s_rec[kSetupThreads / 64][kStageRows * kRecStride];
 	if(threadIdx.x < 6)
 		s_counts[threadIdx.x] = 0;
 	const uint32_t q0 = wg.id * (uint32_t)kSetupThreads;
 	const uint32_t nq = (uint32_t)c.num_quads;
-	// the two searches over the whole instance table run once per work-group (one lane of
-	// each of two waves); each quad then searches the few instances of its work-group in LDS
-	if(q0 < nq && (threadIdx.x == 0 || threadIdx.x == 64))
-		s_inst[threadIdx.x >> 6] = find_instance(c, b, threadIdx.x == 0 ? q0 : min(q0 + kSetupThreads - 1, nq - 1));
+	// the two searches over the whole instance table run once per work-group (by one wave
+	// each); each quad then searches the few instances of its work-group in LDS
+	if(q0 < nq && threadIdx.x < 128) {
+		const int i = find_instance_wave(c, b, threadIdx.x < 64 ? q0 : min(q0 + kSetupThreads - 1, nq - 1));
+		if(lane_id() == 0)
+			s_inst[threadIdx.x >> 6] = i;
+	}
 	__syncthreads();
 	const int i0 = q0 < nq ? s_inst[0] : 0, span = q0 < nq ? s_inst[1] - i0 + 1 : 0;
 	const bool local = span <= kSetupThreads;
@@ -300,9 +365,10 @@ __device__ __forceinline__ void setup_kernel_body(const FrameConst &c, const Fra
 	__syncthreads();
 
 	uint32_t q = q0 + threadIdx.x;
-	int kind = -1;
+	int kind = -1, lo = 0;
+	uint32_t vi[4] = {0u, 0u, 0u, 0u}, flags = 0;
+	QuadSetup qs = {};
 	if(q < nq) {
-		int lo;
 		if(local) {
 			int l = 0, h = span - 1;
 			while(l < h) {
@@ -319,14 +385,20 @@ __device__ __forceinline__ void setup_kernel_body(const FrameConst &c, const Fra
 		lucid_instance_data ins = b.instances[lo];
 		uint32_t k = q - (local ? s_prefix[lo - i0] : (uint32_t)b.inst_prefix[lo]);
 		const uint32_t *ix = b.quad_indices + (size_t)ins.index_offset + (size_t)k * 4;
-		uint32_t vi[4];
 #pragma unroll
 		for(int j = 0; j < 4; j++)
 			vi[j] = ix[j] + (uint32_t)ins.vertex_offset;
-		kind = process_quad(c, b, q, (uint32_t)lo, ins.flags, vi);
+		flags = ins.flags;
+		kind = process_quad(c, b, q, vi, qs);
 		if(kind >= 2)
 			b.quad_aabb[q] = kInvalidAabb;
 	}
+	const bool visible = kind == 0 || kind == 1;
+#pragma unroll
+	for(int s = 0; s < 2; s++)
+		store_wave_records(c, b, q0 + (threadIdx.x & ~63u), s,
+						   visible && !((qs.cull_flags >> s) & 1u), qs, flags, (uint32_t)lo, vi,
+						   s_rec[threadIdx.x >> 6]);
 	// wave-aggregated counters and this work-group's large-quad sub-list
 	uint64_t large = ballot(kind == 1);
 	const uint32_t stripe = wg.id % kLargeStripes;

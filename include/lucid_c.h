@@ -204,7 +204,7 @@ int lucid_batch_finish(lucid_batch *b);
  * that forbid hipMalloc). Same kernels, inputs and outputs as lucid_render on a renderer of
  * width x height with `opts` and `tuning` (NULL: the defaults 1, 128, 1024, 1); results are
  * identical to that renderer's. Every internal buffer lives in a fixed device array of the
- * library (65 MiB, one copy per GPU the library runs on, held until the process ends), so the
+ * library (78 MiB, one copy per GPU the library runs on, held until the process ends), so the
  * frame is limited to at most 256 bins of 32 x 32 pixels (e.g. 512 x 512), 65536 quads and
  * 1024 instances (larger: LUCID_ERR_INVALID_ARG), no albedo textures (LUCID_ERR_UNSUPPORTED),
  * and to that array's pools: high bins (1024+ triangles) may hold 131072 triangle

@@ -24,19 +24,17 @@ constexpr int kBlockSize = 8;
 constexpr uint32_t kInvalidAabb = 0xffffffffu;
 constexpr int kLowLevelLimit = 1024; // bin_categorizer.glsl:352
 constexpr int kMaxBlockTris = 256;   // raster_low.glsl:17 (promotion threshold)
-constexpr int kLowRowCap = 1024;     // records per block row of a low bin (< 1024 tris)
 
 // Internal control words (separate from LucidInfo, whose layout is the reference's).
 enum CtrlWord : int {
 	kCtrlRecorded = 0,      // 1: this frame's rasterisation records the backward's pass A
-	kCtrlRecordCursor = 1,  // high-bin record pool size the frame needs (uint4 units)
 	kCtrlFallbackCount = 2, // pixels in the exact-fallback queue
-	kCtrlOverflow = 3,      // bit 0 bin lists, 1 record pool, 2 fallback queue, 3 spill pool
+	kCtrlOverflow = 3,      // kOvf* bits
 	kCtrlSpillCursor = 4,   // bump allocator of the deep-pixel spill pool (u64 units)
 	kCtrlTotalBinQuads = 5,
 	kCtrlTotalBinTris = 6,
 	kCtrlFallbackPixels = 7,
-	kCtrlListCursor = 8,    // high-bin block-list space the frame needs (u32 units)
+	kCtrlListCursor = 8,    // high-bin block-list space the frame needs (entries)
 	kCtrlOverflowCarry = 9, // overflow bits of earlier frames not yet seen by the host
 	kCtrlSortedCursor = 10, // pre-sorted pool size a frame needed, after an overflow (u32 units)
 	kCtrlBwdRows = 11,      // gradient rows of the block kernel (set by the row scan)
@@ -83,8 +81,8 @@ __host__ __device__ constexpr uint32_t large_stripe_cap(uint32_t num_quads) {
 }
 
 // Overflow bits of kCtrlOverflow
-constexpr uint32_t kOvfBinLists = 1u, kOvfRecords = 2u, kOvfFallback = 4u, kOvfSpill = 8u,
-				   kOvfLists = 16u, kOvfSorted = 32u, kOvfGradRows = 64u;
+constexpr uint32_t kOvfBinLists = 1u, kOvfFallback = 4u, kOvfSpill = 8u, kOvfLists = 16u,
+				   kOvfSorted = 32u, kOvfGradRows = 64u;
 
 // Buffers of the backward pass (passed by value beside FrameBufs).
 constexpr int kGradWords = 10; // per row: corner 0 rgb, corner 1 rgb, corner 2 rgb, alpha
@@ -211,17 +209,15 @@ struct FrameBufs {
 	uint32_t *bin_quads, *bin_tris;
 	uint64_t bin_quads_cap, bin_tris_cap;
 	// raster
-	uint4 *low_records;  // bin_count * 4 * kLowRowCap
-	uint4 *high_records; // pool
-	uint64_t high_records_cap;
-	uint4 *blk_slot;     // bin_count * 16: list offset, list length, record offset, record count
+	uint2 *blk_slot;     // bin_count * 16: list offset, list length (entries)
 	uint32_t *blk_flags; // bin_count * 16
 	uint32_t *blk_sorted; // bin_count * 16: offset of the pre-sorted arrays
 	uint32_t *big_queue;  // bin_count * 16: blocks left to high_finalize's long-list pass
-	uint32_t *blk_lists;  // low bins: fixed bin_count * 16 * kRegSortCap; then high bump region
+	// block lists, one entry {triangle, depth key, pixel mask (2 words)} per (block, triangle):
+	// low bins take a fixed bin_count * 16 * kRegSortCap, then the high bins' bump region
+	uint4 *blk_lists;
 	uint64_t blk_lists_cap;
 	uint32_t *blk_count;  // bin_count * 16: list lengths of high bins (atomic counters)
-	uint32_t *band_count; // bin_count * 4: record counts of high-bin bands (atomic counters)
 	uint32_t *sorted_pool;
 	uint64_t sorted_cap;
 	uint4 *fallback_queue; // one {slot, px, py, whole} per pixel
@@ -537,37 +533,24 @@ __device__ __forceinline__ uint32_t row_scan_step(RowScan &s) {
 	return (uint32_t)a | ((uint32_t)b << 5);
 }
 
-__device__ __forceinline__ uint32_t span_bx_mask(uint32_t span) {
-	uint32_t a = span & 31u, b = (span >> 5) & 31u;
-	return ((15u << (a >> 3)) & (15u >> (3u - (b >> 3)))) & 15u;
+// The pixels of a row span in the 32 columns of its bin (none for the empty span (31, 0)).
+__device__ __forceinline__ uint32_t span_bits(uint32_t span) {
+	return (~0u >> (~(span >> 5) & 31u)) & (~0u << (span & 31u));
 }
 
-// Block-row record: 8 row spans (10 bits each) of one triangle in one 8-row band.
-//   x = triangle id, y = rows 0-2, z = rows 3-5, w = rows 6-7 | bx_mask << 20
-__device__ __forceinline__ uint32_t record_span(uint4 rec, int row) {
-	uint32_t w = row < 3 ? rec.y : row < 6 ? rec.z : rec.w;
-	int sh = (row < 3 ? row : row < 6 ? row - 3 : row - 6) * 10;
-	return (w >> sh) & 0x3ffu;
+// Pixel mask of block column bx over four rows (8 bits per row) from their spans (16 bits each).
+__device__ __forceinline__ uint32_t group_mask(uint2 spans, uint32_t bx) {
+	// v_perm_b32: byte 0 from the low operand's byte bx, byte 1 from the high operand's
+	const uint32_t sel = 0x0c0c0400u + bx * 0x0101u;
+	const uint32_t r01 = __builtin_amdgcn_perm(span_bits(spans.x >> 16), span_bits(spans.x), sel);
+	const uint32_t r23 = __builtin_amdgcn_perm(span_bits(spans.y >> 16), span_bits(spans.y), sel);
+	return r01 | (r23 << 16);
 }
 
-__device__ __forceinline__ uint32_t record_bx_mask(uint4 rec) { return (rec.w >> 20) & 15u; }
-
-// 64-bit coverage mask of block column bx (bit y*8 + x) from a record.
-__device__ __forceinline__ uint64_t record_block_mask(uint4 rec, int bx) {
-	uint64_t m = 0;
-	int x0 = bx * 8;
-#pragma unroll
-	for(int r = 0; r < 8; r++) {
-		uint32_t sp = record_span(rec, r);
-		int a = (int)(sp & 31u) - x0, b = (int)((sp >> 5) & 31u) - x0;
-		a = a < 0 ? 0 : a;
-		b = b > 7 ? 7 : b;
-		if(b >= a) {
-			uint32_t bits = ((1u << (b - a + 1)) - 1u) << a;
-			m |= (uint64_t)bits << (r * 8);
-		}
-	}
-	return m;
+// Which of the four bytes of x are not zero, as four bits.
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t x) {
+	const uint32_t top = (((x & 0x7f7f7f7fu) + 0x7f7f7f7fu) | x) & 0x80808080u;
+	return ((top >> 7) * 0x10204080u) >> 28;
 }
 
 // ------------------------------------------------------------------ shading records

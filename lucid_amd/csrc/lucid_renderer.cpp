@@ -106,8 +106,8 @@ struct lucid_renderer {
 	DevBuf tri_tex;            // texture coordinates per triangle, once a frame is textured
 	bool tex_enabled = false;
 	DevBuf wg_hist, bin_quads, bin_tris;
-	DevBuf low_records, high_records, fallback_queue, spill;
-	DevBuf blk_slot, blk_flags, blk_sorted, blk_lists, blk_count, band_count, sorted_pool;
+	DevBuf fallback_queue, spill;
+	DevBuf blk_slot, blk_flags, blk_sorted, blk_lists, blk_count, sorted_pool;
 	// backward
 	DevBuf grad_row_base, grad_range_base, grad_rows, grad_row_tri, grad_start, grad_seq,
 		red_counts, red_offsets, red_grouped, tri_grad, red_temp;
@@ -135,7 +135,7 @@ struct lucid_renderer {
 	} retained;
 
 	int64_t quad_cap = 0;
-	uint64_t bin_quads_cap = 0, bin_tris_cap = 0, high_records_cap = 0, spill_cap = 0;
+	uint64_t bin_quads_cap = 0, bin_tris_cap = 0, spill_cap = 0;
 	uint64_t blk_lists_cap = 0, sorted_cap = 0;
 	uint32_t fallback_cap = 0;
 
@@ -227,12 +227,6 @@ int grow_after_overflow(lucid_renderer *r) {
 		LUCID_CHECK(r->bin_tris.reserve(need * 4));
 		r->bin_tris_cap = need;
 	}
-	if(flags & kOvfRecords) {
-		uint64_t need = std::max<uint64_t>((uint64_t)r->status[kCtrlRecordCursor],
-										   r->high_records_cap * 2);
-		LUCID_CHECK(r->high_records.reserve(need * 16));
-		r->high_records_cap = need;
-	}
 	if(flags & kOvfSpill) {
 		uint64_t need = std::max<uint64_t>((uint64_t)r->status[kCtrlSpillCursor], r->spill_cap * 2);
 		LUCID_CHECK(r->spill.reserve(need * 8));
@@ -241,8 +235,8 @@ int grow_after_overflow(lucid_renderer *r) {
 	if(flags & kOvfLists) {
 		uint64_t low = (uint64_t)r->bin_count * 16 * kRegSortCap;
 		uint64_t need = std::max<uint64_t>(low + (uint64_t)r->status[kCtrlListCursor],
-										   r->blk_lists_cap * 2);
-		LUCID_CHECK(r->blk_lists.reserve(need * 4));
+										   r->blk_lists_cap * 5 / 4);
+		LUCID_CHECK(r->blk_lists.reserve(need * 16));
 		r->blk_lists_cap = need;
 	}
 	if(flags & kOvfSorted) {
@@ -366,21 +360,17 @@ int lucid_create(const lucid_create_info *ci, lucid_renderer **out) {
 	chk(r->info.reserve(((size_t)LUCID_INFO_U32_SIZE + 10 * (size_t)NB) * 4));
 	chk(r->ctrl.reserve(kCtrlAllocWords * 4));
 	chk(r->wg_hist.reserve((size_t)kNumBinWgs * 2 * NB * 4));
-	chk(r->low_records.reserve((size_t)NB * 4 * kLowRowCap * 16));
 	// one 16-byte item per pixel sent to the exact sort; grows after an overflow
 	r->fallback_cap = (uint32_t)NB * 16 * 8;
 	chk(r->fallback_queue.reserve((size_t)r->fallback_cap * 16));
-	r->high_records_cap = 1u << 22;
-	chk(r->high_records.reserve(r->high_records_cap * 16));
 	r->spill_cap = 1u << 20;
 	chk(r->spill.reserve(r->spill_cap * 8));
-	chk(r->blk_slot.reserve((size_t)NB * 16 * 16));
+	chk(r->blk_slot.reserve((size_t)NB * 16 * 8));
 	chk(r->blk_flags.reserve((size_t)NB * 16 * 4));
 	chk(r->blk_sorted.reserve((size_t)NB * 16 * 4 * 2)); // then the long-list queue
 	chk(r->blk_count.reserve((size_t)NB * 16 * 4));
-	chk(r->band_count.reserve((size_t)NB * 4 * 4));
 	r->blk_lists_cap = (uint64_t)NB * 16 * kRegSortCap + (1u << 22);
-	chk(r->blk_lists.reserve(r->blk_lists_cap * 4));
+	chk(r->blk_lists.reserve(r->blk_lists_cap * 16));
 	r->sorted_cap = 1u << 22;
 	chk(r->sorted_pool.reserve(r->sorted_cap * 4));
 	chk(hipHostMalloc((void **)&r->status, kCtrlWords * 4, hipHostMallocDefault));
@@ -622,21 +612,17 @@ int prepare_frame(lucid_renderer *r, const lucid_frame_inputs *in, const lucid_f
 	b.bin_tris = r->bin_tris.as<uint32_t>();
 	b.bin_quads_cap = r->bin_quads_cap;
 	b.bin_tris_cap = r->bin_tris_cap;
-	b.low_records = r->low_records.as<uint4>();
-	b.high_records = r->high_records.as<uint4>();
-	b.high_records_cap = r->high_records_cap;
 	b.fallback_queue = r->fallback_queue.as<uint4>();
 	b.fallback_cap = r->fallback_cap;
 	b.spill = r->spill.as<uint64_t>();
 	b.spill_cap = r->spill_cap;
-	b.blk_slot = r->blk_slot.as<uint4>();
+	b.blk_slot = r->blk_slot.as<uint2>();
 	b.blk_flags = r->blk_flags.as<uint32_t>();
 	b.blk_sorted = r->blk_sorted.as<uint32_t>();
 	b.big_queue = b.blk_sorted + (size_t)r->bin_count * 16;
-	b.blk_lists = r->blk_lists.as<uint32_t>();
+	b.blk_lists = r->blk_lists.as<uint4>();
 	b.blk_lists_cap = r->blk_lists_cap;
 	b.blk_count = r->blk_count.as<uint32_t>();
-	b.band_count = r->band_count.as<uint32_t>();
 	b.sorted_pool = r->sorted_pool.as<uint32_t>();
 	b.sorted_cap = r->sorted_cap;
 	b.image = out ? out->image_rgba8 : nullptr;
@@ -1294,8 +1280,7 @@ namespace {
 constexpr int kNaMaxBins = 256;                        // e.g. 512 x 512 or 1024 x 256 pixels
 constexpr int64_t kNaMaxQuads = (int64_t)1 << 16;
 constexpr int kNaMaxInstances = 1024;
-constexpr uint64_t kNaHighRecords = (uint64_t)1 << 19; // uint4 records of high bins
-constexpr uint64_t kNaListsExtra = (uint64_t)1 << 21;  // u32 list entries of high bins
+constexpr uint64_t kNaListsExtra = (uint64_t)1 << 21;  // list entries of high bins
 constexpr uint64_t kNaSorted = (uint64_t)1 << 19;      // u32 words of pre-sorted blocks
 constexpr uint64_t kNaSpill = (uint64_t)1 << 17;       // u64 keys of deep pixels
 constexpr uint32_t kNaFallback = (uint32_t)kNaMaxBins * 16 * 8; // pixels queued for the exact sort
@@ -1305,9 +1290,8 @@ constexpr int kNaMaxDevices = 64;
 
 struct NaLayout {
 	size_t info, ctrl, instances, inst_prefix, inst_colors, quad_aabb, tri_scan, tri_depth,
-		tri_shade, large_list, wg_hist, bin_quads, bin_tris, low_records, high_records, fallback,
-		spill, blk_slot, blk_flags, blk_sorted, blk_lists, blk_count, band_count, sorted_pool,
-		total;
+		tri_shade, large_list, wg_hist, bin_quads, bin_tris, fallback, spill, blk_slot, blk_flags,
+		blk_sorted, blk_lists, blk_count, sorted_pool, total;
 };
 
 // Byte offsets of the frame's buffers in `scratch` (each 256-byte aligned), sized as
@@ -1318,9 +1302,9 @@ constexpr NaLayout na_layout() {
 	const size_t nb = kNaMaxBins, q = (size_t)kNaMaxQuads, t = 2 * q;
 	size_t *fields[] = {&l.info,      &l.ctrl,         &l.instances,  &l.inst_prefix, &l.inst_colors,
 						&l.quad_aabb, &l.tri_scan,     &l.tri_depth,  &l.tri_shade,   &l.large_list,
-						&l.wg_hist,   &l.bin_quads,    &l.bin_tris,   &l.low_records, &l.high_records,
-						&l.fallback,  &l.spill,        &l.blk_slot,   &l.blk_flags,   &l.blk_sorted,
-						&l.blk_lists, &l.blk_count,    &l.band_count, &l.sorted_pool};
+						&l.wg_hist,   &l.bin_quads,    &l.bin_tris,   &l.fallback,    &l.spill,
+						&l.blk_slot,  &l.blk_flags,    &l.blk_sorted, &l.blk_lists,   &l.blk_count,
+						&l.sorted_pool};
 	const size_t bytes[] = {
 		((size_t)LUCID_INFO_U32_SIZE + 10 * nb) * 4,
 		(size_t)kCtrlAllocWords * 4,
@@ -1335,16 +1319,13 @@ constexpr NaLayout na_layout() {
 		(size_t)kNumBinWgs * 2 * nb * 4,
 		kNaBinQuads * 4,
 		kNaBinTris * 4,
-		nb * 4 * kLowRowCap * 16,
-		kNaHighRecords * 16,
 		(size_t)kNaFallback * 16,
 		kNaSpill * 8,
-		nb * 16 * 16,
+		nb * 16 * 8,
 		nb * 16 * 4,
 		nb * 16 * 4 * 2, // blk_sorted, then the long-list queue
-		(nb * 16 * kRegSortCap + kNaListsExtra) * 4,
+		(nb * 16 * kRegSortCap + kNaListsExtra) * 16,
 		nb * 16 * 4,
-		nb * 4 * 4,
 		kNaSorted * 4,
 	};
 	static_assert(sizeof(fields) / sizeof(fields[0]) == sizeof(bytes) / sizeof(bytes[0]),
@@ -1358,7 +1339,7 @@ constexpr NaLayout na_layout() {
 }
 
 constexpr NaLayout kNaLayout = na_layout();
-static_assert(kNaLayout.total <= ((size_t)72 << 20), "the allocation-free scratch stays modest");
+static_assert(kNaLayout.total <= ((size_t)80 << 20), "the allocation-free scratch stays modest");
 
 } // namespace
 
@@ -1453,21 +1434,17 @@ int lucid_render_noalloc(int width, int height, uint32_t opts, const lucid_tunin
 	b.bin_tris = (uint32_t *)(base + L.bin_tris);
 	b.bin_quads_cap = kNaBinQuads;
 	b.bin_tris_cap = kNaBinTris;
-	b.low_records = (uint4 *)(base + L.low_records);
-	b.high_records = (uint4 *)(base + L.high_records);
-	b.high_records_cap = kNaHighRecords;
 	b.fallback_queue = (uint4 *)(base + L.fallback);
 	b.fallback_cap = kNaFallback;
 	b.spill = (uint64_t *)(base + L.spill);
 	b.spill_cap = kNaSpill;
-	b.blk_slot = (uint4 *)(base + L.blk_slot);
+	b.blk_slot = (uint2 *)(base + L.blk_slot);
 	b.blk_flags = (uint32_t *)(base + L.blk_flags);
 	b.blk_sorted = (uint32_t *)(base + L.blk_sorted);
 	b.big_queue = b.blk_sorted + (size_t)kNaMaxBins * 16;
-	b.blk_lists = (uint32_t *)(base + L.blk_lists);
+	b.blk_lists = (uint4 *)(base + L.blk_lists);
 	b.blk_lists_cap = (uint64_t)kNaMaxBins * 16 * kRegSortCap + kNaListsExtra;
 	b.blk_count = (uint32_t *)(base + L.blk_count);
-	b.band_count = (uint32_t *)(base + L.band_count);
 	b.sorted_pool = (uint32_t *)(base + L.sorted_pool);
 	b.sorted_cap = kNaSorted;
 	b.image = out->image_rgba8;

@@ -2,15 +2,14 @@
 // (≙ data/shaders/raster_low.glsl, raster_high.glsl, shared/raster.glsl, shared/shading.glsl).
 //
 // Kernels (wave64; an 8x8 block of pixels is one wave, one lane per pixel):
-//   rowgen_low   one work-group per bin with fewer than 1024 triangles: block-row records with
-//                the reference's 8-row scanline rule and per-block index lists; promotes the bin
-//                to the high path when an 8x8 block holds more than 256 triangles
-//                (raster_low.glsl:39-106,229-237).
-//   rowgen_high  one work-group per (high bin, 8-row band) with the 4-row rule of
+//   rowgen_low   one work-group per bin with fewer than 1024 triangles: block lists with the
+//                reference's 8-row scanline rule; promotes the bin to the high path when an 8x8
+//                block holds more than 256 triangles (raster_low.glsl:39-106,229-237).
+//   rowgen_high  eight work-groups per high bin: block lists with the 4-row rule of
 //                raster_high.glsl:54-90.
-//   high_prep / high_finalize  allocation for high bins; blocks with more than 256 triangles
-//                are sorted by centroid depth (LDS bitonic, whole work-group) and split into
-//                pixel-row parts so that several waves share a dense block.
+//   high_prep / high_finalize  allocation for high bins; long block lists are sorted by
+//                centroid depth (LDS bitonic, whole work-group) and split into depth ranges so
+//                that several waves share a dense block.
 //   block_raster one wave per block: sorts short lists itself in registers, expands coverage
 //                masks into dense 64-sample chunks, shades, routes samples to pixel lanes and
 //                blends front to back (block_raster_big: one wave per part of a sorted block).
@@ -741,31 +740,33 @@ __device__ __forceinline__ uint32_t next_pow2(uint32_t x) {
 	return x <= 1 ? 1u : 1u << (32 - __clz(x - 1));
 }
 
-// ------------------------------------------------------------------ records and keys
+// ------------------------------------------------------------------ block entries and keys
 
-__device__ __forceinline__ uint4 make_record(uint32_t t, const uint32_t sp[8], uint32_t bxm) {
-	return make_uint4(t, sp[0] | (sp[1] << 10) | (sp[2] << 20), sp[3] | (sp[4] << 10) | (sp[5] << 20),
-					  sp[6] | (sp[7] << 10) | (bxm << 20));
+// A block list entry {triangle, depth key, pixel mask}: everything the sorts and walks need
+// to know of a (block, triangle) pair, in list order, so that they read whole lists with
+// coalesced loads and gather nothing.
+__device__ __forceinline__ uint64_t entry_mask(uint4 e) {
+	return ((uint64_t)e.w << 32) | e.z;
 }
 
-// Inverse depth of triangle t inside a block at the centroid of its covered pixels, from
-// its pixel mask m (bit 8 r + c: row r, column c of the block whose corner pixel is
-// (px0, py0)): the block-level sort key (ties and centroid error are resolved exactly per
-// pixel later). The column and row sums are integers, taken bit by bit with masked
+// Block-level depth key ~ord(inverse depth) of a triangle (depth plane d) inside a block at
+// the centroid of its covered pixels, from its pixel mask m (bit 8 r + c: row r, column c of
+// the block whose corner pixel is (px0, py0)); ties and centroid error are resolved exactly
+// per pixel later. The column and row sums are integers, taken bit by bit with masked
 // popcounts: the sum of the columns is sum_k 2^k popcount(m & pixels whose column has bit
-// k), likewise for the rows.
-__device__ __forceinline__ float mask_inv_depth(const FrameBufs &b, uint32_t t, uint64_t m,
-												int px0, int py0) {
+// k), likewise for the rows. s_inv[n] = 1 / n.
+__device__ __forceinline__ uint32_t mask_depth_key(uint4 d, uint64_t m, int px0, int py0,
+												   const float *s_inv) {
 	auto pc = [](uint64_t x) { return (int)__popcll(x); };
 	const int n = pc(m);
 	const int sc = pc(m & 0xAAAAAAAAAAAAAAAAull) + 2 * pc(m & 0xCCCCCCCCCCCCCCCCull) +
 				   4 * pc(m & 0xF0F0F0F0F0F0F0F0ull);
 	const int sr = pc(m & 0xFF00FF00FF00FF00ull) + 2 * pc(m & 0xFFFF0000FFFF0000ull) +
 				   4 * pc(m & 0xFFFFFFFF00000000ull);
-	const float inv_n = 1.0f / (float)(n > 0 ? n : 1);
-	const float cx = (float)px0 + (float)(2 * sc) * 0.5f * inv_n;
+	const float inv_n = s_inv[n];
+	const float cx = (float)px0 + (float)sc * inv_n;
 	const float cy = (float)py0 + (float)sr * inv_n;
-	return sample_inv_depth(b, t, cx, cy);
+	return inv_ord_f32(bits2f(d.x) * cx + (bits2f(d.y) * cy + bits2f(d.z)));
 }
 
 // Depth rank of a block entry from its depth key ~ord(inverse depth) (ascending = nearest
@@ -799,30 +800,26 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 
 // Depth order of a block list of m <= 256 entries, sorted by one wave in registers: sorted
 // entry 64 k + lane is list position pos[k]. Keys are (24-bit depth rank << 8 | position).
-// With s_msk / s_tri (LDS, kRegSortCap entries each, or null), each entry's pixel mask and
-// triangle id are also left there at its list position, for the caller to read in sorted
-// order (after a wave_sync_lds) instead of gathering the records again.
-__device__ __forceinline__ void sort_block_positions(const FrameBufs &b, const uint4 *recs,
-													 const uint32_t *list, uint32_t m, int bx,
-													 int px0, int py0, uint32_t (&pos)[4],
-													 uint64_t *s_msk = nullptr,
-													 uint32_t *s_tri = nullptr) {
+// Each entry's pixel mask and triangle id are left in s_msk / s_tri (LDS, kRegSortCap entries
+// each) at its list position, for the caller to read in sorted order after a wave_sync_lds.
+__device__ __forceinline__ void sort_block_positions(const uint4 *list, uint32_t m,
+													 uint32_t (&pos)[4], uint64_t *s_msk,
+													 uint32_t *s_tri) {
 	static_assert(kRegSortCap <= 256, "list positions fit 8 bits of the key");
 	const int lane = lane_id();
 	uint32_t dk[4];
 	uint32_t lo = ~0u, hi = 0u;
+	uint4 e[4];
+#pragma unroll
+	for(int k = 0; k < 4; k++)
+		e[k] = k * 64 + lane < (int)m ? list[k * 64 + lane] : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
 	for(int k = 0; k < 4; k++) {
 		const uint32_t j = k * 64 + lane;
-		dk[k] = 0u;
+		dk[k] = e[k].y;
 		if(j < m) {
-			const uint4 rec = recs[list[j]];
-			const uint64_t msk = record_block_mask(rec, bx);
-			if(s_msk) {
-				s_msk[j] = msk;
-				s_tri[j] = rec.x;
-			}
-			dk[k] = inv_ord_f32(mask_inv_depth(b, rec.x, msk, px0, py0));
+			s_msk[j] = entry_mask(e[k]);
+			s_tri[j] = e[k].x;
 			lo = min(lo, dk[k]);
 			hi = max(hi, dk[k]);
 		}
@@ -904,14 +901,146 @@ __device__ __forceinline__ void enqueue_pixels(const FrameBufs &b, uint32_t slot
 	}
 }
 
+// ------------------------------------------------------------------ row generation
+//
+// Both row generators hand their live triangles to waves 64 at a time (sorted by height, so
+// that the lanes of a wave scan about as many rows); rowgen_wave scans them and writes their
+// block entries. A lane scans its triangle's rows in one loop, four rows (a group) per step,
+// and leaves the row spans in LDS. The wave then lists its (block, triangle) pairs block by
+// block, reserves each block's list positions with one atomic instruction, and makes the
+// entries with one pair per lane: the pixel mask from the spans, the depth key from the mask
+// and the depth plane. All lanes are busy there (a triangle covers a few of a bin's 16 blocks),
+// and neighbouring lanes write neighbouring entries of a list.
+//
+// Both are bound by the latency of their gathers (VALU about half busy), so the staging is
+// kept small: 25 KB per work-group of four waves. Masks instead of spans in LDS (46 KB) saved a
+// third of the VALU work and was slower (5.2 M mesh triangles: 348 us against 270), as was
+// loading the next triangles' records ahead (304). Writing whole entries here instead of row
+// records and index lists takes the two dependent gathers per entry out of the sorts and walks
+// (before -> after): mesh rowgen_high 350 -> 270, high_finalize 406 -> 274 us; 1 M soup
+// triangles 131 -> 116 and 139 -> 113 us, rowgen_low 23 -> 30 us with the register-sorted
+// blocks' walk 60 -> 54 us.
+
+// Staging of one wave.
+struct RowgenWave {
+	uint2 rows[64][8];      // spans of a lane's row groups, group g at g ^ (lane / 2 % 8)
+	uint16_t pair[64 * 16]; // lane | block << 6
+	uint32_t base[16];      // per block: list entry of pair p of the block, minus p
+};
+// A work-group's LDS: its sorted triangles (each thread takes its up to kRowgenRound of them
+// into registers first), then the waves' staging.
+constexpr int kRowgenRound = 1024; // list entries per sorting round
+template <int THREADS> union RowgenLds {
+	uint32_t sorted[kRowgenRound];
+	RowgenWave wave[THREADS / 64];
+};
+// rowgen_low's work-group: a low bin's triangles are few, so a single frame's bins take twice
+// the waves (each then scans one or two chunks); a batch has bins enough to fill the chip and
+// keeps to the smaller groups. 1280 x 720 lit mesh frame 26.2 -> 23.6 us with 512 threads, the
+// 32-frame batch 240 us with 256 and 271 us with 512.
+constexpr int kRowgenLowThreads = 512, kRowgenLowThreadsBatch = 256;
+
+// What a lane scans: a triangle (~0: none), its scan parameters and depth plane.
+struct ScanTri {
+	uint32_t t;
+	uint4 s0, s1, depth;
+};
+__device__ __forceinline__ ScanTri load_scan_tri(const FrameBufs &b, uint32_t t) {
+	ScanTri tr;
+	tr.t = t;
+	tr.s0 = tr.s1 = tr.depth = make_uint4(0u, 0u, 0u, 0u);
+	if(t != 0xffffffffu) {
+		const size_t i = tri_rec(b, t);
+		tr.s0 = b.tri_scan[2 * i], tr.s1 = b.tri_scan[2 * i + 1], tr.depth = b.tri_depth[i];
+	}
+	return tr;
+}
+
+// Scans the lanes' triangles from row group g0 to g1 of the bin at
+// (bin_x, bin_y) and appends their entries to the bin's 16 block lists. `first` is the list
+// offset of block `lane` (lanes 0-15), `reserve(n)` takes n positions of the list of block
+// `lane` and returns the first; positions from `cap` on are not written (lists of a low bin
+// that will be promoted).
+template <class Reserve>
+__device__ __forceinline__ void rowgen_wave(const FrameBufs &b, RowgenWave &w, const float *s_inv,
+											int bin_x, int bin_y, const ScanTri &tr, int g0, int g1,
+											uint32_t first, uint32_t cap, Reserve &&reserve) {
+	const int lane = lane_id();
+	uint32_t cols = 0; // blocks the triangle covers, one bit each
+	const uint4 d = tr.depth;
+	const uint32_t t = tr.t;
+	if(t != 0xffffffffu) {
+		RowScan rs;
+		row_scan_init(rs, tr.s0, tr.s1, (float)bin_x, (float)(bin_y + g0 * 4));
+		uint2 *rows = w.rows[lane];
+		const int sw = (lane >> 1) & 7;
+		const uint2 empty = make_uint2(kBinMask | (kBinMask << 16), kBinMask | (kBinMask << 16));
+		if(g0 & 1) // the other half of the first and the last 8-row band
+			rows[(g0 - 1) ^ sw] = empty;
+		if(!(g1 & 1))
+			rows[(g1 + 1) ^ sw] = empty;
+		for(int g = g0; g <= g1; g++) {
+			uint32_t v[4], any = 0;
+#pragma unroll
+			for(int r = 0; r < 4; r++) {
+				v[r] = row_scan_step(rs);
+				any |= span_bits(v[r]);
+			}
+			rows[g ^ sw] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+			cols |= nonzero_bytes(any) << (4 * (g >> 1));
+		}
+	}
+	const uint64_t below = (1ull << lane) - 1ull;
+	const uint32_t first0 = __builtin_amdgcn_readfirstlane(first);
+	uint32_t run = 0, off = 0, num = 0;
+#pragma unroll
+	for(int k = 0; k < 16; k++) {
+		const bool mine = (cols >> k) & 1u;
+		const uint64_t sel = ballot(mine);
+		if(mine)
+			w.pair[run + (uint32_t)__popcll(sel & below)] = (uint16_t)(lane | (k << 6));
+		const uint32_t n = (uint32_t)__popcll(sel);
+		if(lane == k)
+			off = run, num = n;
+		run += n;
+	}
+	if(lane < 16)
+		w.base[lane] = first + (num ? reserve(num) : 0u) - off;
+	wave_sync_lds();
+	for(uint32_t p0 = 0; p0 < run; p0 += 64) {
+		// (the whole wave stays in the loop: the planes come from the lanes' registers)
+		const uint32_t p = p0 + lane, pr = p < run ? w.pair[p] : 0u;
+		const uint32_t l = pr & 63u, k = pr >> 6, by = k >> 2, bx = k & 3u;
+		const uint32_t idx = w.base[k] + p;
+		const uint32_t sw = (l >> 1) & 7u;
+		const uint32_t lo = group_mask(w.rows[l][(2 * by) ^ sw], bx);
+		const uint32_t hi = group_mask(w.rows[l][(2 * by + 1) ^ sw], bx);
+		const uint4 dl = make_uint4(__shfl(d.x, (int)l, 64), __shfl(d.y, (int)l, 64),
+									__shfl(d.z, (int)l, 64), 0u);
+		const uint32_t tl = __shfl(t, (int)l, 64);
+		const uint64_t m = ((uint64_t)hi << 32) | lo;
+		const uint32_t key =
+			mask_depth_key(dl, m, bin_x + (int)bx * 8, bin_y + (int)by * 8, s_inv);
+		if(p < run && (cap == ~0u || idx - (first0 + k * cap) < cap))
+			b.blk_lists[idx] = make_uint4(tl, key, lo, hi);
+	}
+	wave_sync_lds(); // the staging is used again
+}
+
+__device__ __forceinline__ void fill_inverses(float *s_inv) { // s_inv[n] = 1 / n, n <= 64
+	if(threadIdx.x <= 64)
+		s_inv[threadIdx.x] = 1.0f / (float)(threadIdx.x > 0 ? threadIdx.x : 1);
+}
+
 // ------------------------------------------------------------------ rowgen_low
 
+template <int THREADS>
 __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
-		return;
 	const int bin = wg.id;
+	const uint32_t overflow = b.ctrl[kCtrlOverflow]; // loaded beside the bin's counts
 	const BinInfo bi = load_bin(c, b, bin);
-	uint4 *slots = b.blk_slot + (size_t)bin * 16;
+	if(overflow & kOvfBinLists)
+		return;
 	uint32_t *flags = b.blk_flags + (size_t)bin * 16;
 	if(bi.nlevel == 0) {
 		if(threadIdx.x < 16)
@@ -921,36 +1050,36 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 	if(bi.nlevel >= (uint32_t)kLowLevelLimit)
 		return; // rowgen_high writes this bin's slots
 
-	__shared__ uint32_t s_row_n[4];
+	constexpr int kChunks = kRowgenRound / THREADS; // list positions per thread
+	__shared__ RowgenLds<THREADS> s;
+	__shared__ float s_inv[65];
 	__shared__ uint32_t s_blk_n[16];
+	// The bin's live triangles (its list has fewer than kLowLevelLimit entries: one position
+	// per thread and chunk) are counting-sorted by their number of 8-row bands, so that the
+	// waves' row loops run about as long as each of their triangles needs.
+	static_assert(kLowLevelLimit <= kRowgenRound, "a low bin's list in one round");
+	__shared__ uint32_t s_nb[4], s_nb_off[4], s_nlive;
+	fill_inverses(s_inv);
 	if(threadIdx.x < 16)
 		s_blk_n[threadIdx.x] = 0;
 	if(threadIdx.x < 4)
-		s_row_n[threadIdx.x] = 0;
-	__syncthreads();
-
-	uint4 *recs = b.low_records + (size_t)bin * 4 * kLowRowCap;
-	uint32_t *lists = b.blk_lists + (size_t)bin * 16 * kRegSortCap;
-	// The bin's live triangles (its list has fewer than kLowLevelLimit entries: one position
-	// per thread and chunk) are counting-sorted by their number of 8-row bands, so that the
-	// waves' band loops run about as long as each of their triangles needs.
-	static_assert(kLowLevelLimit <= 4 * kRowgenThreads, "a low bin's list in one round");
-	__shared__ uint32_t s_sorted[kLowLevelLimit];
-	__shared__ uint32_t s_nb[4], s_nb_off[4], s_nlive;
-	if(threadIdx.x < 4)
 		s_nb[threadIdx.x] = 0;
 	__syncthreads();
-	uint32_t tk[4];
-	int hk[4];
+	uint32_t tk[kChunks];
+	int hk[kChunks];
+	// first and last 8-row band of a triangle in this bin, from its row range
+	auto bands = [&](uint32_t yr, int &lo_by, int &hi_by) {
+		lo_by = min(max((int)(yr & 0xffffu) - bi.bin_y, 0), kBinMask) >> 3;
+		hi_by = min(max((int)(yr >> 16) - bi.bin_y, 0), kBinMask) >> 3;
+	};
 #pragma unroll
-	for(int k = 0; k < 4; k++) {
-		const uint32_t i = k * kRowgenThreads + threadIdx.x;
+	for(int k = 0; k < kChunks; k++) {
+		const uint32_t i = k * THREADS + threadIdx.x;
 		const uint32_t t = i < bi.nlevel ? bin_tri_at(b, i, bi.qc, bi.qo, bi.to) : 0xffffffffu;
 		int h = -1;
 		if(t != 0xffffffffu) {
-			const uint32_t yr = b.tri_scan[2 * (size_t)tri_rec(b, t)].w;
-			const int lo_by = min(max((int)(yr & 0xffffu) - bi.bin_y, 0), kBinMask) >> 3;
-			const int hi_by = min(max((int)(yr >> 16) - bi.bin_y, 0), kBinMask) >> 3;
+			int lo_by, hi_by;
+			bands(b.tri_scan[2 * (size_t)tri_rec(b, t)].w, lo_by, hi_by);
 			h = hi_by > lo_by ? hi_by - lo_by : 0;
 			atomicAdd(&s_nb[h], 1u);
 		}
@@ -965,37 +1094,25 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 	}
 	__syncthreads();
 #pragma unroll
-	for(int k = 0; k < 4; k++)
+	for(int k = 0; k < kChunks; k++)
 		if(hk[k] >= 0)
-			s_sorted[atomicAdd(&s_nb_off[hk[k]], 1u)] = tk[k];
+			s.sorted[atomicAdd(&s_nb_off[hk[k]], 1u)] = tk[k];
 	__syncthreads();
 	const uint32_t nlive = s_nlive;
-	// block-row records, 8-row rule (raster_low.glsl:39-79), one live triangle per lane
-	for(uint32_t q = threadIdx.x; q < nlive; q += kRowgenThreads) {
-		const uint32_t t = s_sorted[q];
-		uint4 s0 = b.tri_scan[2 * (size_t)tri_rec(b, t)], s1 = b.tri_scan[2 * (size_t)tri_rec(b, t) + 1];
-		int min_by = min(max((int)(s0.w & 0xffffu) - bi.bin_y, 0), kBinMask) >> 3;
-		int max_by = min(max((int)(s0.w >> 16) - bi.bin_y, 0), kBinMask) >> 3;
-		RowScan rs;
-		row_scan_init(rs, s0, s1, (float)bi.bin_x, (float)(bi.bin_y + min_by * 8));
-		for(int by = min_by; by <= max_by; by++) {
-			uint32_t sp[8], bxm = 0;
+	const int lane = lane_id(), wave = threadIdx.x >> 6;
 #pragma unroll
-			for(int r = 0; r < 8; r++) {
-				sp[r] = row_scan_step(rs);
-				bxm |= span_bx_mask(sp[r]);
-			}
-			if(!bxm)
-				continue;
-			uint32_t idx = atomicAdd(&s_row_n[by], 1u);
-			recs[by * kLowRowCap + idx] = make_record(t, sp, bxm);
-			for(int bx = 0; bx < 4; bx++)
-				if(bxm & (1u << bx)) {
-					uint32_t k = atomicAdd(&s_blk_n[by * 4 + bx], 1u);
-					if(k < (uint32_t)kRegSortCap)
-						lists[(by * 4 + bx) * kRegSortCap + k] = idx;
-				}
-		}
+	for(int k = 0; k < kChunks; k++)
+		tk[k] = k * THREADS + threadIdx.x < nlive ? s.sorted[k * THREADS + threadIdx.x] : 0xffffffffu;
+	__syncthreads(); // the staging takes the sorted list's place
+	const uint32_t first = ((uint32_t)bin * 16 + (uint32_t)(lane & 15)) * kRegSortCap;
+	// 8-row rule (raster_low.glsl:39-79): the scan starts at the first row of a band
+	for(int k = 0; k * THREADS + wave * 64 < (int)nlive; k++) {
+		const ScanTri tr = load_scan_tri(b, k == 0 ? tk[0] : k == 1 ? tk[1] : k == 2 ? tk[2 % kChunks] : tk[3 % kChunks]);
+		int lo_by = 0, hi_by = -1;
+		if(tr.t != 0xffffffffu)
+			bands(tr.s0.w, lo_by, hi_by);
+		rowgen_wave(b, s.wave[wave], s_inv, bi.bin_x, bi.bin_y, tr, lo_by * 2, hi_by * 2 + 1, first,
+					(uint32_t)kRegSortCap, [&](uint32_t n) { return atomicAdd(&s_blk_n[lane], n); });
 	}
 	__syncthreads();
 	bool promote = false;
@@ -1012,30 +1129,26 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 		return;
 	}
 	if(threadIdx.x < 16) {
-		int blk = threadIdx.x, by = blk >> 2;
-		slots[blk] = make_uint4((uint32_t)((size_t)bin * 16 * kRegSortCap + blk * kRegSortCap),
-								s_blk_n[blk],
-								(uint32_t)((size_t)bin * 4 * kLowRowCap + by * kLowRowCap),
-								s_row_n[by]);
-		flags[blk] = LUCID_BIN_LEVEL_LOW;
+		b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(first, s_blk_n[threadIdx.x]);
+		flags[threadIdx.x] = LUCID_BIN_LEVEL_LOW;
 	}
 }
 
-__global__ __launch_bounds__(kRowgenThreads) void rowgen_low_kernel(FrameConst c, FrameBufs b) {
-	rowgen_low_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
+__global__ __launch_bounds__(kRowgenLowThreads) void rowgen_low_kernel(FrameConst c, FrameBufs b) {
+	rowgen_low_kernel_body<kRowgenLowThreads>(c, b, WgPos{blockIdx.x, gridDim.x});
 }
-__global__ __launch_bounds__(kRowgenThreads) void rowgen_low_kernel_batch(const FrameDesc *__restrict__ frames,
+__global__ __launch_bounds__(kRowgenLowThreadsBatch) void rowgen_low_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
 	const uint32_t f = batch_frame(sb, blockIdx.x);
 	const FrameDesc &d = sb.frames[f];
-	rowgen_low_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
+	rowgen_low_kernel_body<kRowgenLowThreadsBatch>(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
 }
 
 // ------------------------------------------------------------------ high bins
 
-// Allocates record and list space of every high bin (promotions included) with an exclusive
-// scan over the high list, and clears the counters rowgen_high accumulates into.
+// Allocates the list space of every high bin (promotions included) with an exclusive scan
+// over the high list, and clears the counters rowgen_high accumulates into.
 __device__ __forceinline__ void high_prep_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
 	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
 		return;
@@ -1072,15 +1185,13 @@ __device__ __forceinline__ void high_prep_kernel_body(const FrameConst &c, const
 		bool bad = false;
 		if(i < nh) {
 			uint64_t ex = (uint64_t)s_wave[wave] + inc - n; // tris of earlier high bins
-			uint64_t rec = 4 * ex, lst = list0 + 16 * ex;
-			bool ok = rec + 4ull * n <= b.high_records_cap && lst + 16ull * n <= b.blk_lists_cap;
+			uint64_t lst = list0 + 16 * ex;
+			bool ok = lst + 16ull * n <= b.blk_lists_cap;
 			if(!ok)
-				atomicOr(&b.ctrl[kCtrlOverflow], kOvfRecords | kOvfLists);
+				atomicOr(&b.ctrl[kCtrlOverflow], kOvfLists);
 			bad = !ok; // (ex then need not fit 32 bits: the bin's slots are not used)
-			if(i == nh - 1) { // sizes the host grows the pools to after an overflow
-				b.ctrl[kCtrlRecordCursor] = (uint32_t)min(rec + 4ull * n, 0xffffffffull);
+			if(i == nh - 1) // the size the host grows the lists to after an overflow
 				b.ctrl[kCtrlListCursor] = (uint32_t)min(16ull * (ex + n), 0xffffffffull);
-			}
 			s_ex[threadIdx.x] = (uint32_t)ex;
 			s_n[threadIdx.x] = n;
 		}
@@ -1093,17 +1204,13 @@ __device__ __forceinline__ void high_prep_kernel_body(const FrameConst &c, const
 		// the chunk's block slots, 16 consecutive ones per bin, one per thread and step
 		const uint32_t nb = min(nh - base, 1024u);
 		for(uint32_t p = threadIdx.x; p < nb * 16; p += 1024) {
-			const uint32_t k = p >> 4, blk = p & 15, band = blk >> 2, bx = blk & 3;
+			const uint32_t k = p >> 4, blk = p & 15;
 			const uint32_t bin = high[base + k], n = s_n[k];
 			const uint64_t ex = s_ex[k], lst = list0 + 16 * ex;
-			b.blk_slot[(size_t)bin * 16 + blk] =
-				make_uint4((uint32_t)(lst + (uint64_t)(band * 4 + bx) * n), 0u,
-						   (uint32_t)(4 * ex + (uint64_t)band * n), 0u);
+			b.blk_slot[(size_t)bin * 16 + blk] = make_uint2((uint32_t)(lst + (uint64_t)blk * n), 0u);
 			b.blk_count[(size_t)bin * 16 + blk] = 0;
 			b.blk_flags[(size_t)bin * 16 + blk] = (s_bad[k >> 5] >> (k & 31)) & 1u ? kSlotPromoted : 0u;
 		}
-		for(uint32_t p = threadIdx.x; p < nb * 4; p += 1024)
-			b.band_count[(size_t)high[base + (p >> 2)] * 4 + (p & 3)] = 0;
 		__syncthreads();
 	}
 }
@@ -1119,18 +1226,13 @@ __global__ __launch_bounds__(1024) void high_prep_kernel_batch(const FrameDesc *
 	high_prep_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
 }
 
-// Block-row records of a high bin with the 4-row rule (raster_high.glsl:54-90). Each lane
-// takes one triangle of the bin and scans its rows once, from the first row of its 4-row
-// group (the start row fixes the scanline arithmetic) to its last row, then emits one record
-// per 8-row band it covers; kRowgenSplit work-groups share a bin. A wave's row loop runs as
-// long as its tallest triangle, so each work-group first sorts its triangles by height (a
-// counting sort over the 8 heights in 4-row groups, up to kRowgenRound list chunks at a
-// time) and its waves scan them 64 at a time in that order. Record and list positions come
-// from wave-aggregated atomics.
-constexpr int kRowgenRound = 4; // list chunks of kRowgenThreads entries per sorting round
-
+// Block lists of a high bin with the 4-row rule (raster_high.glsl:54-90): a triangle's scan
+// starts at the first row of its 4-row group (the start row fixes the scanline arithmetic).
+// kRowgenSplit work-groups share a bin. A wave's row loop runs as long as its tallest
+// triangle, so each work-group first sorts its triangles by height (a counting sort over the
+// 8 heights in 4-row groups, up to kRowgenRound list chunks at a time).
 __device__ __forceinline__ void rowgen_high_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfRecords | kOvfLists))
+	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfLists))
 		return;
 	const lucid_info *info = (const lucid_info *)b.info;
 	const uint32_t slot = wg.id / kRowgenSplit;
@@ -1140,115 +1242,31 @@ __device__ __forceinline__ void rowgen_high_kernel_body(const FrameConst &c, con
 	const uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
 	const int bin = (int)counts[LUCID_COUNTS_HIGH_BINS * c.bin_count + slot];
 	const BinInfo bi = load_bin(c, b, bin);
-	const uint4 *slot16 = b.blk_slot + (size_t)bin * 16;
-	uint32_t *band_n = b.band_count + (size_t)bin * 4;
-	uint32_t *blk_n = b.blk_count + (size_t)bin * 16;
 	const int lane = lane_id(), wave = threadIdx.x >> 6;
+	const uint32_t first = b.blk_slot[(size_t)bin * 16 + (lane & 15)].x;
+	uint32_t *blk_n = b.blk_count + (size_t)bin * 16;
 	const uint32_t stride = kRowgenThreads * kRowgenSplit;
-	constexpr int kHeights = kBinSize / 4;
-	__shared__ uint32_t s_sorted[kRowgenRound * kRowgenThreads];
+	constexpr int kHeights = kBinSize / 4, kChunks = kRowgenRound / kRowgenThreads;
+	__shared__ RowgenLds<kRowgenThreads> s;
+	__shared__ float s_inv[65];
 	__shared__ uint32_t s_cnt[kHeights], s_off[kHeights], s_n;
-	// the row spans of each lane's triangle: rows[r][lane] of the wave
-	__shared__ uint16_t s_rows[kRowgenThreads / 64][kBinSize][64];
-	uint16_t *rows = &s_rows[wave][0][lane];
+	fill_inverses(s_inv);
 	// first row group and height in row groups of triangle t in this bin
 	auto groups = [&](uint32_t yr, int &g0, int &g1) {
 		g0 = min(max((int)(yr & 0xffffu) - bi.bin_y, 0), kBinMask) >> 2;
 		g1 = min(max((int)(yr >> 16) - bi.bin_y, 0), kBinMask) >> 2;
 	};
-	auto scan_tri = [&](uint32_t t) { // called by the whole wave; t = ~0 on idle lanes
-		int row_lo = 0, row_hi = -1;
-		RowScan rs;
-		if(t != 0xffffffffu) {
-			const uint4 s0 = b.tri_scan[2 * (size_t)tri_rec(b, t)], s1 = b.tri_scan[2 * (size_t)tri_rec(b, t) + 1];
-			int g0, g1;
-			groups(s0.w, g0, g1);
-			row_lo = g0 * 4, row_hi = g1 * 4 + 3;
-			row_scan_init(rs, s0, s1, (float)bi.bin_x, (float)(bi.bin_y + row_lo));
-		}
-		uint32_t bxm_all = 0; // block-column masks of the four bands, 4 bits each
-		for(int r = row_lo; r <= row_hi; r++) {
-			const uint32_t v = row_scan_step(rs);
-			rows[r * 64] = (uint16_t)v;
-			bxm_all |= span_bx_mask(v) << (4 * (r >> 3));
-		}
-		// each band's record: rows 0-5 in lo (10 bits each), rows 6-7 in hi; rows the
-		// triangle does not reach stay empty (31, 0)
-		uint64_t lo_b[4];
-		uint32_t hi_b[4], bxm_b[4];
-#pragma unroll
-		for(int by = 0; by < 4; by++) {
-			const uint32_t bxm = (bxm_all >> (4 * by)) & 15u;
-			lo_b[by] = 0, hi_b[by] = 0, bxm_b[by] = bxm;
-			if(!ballot(bxm != 0))
-				continue;
-			if(bxm) {
-				uint64_t lo = 0;
-				uint32_t hi = 0;
-#pragma unroll
-				for(int k = 0; k < 8; k++) {
-					const int r = by * 8 + k;
-					const uint32_t v = r >= row_lo && r <= row_hi ? (uint32_t)rows[r * 64] : (uint32_t)kBinMask;
-					if(k < 6)
-						lo |= (uint64_t)v << (10 * k);
-					else
-						hi |= v << (10 * (k - 6));
-				}
-				lo_b[by] = lo, hi_b[by] = hi;
-			}
-		}
-		// per band: its record counter, then its four block-list counters; lane 5 by + k
-		// reserves counter k of band by (one atomic instruction for all of them)
-		uint64_t emit[4], sel[4][4];
-		uint32_t add = 0;
-		uint32_t *ctr = band_n;
-#pragma unroll
-		for(int by = 0; by < 4; by++) {
-			emit[by] = ballot(bxm_b[by] != 0);
-			if(lane == 5 * by)
-				add = (uint32_t)__popcll(emit[by]), ctr = band_n + by;
-#pragma unroll
-			for(int bx = 0; bx < 4; bx++) {
-				sel[by][bx] = ballot((bxm_b[by] >> bx) & 1u);
-				if(lane == 5 * by + 1 + bx)
-					add = (uint32_t)__popcll(sel[by][bx]), ctr = blk_n + by * 4 + bx;
-			}
-		}
-		uint32_t got = 0;
-		if(lane < 20 && add)
-			got = atomicAdd(ctr, add);
-		const uint64_t below = (1ull << lane) - 1ull;
-#pragma unroll
-		for(int by = 0; by < 4; by++) {
-			if(!emit[by])
-				continue;
-			const uint32_t bxm = bxm_b[by];
-			const uint32_t rbase = __shfl(got, 5 * by, 64);
-			const uint32_t idx = rbase + (uint32_t)__popcll(emit[by] & below);
-			if(bxm)
-				b.high_records[slot16[by * 4].z + idx] =
-					make_uint4(t, (uint32_t)lo_b[by] & 0x3fffffffu,
-							   (uint32_t)(lo_b[by] >> 30) & 0x3fffffffu, hi_b[by] | (bxm << 20));
-#pragma unroll
-			for(int bx = 0; bx < 4; bx++) {
-				const uint32_t lb = __shfl(got, 5 * by + 1 + bx, 64);
-				if((bxm >> bx) & 1u)
-					b.blk_lists[slot16[by * 4 + bx].x + lb +
-								(uint32_t)__popcll(sel[by][bx] & below)] = idx;
-			}
-		}
-	};
 	// the work-group's list positions: chunks split, split + kRowgenSplit, ... of
 	// kRowgenThreads entries; culled triangles (every second one of a soup quad) are dropped
-	const uint32_t round_len = stride * kRowgenRound;
+	const uint32_t round_len = stride * kChunks;
 	for(uint32_t base = split * kRowgenThreads; base < bi.nlevel; base += round_len) {
 		if(threadIdx.x < kHeights)
 			s_cnt[threadIdx.x] = 0;
 		__syncthreads();
-		uint32_t tk[kRowgenRound];
-		int hk[kRowgenRound];
+		uint32_t tk[kChunks];
+		int hk[kChunks];
 #pragma unroll
-		for(int k = 0; k < kRowgenRound; k++) {
+		for(int k = 0; k < kChunks; k++) {
 			const uint32_t i = base + k * stride + threadIdx.x;
 			const uint32_t t = i < bi.nlevel ? bin_tri_at(b, i, bi.qc, bi.qo, bi.to) : 0xffffffffu;
 			int h = -1;
@@ -1269,13 +1287,23 @@ __device__ __forceinline__ void rowgen_high_kernel_body(const FrameConst &c, con
 		}
 		__syncthreads();
 #pragma unroll
-		for(int k = 0; k < kRowgenRound; k++)
+		for(int k = 0; k < kChunks; k++)
 			if(hk[k] >= 0)
-				s_sorted[atomicAdd(&s_off[hk[k]], 1u)] = tk[k];
+				s.sorted[atomicAdd(&s_off[hk[k]], 1u)] = tk[k];
 		__syncthreads();
 		const uint32_t n = s_n;
-		for(uint32_t q = wave * 64; q < n; q += kRowgenThreads)
-			scan_tri(q + lane < n ? s_sorted[q + lane] : 0xffffffffu);
+#pragma unroll
+		for(int k = 0; k < kChunks; k++)
+			tk[k] = k * kRowgenThreads + threadIdx.x < n ? s.sorted[k * kRowgenThreads + threadIdx.x] : 0xffffffffu;
+		__syncthreads(); // the staging takes the sorted list's place
+		for(int k = 0; k * kRowgenThreads + wave * 64 < (int)n; k++) {
+			const ScanTri tr = load_scan_tri(b, k == 0 ? tk[0] : k == 1 ? tk[1] : k == 2 ? tk[2] : tk[3]);
+			int g0 = 0, g1 = -1;
+			if(tr.t != 0xffffffffu)
+				groups(tr.s0.w, g0, g1);
+			rowgen_wave(b, s.wave[wave], s_inv, bi.bin_x, bi.bin_y, tr, g0, g1, first, ~0u,
+						[&](uint32_t num) { return atomicAdd(&blk_n[lane], num); });
+		}
 		if(base + round_len < bi.nlevel)
 			__syncthreads(); // the next round reuses the sorted list
 	}
@@ -1322,7 +1350,7 @@ constexpr uint32_t kMidSortCap = 2048;
 
 template <uint32_t CAP>
 __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfRecords | kOvfLists))
+	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfLists))
 		return;
 	const lucid_info *info = (const lucid_info *)b.info;
 	const uint32_t hslot = wg.id >> 4;
@@ -1335,14 +1363,9 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	if(b.blk_flags[slot] & kSlotPromoted)
 		return; // allocation failed: the frame reports an overflow
 	const uint32_t m = b.blk_count[slot];
-	const uint4 sl = b.blk_slot[slot];
-	const int bin_x = (bin % c.bin_count_x) * kBinSize, bin_y = (bin / c.bin_count_x) * kBinSize;
-	const int px0 = bin_x + bx * 8, py0 = bin_y + by * 8;
-	if constexpr(CAP == kMidSortCap) {
-		const uint32_t nrec = b.band_count[(size_t)bin * 4 + by];
-		if(threadIdx.x == 0)
-			b.blk_slot[slot] = make_uint4(sl.x, m, sl.z, nrec);
-	}
+	const uint32_t list0 = b.blk_slot[slot].x;
+	if(CAP == kMidSortCap && threadIdx.x == 0)
+		b.blk_slot[slot].y = m;
 	if(m <= c.presort_min) { // sorted in registers by the block rasteriser (<= kRegSortCap)
 		if(CAP == kMidSortCap && threadIdx.x == 0)
 			b.blk_flags[slot] = LUCID_BIN_LEVEL_HIGH;
@@ -1356,7 +1379,8 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	}
 	if(m > (uint32_t)kBigSortCap) {
 		if(threadIdx.x < 64) {
-			const int px = px0 + (threadIdx.x & 7), py = py0 + (threadIdx.x >> 3);
+			const int px = (bin % c.bin_count_x) * kBinSize + bx * 8 + (threadIdx.x & 7);
+			const int py = (bin / c.bin_count_x) * kBinSize + by * 8 + (threadIdx.x >> 3);
 			if(threadIdx.x == 0) {
 				b.blk_flags[slot] = LUCID_BIN_LEVEL_HIGH | kSlotWhole;
 				atomicAdd(&((lucid_info *)b.info)->stats[3], 1u); // blocks too long to pre-sort
@@ -1374,8 +1398,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	__shared__ uint8_t s_smp[CAP]; // samples (pixel-mask bits) of each entry, in list order
 	static_assert(kBigSortCap <= (1 << 13), "list positions fit 13 bits of the key");
 	static_assert(kSortThreads == 256, "four waves share the chunks");
-	const uint32_t *list = b.blk_lists + sl.x;
-	const uint4 *recs = b.high_records + sl.z;
+	const uint4 *list = b.blk_lists + list0;
 	const int wave_s = threadIdx.x >> 6, lane_s = lane_id();
 	const uint32_t P = max(256u, next_pow2(m));
 	const uint32_t nchunks = P / 256;
@@ -1384,14 +1407,10 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	const int pb = 31 - __clz(P);
 	const uint32_t pmask = P - 1u;
 	const bool unsorted = (c.opts & LUCID_OPT_UNSORTED) != 0; // the unsorted baseline
-	// The block's pool space (allocated first): the sorted entries (header, triangle ids,
-	// masks) and a scratch copy of the same in list order, which pass 1 fills so that the
-	// sorted output is gathered from the block's own (cache-resident) scratch instead of
-	// the scattered records.
-	const uint32_t sorted_words = sorted_mask_offset(m) + 2 * m;
-	const uint32_t scratch_mask = sorted_words + ((m + 1u) & ~1u);
+	// the block's pool space (allocated first) for the sorted entries: header, triangle ids,
+	// masks
 	if(threadIdx.x == 0) {
-		const uint32_t need = scratch_mask + 2 * m + 1; // + 1: even rounding of the base
+		const uint32_t need = sorted_mask_offset(m) + 2 * m + 1; // + 1: even rounding of the base
 		const uint32_t stripe = slot % kSortStripes;
 		const uint64_t region = (b.sorted_cap / kSortStripes) & ~1ull;
 		const uint32_t off = atomicAdd(sort_cursor(b.ctrl, stripe), need);
@@ -1412,11 +1431,8 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 		return;
 	}
 	uint32_t *hdr = b.sorted_pool + s_base;
-	uint32_t *scratch_tri = hdr + sorted_words;
-	uint64_t *scratch_msk = (uint64_t *)(hdr + scratch_mask);
-	// Keys are (depth rank << pb | list position). Pass 1 gathers the records once:
-	// depth keys (in s_key), the scratch copy, the total of the sample counts and the
-	// block's key range.
+	// Keys are (depth rank << pb | list position). Pass 1 reads the entries once: depth keys
+	// (in s_key), sample counts and the block's key range.
 	uint32_t lo = ~0u, hi = 0u;
 	uint32_t mine = 0;
 	for(uint32_t ch = wave_s; ch < nchunks; ch += kSortThreads / 64) {
@@ -1424,20 +1440,14 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 		for(int e = 0; e < 4; e++) {
 			const uint32_t j = ch * 256 + e * 64 + lane_s;
 			if(j < m) {
-				const uint4 rec = recs[list[j]];
-				const uint64_t msk = record_block_mask(rec, bx);
-				scratch_tri[j] = rec.x;
-				scratch_msk[j] = msk;
-				s_smp[j] = (uint8_t)__popcll(msk);
-				mine += (uint32_t)__popcll(msk);
-				if(unsorted) {
-					s_key[j] = j; // list order: rank 0, the position alone
-				} else {
-					const uint32_t dk = inv_ord_f32(mask_inv_depth(b, rec.x, msk, px0, py0));
-					s_key[j] = dk;
-					lo = min(lo, dk);
-					hi = max(hi, dk);
-				}
+				const uint4 en = list[j];
+				const uint32_t smp = (uint32_t)__popc(en.z) + (uint32_t)__popc(en.w);
+				s_smp[j] = (uint8_t)smp;
+				mine += smp;
+				// the unsorted baseline: list order (rank 0, the position alone)
+				s_key[j] = unsorted ? j : en.y;
+				lo = min(lo, en.y);
+				hi = max(hi, en.y);
 			}
 		}
 	}
@@ -1517,7 +1527,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	// that, but the backward's pass A flushes its window at every slice, so in frames with
 	// fp32 samples (the differentiable ones) each run of equal ranks that lies within one
 	// round (and is at most kTieRun long) is put in exact depth-key order here: its members
-	// recompute their full depth key and take their place among the run.
+	// take their place among the run by their full depth keys.
 	const bool exact_runs = (c.opts & LUCID_OPT_FP32_SAMPLES) != 0 && !unsorted;
 	uint32_t carry = 0, found = 0;
 	if(!exact_runs) {
@@ -1551,20 +1561,17 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 			run += s_smp[key & pmask];
 		}
 		for(uint32_t i = threadIdx.x; i < m; i += 4 * kSortThreads) {
-			uint32_t tk[4];
-			uint64_t mk[4];
+			uint4 en[4];
 #pragma unroll
 			for(int k = 0; k < 4; k++) {
 				const uint32_t ik = i + k * kSortThreads;
-				const uint32_t pos = ik < m ? s_key[ik] & pmask : 0u;
-				tk[k] = ik < m ? scratch_tri[pos] : 0u;
-				mk[k] = ik < m ? scratch_msk[pos] : 0ull;
+				en[k] = ik < m ? list[s_key[ik] & pmask] : make_uint4(0u, 0u, 0u, 0u);
 			}
 #pragma unroll
 			for(int k = 0; k < 4; k++) {
 				const uint32_t ik = i + k * kSortThreads;
 				if(ik < m)
-					tri_out[ik] = tk[k], mask_out[ik] = mk[k];
+					tri_out[ik] = en[k].x, mask_out[ik] = entry_mask(en[k]);
 			}
 		}
 	}
@@ -1576,12 +1583,10 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 		bool tie = false;
 		if(i < m) {
 			key = s_key[i];
-			tri = scratch_tri[key & pmask];
-			msk = scratch_msk[key & pmask];
+			const uint4 en = list[key & pmask];
+			tri = en.x, dk = en.y, msk = entry_mask(en);
 			tie = exact_runs && ((i > 0 && (s_key[i - 1] >> pb) == (key >> pb)) ||
 								 (i + 1 < m && (s_key[i + 1] >> pb) == (key >> pb)));
-			if(tie)
-				dk = inv_ord_f32(mask_inv_depth(b, tri, msk, px0, py0));
 		}
 		s_tdk[r & 1][threadIdx.x] = dk;
 		const uint32_t smp = (uint32_t)__popcll(msk);
@@ -1651,7 +1656,7 @@ __global__ __launch_bounds__(kSortThreads) void high_finalize_kernel(FrameConst 
 // queue entries w, w + count, ... (the queue is complete: the first pass has finished).
 __device__ __forceinline__ void high_finalize_long_body(const FrameConst &c, const FrameBufs &b,
 														 WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfRecords | kOvfLists))
+	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfLists))
 		return;
 	const uint32_t n = b.ctrl[kCtrlBigSorts];
 	for(uint32_t q = wg.id; q < n; q += wg.count) {
@@ -1958,7 +1963,7 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 		write_pixel(c, b, px, py, bg, 0u);
 		return;
 	}
-	const uint4 sl = b.blk_slot[slot];
+	const uint2 sl = b.blk_slot[slot];
 	const uint32_t m = sl.y;
 	if(m == 0) {
 		write_pixel(c, b, px, py, bg, 0u);
@@ -1966,8 +1971,7 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	}
 	if(b.ctrl[kCtrlRecorded])
 		return; // the recording pass A renders this block
-	const uint4 *recs = (level == LUCID_BIN_LEVEL_LOW ? b.low_records : b.high_records) + sl.z;
-	const uint32_t *list = b.blk_lists + sl.x;
+	const uint4 *list = b.blk_lists + sl.x;
 	uint64_t msk_all[4];
 	uint32_t tri_all[4];
 	if(c.opts & LUCID_OPT_UNSORTED) { // list order
@@ -1975,9 +1979,9 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 		for(int j = 0; j < 4; j++) {
 			msk_all[j] = 0, tri_all[j] = 0;
 			if(j * 64 + lane < (int)m) {
-				const uint4 rec = recs[list[j * 64 + lane]];
-				msk_all[j] = record_block_mask(rec, bx);
-				tri_all[j] = rec.x;
+				const uint4 en = list[j * 64 + lane];
+				msk_all[j] = entry_mask(en);
+				tri_all[j] = en.x;
 			}
 		}
 	} else {
@@ -1988,7 +1992,7 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 		uint64_t *s_msk = reinterpret_cast<uint64_t *>(s_rec);
 		uint32_t *s_tri = reinterpret_cast<uint32_t *>(s_msk + kRegSortCap);
 		uint32_t pos[4];
-		sort_block_positions(b, recs, list, m, bx, px0, py0, pos, s_msk, s_tri);
+		sort_block_positions(list, m, pos, s_msk, s_tri);
 		wave_sync_lds();
 #pragma unroll
 		for(int j = 0; j < 4; j++) {
@@ -2081,8 +2085,7 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 	static_assert(sizeof(RangeEnd) <= sizeof(s_rec[0]), "a range's end state fits its staging");
 	auto range_end = [&](int w) -> RangeEnd & { return *reinterpret_cast<RangeEnd *>(&s_rec[w][0]); };
 	const int wave = threadIdx.x >> 6, lane = lane_id();
-	const uint4 sl = b.blk_slot[slot];
-	const uint32_t m = sl.y;
+	const uint32_t m = b.blk_slot[slot].y;
 	const uint32_t *hdr = b.sorted_pool + b.blk_sorted[slot];
 	const uint32_t nw = hdr[0];
 	const uint32_t *tri = hdr + kSortedHeader;
@@ -2173,32 +2176,26 @@ __global__ __launch_bounds__(kBigWaves * 64) void block_raster_big_kernel_batch(
 // ------------------------------------------------------------------ exact fallback
 
 // Collects the keys (depth key << 32 | triangle id) of one pixel's fragments into `dst`
-// (LDS or global) from the block's list; returns the count. Entries beyond `cap` are
-// counted but not stored.
-__device__ uint32_t gather_pixel_keys(const FrameBufs &b, const uint4 *recs, const uint32_t *list,
-									  uint32_t m, int row, int xb, float px, float py,
-									  uint64_t *dst, uint32_t cap, bool global_dst) {
+// (LDS or global) from the block's list (the entries whose pixel mask has `bit`); returns the
+// count. Entries beyond `cap` are counted but not stored.
+__device__ uint32_t gather_pixel_keys(const FrameBufs &b, const uint4 *list, uint32_t m,
+									  int bit, float px, float py, uint64_t *dst, uint32_t cap,
+									  bool global_dst) {
 	constexpr int kU = 4; // entries per lane per step: their loads are issued together
 	const int lane = lane_id();
 	uint32_t n = 0;
 	for(uint32_t base = 0; base < m; base += 64 * kU) {
-		uint32_t idx[kU];
+		uint4 rec[kU];
 #pragma unroll
 		for(int k = 0; k < kU; k++) {
 			const uint32_t j = base + k * 64 + lane;
-			idx[k] = j < m ? list[j] : 0xffffffffu;
+			rec[k] = j < m ? list[j] : make_uint4(0u, 0u, 0u, 0u);
 		}
-		uint4 rec[kU];
-#pragma unroll
-		for(int k = 0; k < kU; k++)
-			rec[k] = idx[k] != 0xffffffffu ? recs[idx[k]] : make_uint4(0u, kBinMask, kBinMask, kBinMask);
 		bool hit[kU];
 		uint4 d[kU];
 #pragma unroll
 		for(int k = 0; k < kU; k++) {
-			const uint32_t sp = record_span(rec[k], row);
-			const int a = (int)(sp & 31u), e = (int)((sp >> 5) & 31u);
-			hit[k] = idx[k] != 0xffffffffu && a <= xb && xb <= e;
+			hit[k] = (entry_mask(rec[k]) >> bit) & 1ull;
 			d[k] = hit[k] ? b.tri_depth[tri_rec(b, rec[k].x)] : make_uint4(0u, 0u, 0u, 0u);
 		}
 #pragma unroll
@@ -2260,15 +2257,12 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 it
 	const uint32_t slot = item.x;
 	const int px = (int)item.y, py = (int)item.z;
 	const bool whole = item.w != 0;
-	const int blk = (int)(slot & 15u), bx = blk & 3;
-	const uint32_t level = b.blk_flags[slot] & kSlotLevelMask;
-	const uint4 sl = b.blk_slot[slot];
-	const uint4 *recs = (level == LUCID_BIN_LEVEL_LOW ? b.low_records : b.high_records) + sl.z;
-	const uint32_t *list = b.blk_lists + sl.x;
+	const uint2 sl = b.blk_slot[slot];
+	const uint4 *list = b.blk_lists + sl.x;
 	const uint32_t m = sl.y;
-	const int row = py & 7, xb = bx * 8 + (px & 7);
+	const int bit = (py & 7) * 8 + (px & 7);
 	const float fx = (float)px, fy = (float)py;
-	const uint32_t n = gather_pixel_keys(b, recs, list, m, row, xb, fx, fy, s_keys, kFallbackCap, false);
+	const uint32_t n = gather_pixel_keys(b, list, m, bit, fx, fy, s_keys, kFallbackCap, false);
 	Accum acc;
 	if(n <= (uint32_t)kFallbackCap) {
 		const uint32_t P = next_pow2(n < 2 ? 2 : n);
@@ -2292,7 +2286,7 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 it
 		if(off == 0xffffffffu)
 			return; // the frame reports an overflow and is rendered again
 		uint64_t *g = b.spill + off;
-		gather_pixel_keys(b, recs, list, m, row, xb, fx, fy, g, P, true);
+		gather_pixel_keys(b, list, m, bit, fx, fy, g, P, true);
 		for(uint32_t i = n + lane; i < P; i += 64)
 			__hip_atomic_store(&g[i], ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		__threadfence();
@@ -2476,14 +2470,11 @@ struct BlockEntries {
 // Valid for the blocks the block kernels process (not empty, whole or promoted, m > 0).
 // For lists sorted here only wave 0 may call it (it fills s_tri_all / s_mask_all).
 __device__ __forceinline__ BlockEntries bwd_block_entries(const FrameConst &c, const FrameBufs &b,
-														  uint32_t slot, uint32_t flags, uint4 sl,
+														  uint32_t slot, uint32_t flags, uint2 sl,
 														  int wave, uint32_t *s_tri_all,
 														  uint64_t *s_mask_all) {
 	const int lane = lane_id();
 	const uint32_t m = sl.y;
-	const int bin = slot >> 4, blk = slot & 15, by = blk >> 2, bx = blk & 3;
-	const int px0 = (bin % c.bin_count_x) * kBinSize + bx * 8;
-	const int py0 = (bin / c.bin_count_x) * kBinSize + by * 8;
 	BlockEntries ent;
 	if(flags & kSlotPresorted) {
 		const uint32_t *hdr = b.sorted_pool + b.blk_sorted[slot];
@@ -2494,18 +2485,19 @@ __device__ __forceinline__ BlockEntries bwd_block_entries(const FrameConst &c, c
 		ent.e1 = (uint32_t)wave < ent.nw ? hdr[2 + wave] : m;
 		return ent;
 	}
-	const uint32_t level = flags & kSlotLevelMask;
-	const uint4 *recs = (level == LUCID_BIN_LEVEL_LOW ? b.low_records : b.high_records) + sl.z;
-	const uint32_t *list = b.blk_lists + sl.x;
-	uint32_t pos[4];
-	sort_block_positions(b, recs, list, m, bx, px0, py0, pos);
+	uint32_t pos[4], t[4];
+	uint64_t k[4];
+	sort_block_positions(b.blk_lists + sl.x, m, pos, s_mask_all, s_tri_all);
+	wave_sync_lds();
 #pragma unroll
 	for(int j = 0; j < 4; j++)
-		if(j * 64 + lane < (int)m) {
-			uint4 rec = recs[list[pos[j]]];
-			s_mask_all[j * 64 + lane] = record_block_mask(rec, bx);
-			s_tri_all[j * 64 + lane] = rec.x;
-		}
+		if(j * 64 + lane < (int)m)
+			k[j] = s_mask_all[pos[j]], t[j] = s_tri_all[pos[j]];
+	wave_sync_lds(); // read in list order before they are written in depth order
+#pragma unroll
+	for(int j = 0; j < 4; j++)
+		if(j * 64 + lane < (int)m)
+			s_mask_all[j * 64 + lane] = k[j], s_tri_all[j * 64 + lane] = t[j];
 	wave_sync_lds();
 	ent.tri = s_tri_all;
 	ent.mask = s_mask_all;
@@ -2585,7 +2577,7 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 	const uint32_t level = flags & kSlotLevelMask;
 	if(level == LUCID_BIN_LEVEL_EMPTY || (flags & (kSlotWhole | kSlotPromoted)))
 		return;
-	const uint4 sl = b.blk_slot[slot];
+	const uint2 sl = b.blk_slot[slot];
 	if(sl.y == 0)
 		return;
 	const bool presorted = (flags & kSlotPresorted) != 0;
@@ -2786,7 +2778,7 @@ __global__ __launch_bounds__(64) void bwd_pass_b_kernel(FrameConst c, FrameBufs 
 	const uint32_t level = flags & kSlotLevelMask;
 	if(level == LUCID_BIN_LEVEL_EMPTY || (flags & (kSlotWhole | kSlotPromoted)))
 		return;
-	const uint4 sl = b.blk_slot[slot];
+	const uint2 sl = b.blk_slot[slot];
 	if(sl.y == 0)
 		return;
 	if(!(flags & kSlotPresorted) && wave != 0)
@@ -2969,16 +2961,13 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 	const int lane = lane_id();
 	const uint32_t slot = item.x;
 	const int px = (int)item.y, py = (int)item.z;
-	const int blk = (int)(slot & 15u), bx = blk & 3;
-	const uint32_t level = b.blk_flags[slot] & kSlotLevelMask;
-	const uint4 sl = b.blk_slot[slot];
-	const uint4 *recs = (level == LUCID_BIN_LEVEL_LOW ? b.low_records : b.high_records) + sl.z;
-	const uint32_t *list = b.blk_lists + sl.x;
+	const uint2 sl = b.blk_slot[slot];
+	const uint4 *list = b.blk_lists + sl.x;
 	const uint32_t m = sl.y;
-	const int row = py & 7, xb = bx * 8 + (px & 7);
+	const int bit = (py & 7) * 8 + (px & 7);
 	const float fx = (float)px, fy = (float)py;
 	const uint32_t n =
-		gather_pixel_keys(b, recs, list, m, row, xb, fx, fy, s_keys, kFallbackCap, false);
+		gather_pixel_keys(b, list, m, bit, fx, fy, s_keys, kFallbackCap, false);
 	const uint64_t *keys = s_keys;
 	bool global_keys = false;
 	if(n <= (uint32_t)kFallbackCap) {
@@ -3001,7 +2990,7 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 		if(off == 0xffffffffu)
 			return;
 		uint64_t *gk = b.spill + off;
-		gather_pixel_keys(b, recs, list, m, row, xb, fx, fy, gk, P, true);
+		gather_pixel_keys(b, list, m, bit, fx, fy, gk, P, true);
 		for(uint32_t i = n + lane; i < P; i += 64)
 			__hip_atomic_store(&gk[i], ~0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		__threadfence();
@@ -3122,7 +3111,7 @@ template <bool FP32, int MODE>
 static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 							hipEvent_t *ev) {
 	constexpr bool TEX = MODE == kShadeTextured;
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenThreads), 0, stream, c, b);
+	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
 	if(ev)
 		(void)hipEventRecord(ev[0], stream);
 	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);
@@ -3153,7 +3142,7 @@ static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t
 template <bool FP32, int W, int MODE>
 static void launch_raster_batch_t(const BatchPlan &p, hipStream_t stream) {
 	constexpr bool TEX = MODE == kShadeTextured;
-	hipLaunchKernelGGL(rowgen_low_kernel_batch, dim3(p.total[kBsRowgenLow]), dim3(kRowgenThreads), 0,
+	hipLaunchKernelGGL(rowgen_low_kernel_batch, dim3(p.total[kBsRowgenLow]), dim3(kRowgenLowThreadsBatch), 0,
 					   stream, p.frames, p.stage_pre(kBsRowgenLow), p.num_frames);
 	hipLaunchKernelGGL(high_prep_kernel_batch, dim3(p.total[kBsHighPrep]), dim3(1024), 0, stream,
 					   p.frames, p.stage_pre(kBsHighPrep), p.num_frames);
@@ -3235,7 +3224,7 @@ hipError_t launch_raster(const FrameConst &c, const FrameBufs &b, hipStream_t st
 // recomputed, not stored), then the gradient row allocation.
 hipError_t launch_backward_prepare(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								   hipStream_t stream) {
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenThreads), 0, stream, c, b);
+	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
 	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);
 	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kRowgenSplit), dim3(kRowgenThreads), 0,
 					   stream, c, b);
@@ -3265,7 +3254,7 @@ __global__ __launch_bounds__(64) void record_gate_kernel(FrameBufs b, BwdBufs g)
 // (which then render only what the recording pass does not).
 hipError_t launch_raster_recording(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								   hipStream_t stream, hipEvent_t *ev) {
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenThreads), 0, stream, c, b);
+	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
 	if(ev)
 		(void)hipEventRecord(ev[0], stream);
 	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);

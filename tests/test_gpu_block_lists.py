@@ -1,0 +1,43 @@
+"""Block lists at the sizes where row generation changes path: bins just below and at the
+high-bin limit (1024 list positions), blocks at and beyond the promotion threshold (256),
+sorting rounds of 1024 positions with a remainder, triangles from a fraction of a pixel to the
+whole bin, and bins cut by the image edge. Bins, lists and fragment counts bit-exact, colours
+within 1/255, as everywhere."""
+
+import numpy as np
+import pytest
+
+from lucid_amd import _lib, scenes
+
+from test_gpu_parity import _check, _render_both
+
+pytestmark = pytest.mark.gpu
+
+
+def _soup(n, w, h, size_px, seed):
+    """n soup triangles inside the first bin (or the image), vertex offsets of size_px."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(1.0, min(31.0, w - 1, h - 1), (n, 1, 2))
+    off = rng.normal(0.0, 1.0, (n, 3, 2)) * size_px
+    ndc = (c + off + 0.5) / np.array([w, h]) * 2.0 - 1.0
+    return scenes.soup_scene(w, h, ndc, rng.uniform(1.0, 90.0, n), rng.uniform(0, 1, (n, 3, 3)),
+                             rng.uniform(0.05, 0.4, n), name=f"bin_{n}_{size_px}")
+
+
+@pytest.mark.parametrize("opts", [0, _lib.OPT_FP32_SAMPLES])
+@pytest.mark.parametrize("n,w,h,size_px", [
+    (1, 8, 8, 40.0), (63, 33, 31, 12.0), (65, 40, 17, 0.6), (511, 32, 32, 2.0),
+    (512, 32, 32, 2.0), (513, 37, 45, 6.0), (1025, 35, 33, 1.5), (5003, 41, 39, 3.0),
+    (600, 64, 64, 60.0)])
+def test_bin_sizes(oracle_mod, n, w, h, size_px, opts):
+    sc = _soup(n, w, h, size_px, seed=n)
+    r, gpu, ref = _render_both(sc, oracle_mod, opts=opts)
+    _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 300])
+def test_promotion_threshold(oracle_mod, n):
+    """n triangles that all cover one block of a low bin."""
+    sc = scenes.block_stack(48, 40, n, center_px=(12, 12), size_px=6.0, seed=n)
+    r, gpu, ref = _render_both(sc, oracle_mod)
+    _check(sc, gpu, ref, oracle_mod)

@@ -157,7 +157,7 @@ __device__ __forceinline__ void bin_count_kernel_body(const FrameConst &c, const
 			uint32_t inc = wave_inclusive_add(v) + carry;
 			if(bx < NBX)
 				ht[by * NBX + bx] = inc;
-			carry = __shfl(inc, 63, 64);
+			carry = wave_read(inc, 63);
 		}
 	}
 	__syncthreads();

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/lucid_c.h"
 #include "../../include/lucid_structs.h"
 
@@ -438,26 +440,85 @@ __device__ __forceinline__ void wave_sync_lds() {
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint32_t wave_inclusive_add(uint32_t v) {
-	int l = lane_id();
-#pragma unroll
-	for(int d = 1; d < 64; d <<= 1) {
-		uint32_t t = __shfl_up(v, d, 64);
-		if(l >= d)
-			v += t;
+// Lane exchanges with constant patterns go through the VALU (DPP and gfx950's row swaps)
+// instead of ds_bpermute_b32, which __shfl compiles to: no LDS traffic, no address register and
+// a few cycles of latency instead of an LDS round trip. All lanes of the wave must be active.
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
+	return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppXor3 = 0x1b; // quad_perm
+constexpr int kDppRor8 = 0x128, kDppXor7 = 0x141, kDppXor15 = 0x140; // row_ror, (half) row mirror
+
+// The two values of a lane pair (lane, lane ^ J), J = 16 or 32: x of the lower lane, y of the
+// upper one, in both lanes.
+struct LanePair {
+	uint32_t x, y;
+};
+template <int J> __device__ __forceinline__ LanePair lane_pair(uint32_t v) {
+	static_assert(J == 16 || J == 32, "rows of 16 lanes");
+	if constexpr(J == 16) {
+		const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+		return LanePair{r[0], r[1]};
+	} else {
+		const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+		return LanePair{r[0], r[1]};
 	}
+}
+
+// The value of lane ^ J, J < 16.
+template <int J> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+	static_assert(J == 1 || J == 2 || J == 4 || J == 8, "within a row of 16 lanes");
+	if constexpr(J == 1)
+		return dpp_mov<kDppXor1>(v);
+	else if constexpr(J == 2)
+		return dpp_mov<kDppXor2>(v);
+	else if constexpr(J == 4)
+		return dpp_mov<kDppXor3>(dpp_mov<kDppXor7>(v));
+	else
+		return dpp_mov<kDppRor8>(v);
+}
+
+// The value of a lane given by a wave-uniform index.
+__device__ __forceinline__ uint32_t wave_read(uint32_t v, int src) {
+	return (uint32_t)__builtin_amdgcn_readlane((int)v, src);
+}
+__device__ __forceinline__ float wave_read(float v, int src) {
+	return __uint_as_float(wave_read(__float_as_uint(v), src));
+}
+
+__device__ __forceinline__ uint32_t wave_inclusive_add(uint32_t v) {
+	// row_shr 1, 2, 4, 8 scan each row of 16 lanes (lanes shifted in from outside read 0), then
+	// lane 15 of each even row is added to the next row and lane 31 to the upper half
+	auto add = [&](auto ctrl, auto rows) {
+		v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value,
+												   decltype(rows)::value, 0xf, false);
+	};
+	using std::integral_constant;
+	add(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});
+	add(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+	add(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+	add(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+	add(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{}); // row_bcast:15
+	add(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{}); // row_bcast:31
 	return v;
 }
 
-__device__ __forceinline__ uint32_t wave_inclusive_max(uint32_t v) {
-	int l = lane_id();
-#pragma unroll
-	for(int d = 1; d < 64; d <<= 1) {
-		uint32_t t = __shfl_up(v, d, 64);
-		if(l >= d)
-			v = v > t ? v : t;
-	}
-	return v;
+// Reduction over the wave with an associative, commutative f; the result is in every lane.
+template <class F> __device__ __forceinline__ uint32_t wave_reduce(uint32_t v, F &&f) {
+	v = f(v, dpp_mov<kDppXor1>(v));
+	v = f(v, dpp_mov<kDppXor2>(v));
+	v = f(v, dpp_mov<kDppXor7>(v));  // (quads hold one value each)
+	v = f(v, dpp_mov<kDppXor15>(v)); // (and half rows)
+	const LanePair r = lane_pair<16>(v);
+	v = f(r.x, r.y);
+	const LanePair h = lane_pair<32>(v);
+	return f(h.x, h.y);
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+	return wave_reduce(v, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+	return wave_reduce(v, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }

@@ -64,9 +64,9 @@ template <> struct SampleColor<false> {
 	__device__ __forceinline__ bool contributes() const { return enc != 0; }
 	__device__ __forceinline__ float4 rgba() const { return decode_rgba8(enc); }
 	__device__ __forceinline__ void zero() { enc = 0; }
-	__device__ __forceinline__ SampleColor shfl(int src) const {
+	__device__ __forceinline__ SampleColor read(int src) const {
 		SampleColor o;
-		o.enc = __shfl(enc, src, 64);
+		o.enc = wave_read(enc, src);
 		return o;
 	}
 };
@@ -83,10 +83,10 @@ template <> struct SampleColor<true> {
 	__device__ __forceinline__ bool contributes() const { return col.w != 0.0f; }
 	__device__ __forceinline__ float4 rgba() const { return col; }
 	__device__ __forceinline__ void zero() { col = make_float4(0, 0, 0, 0); }
-	__device__ __forceinline__ SampleColor shfl(int src) const {
+	__device__ __forceinline__ SampleColor read(int src) const {
 		SampleColor o;
-		o.col.x = __shfl(col.x, src, 64), o.col.y = __shfl(col.y, src, 64);
-		o.col.z = __shfl(col.z, src, 64), o.col.w = __shfl(col.w, src, 64);
+		o.col.x = wave_read(col.x, src), o.col.y = wave_read(col.y, src);
+		o.col.z = wave_read(col.z, src), o.col.w = wave_read(col.w, src);
 		return o;
 	}
 };
@@ -627,71 +627,80 @@ __device__ __forceinline__ void write_pixel(const FrameConst &c, const FrameBufs
 
 // ------------------------------------------------------------------ sorts
 
-__device__ __forceinline__ uint64_t shfl64(uint64_t v, int src) {
-	uint32_t lo = __shfl((uint32_t)v, src, 64), hi = __shfl((uint32_t)(v >> 32), src, 64);
-	return ((uint64_t)hi << 32) | lo;
+// Bitonic network on 64 * E keys held by one wave (key e * 64 + lane of the block in v[e]).
+// Level K merges runs of K / 2 keys in steps J = K / 2 .. 1, each pairing indices i and i ^ J,
+// ascending where (i & K) == 0. A step within a wave is an exchange and one median: of the pair
+// and a bound, 0 keeps the smaller key and ~0 the larger, so the lane mask of the upper partner
+// and the direction fold into the bound (a constant of the step). The block sorts were bound by
+// the LDS pipe when the exchanges went through ds_bpermute_b32 (high_finalize, before -> after:
+// 1 M soup triangles at 1080p 124 -> 89 us, 5.2 M mesh triangles at 1440p 272 -> 193 us).
+__device__ __forceinline__ uint32_t med3_u32(uint32_t a, uint32_t b, uint32_t c) {
+	return max(min(a, b), min(max(a, b), c));
 }
-__device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m) {
-	uint32_t lo = __shfl_xor((uint32_t)v, m, 64), hi = __shfl_xor((uint32_t)(v >> 32), m, 64);
-	return ((uint64_t)hi << 32) | lo;
+// Lanes l of a wave with (l & J) != 0.
+constexpr uint64_t upper_lanes(int J) {
+	uint64_t m = 0;
+	for(int l = 0; l < 64; l++)
+		m |= (l & J) ? 1ull << l : 0ull;
+	return m;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_key(uint64_t v, int m) { return shfl_xor64(v, m); }
-__device__ __forceinline__ uint32_t shfl_xor_key(uint32_t v, int m) { return __shfl_xor(v, m, 64); }
-
-// Ascending bitonic sort of 64*E keys held in registers; element i = e * 64 + lane.
-// Bitonic network steps j = j_start .. 1 of merge level k on 64 * E keys (K: 32- or 64-bit)
-// held by one wave (key e * 64 + lane of the block in v[e]); `base` is the block's index in
-// the whole sequence, which decides each pair's direction: ascending iff (index & k) == 0.
-template <int E, class K>
-__device__ __forceinline__ void bitonic_regs_steps(K (&v)[E], uint32_t base, uint32_t k,
-												   int j_start) {
-	const int lane = lane_id();
+// Steps J, J / 2 .. 1 of level K; K = 0: ascending everywhere (the last level of a sort).
+template <int E, int K, int J> __device__ __forceinline__ void bitonic_steps(uint32_t (&v)[E]) {
+	if constexpr(J >= 64) {
 #pragma unroll
-	for(int j = 64 * E / 2; j > 0; j >>= 1) {
-		if(j > j_start)
-			continue;
-		if(j >= 64) {
-			const int jr = j / 64;
-#pragma unroll
-			for(int e = 0; e < E; e++) {
-				if((e & jr) == 0) {
-					const int pe = e | jr;
-					const bool asc = ((base + (uint32_t)(e * 64 + lane)) & k) == 0;
-					K a = v[e], bb = v[pe];
-					bool sw = (a > bb) == asc;
-					v[e] = sw ? bb : a;
-					v[pe] = sw ? a : bb;
-				}
+		for(int e = 0; e < E; e++) {
+			if((e & (J / 64)) == 0) {
+				const int pe = e | (J / 64);
+				const uint32_t mn = min(v[e], v[pe]), mx = max(v[e], v[pe]);
+				const bool desc = ((e * 64) & K) != 0;
+				v[e] = desc ? mx : mn;
+				v[pe] = desc ? mn : mx;
 			}
-		} else {
+		}
+	} else {
 #pragma unroll
-			for(int e = 0; e < E; e++) {
-				const uint32_t i = base + (uint32_t)(e * 64 + lane);
-				K p = shfl_xor_key(v[e], j);
-				bool asc = (i & k) == 0;
-				bool lower = (lane & j) == 0;
-				K mn = v[e] < p ? v[e] : p, mx = v[e] < p ? p : v[e];
-				v[e] = (asc == lower) ? mn : mx;
+		for(int e = 0; e < E; e++) {
+			const uint64_t desc = K == 0 ? 0ull : K < 64 ? upper_lanes(K) : ((e * 64) & K) ? ~0ull : 0ull;
+			const uint32_t bound = __builtin_amdgcn_inverse_ballot_w64(upper_lanes(J) ^ desc) ? ~0u : 0u;
+			if constexpr(J >= 16) {
+				const LanePair p = lane_pair<J>(v[e]);
+				v[e] = med3_u32(p.x, p.y, bound);
+			} else {
+				v[e] = med3_u32(v[e], lane_xor<J>(v[e]), bound);
 			}
 		}
 	}
+	if constexpr(J > 1)
+		bitonic_steps<E, K, J / 2>(v);
 }
 
-// Bitonic sort levels k = 2 .. 64 * E of a 64 * E block starting at index `base` of a longer
-// sequence (ascending for base = 0 alone; alternating directions per block otherwise, as the
-// network's later levels expect).
-template <int E, class K>
-__device__ __forceinline__ void bitonic_regs_from(K (&v)[E], uint32_t base) {
+// Steps J .. 1 of a level beyond the block (every pair in the block has the same direction):
+// ascending for flip = 0, descending for ~0 (the complements ascend).
+template <int E, int J>
+__device__ __forceinline__ void bitonic_merge(uint32_t (&v)[E], uint32_t flip) {
 #pragma unroll
-	for(int k = 2; k <= 64 * E; k <<= 1)
-		bitonic_regs_steps<E>(v, base, (uint32_t)k, k >> 1);
+	for(int e = 0; e < E; e++)
+		v[e] ^= flip;
+	bitonic_steps<E, 0, J>(v);
+#pragma unroll
+	for(int e = 0; e < E; e++)
+		v[e] ^= flip;
 }
 
-// Ascending bitonic sort of 64 * E keys held by one wave (key e * 64 + lane in v[e]).
-template <int E, class K>
-__device__ __forceinline__ void bitonic_regs(K (&v)[E]) {
-	bitonic_regs_from<E>(v, 0u);
+// Levels K .. 32 * E of a block (the direction depends on the index within it).
+template <int E, int K> __device__ __forceinline__ void bitonic_levels(uint32_t (&v)[E]) {
+	if constexpr(K < 64 * E) {
+		bitonic_steps<E, K, K / 2>(v);
+		bitonic_levels<E, 2 * K>(v);
+	}
+}
+
+// Sorts the block: ascending for flip = 0, descending for flip = ~0 (as the levels of a longer
+// sequence expect of every second block).
+template <int E> __device__ __forceinline__ void bitonic_regs(uint32_t (&v)[E], uint32_t flip = 0u) {
+	bitonic_levels<E, 2>(v);
+	bitonic_merge<E, 32 * E>(v, flip);
 }
 
 // Ascending bitonic sort of P (power of two) keys in LDS by one wave.
@@ -783,20 +792,6 @@ struct DepthGrid {
 	}
 	__device__ __forceinline__ uint32_t rank(uint32_t key) const { return (key - lo) >> shift; }
 };
-
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#pragma unroll
-	for(int m = 1; m < 64; m <<= 1)
-		v = min(v, (uint32_t)__shfl_xor(v, m, 64));
-	return v;
-}
-
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-	for(int m = 1; m < 64; m <<= 1)
-		v = max(v, (uint32_t)__shfl_xor(v, m, 64));
-	return v;
-}
 
 // Depth order of a block list of m <= 256 entries, sorted by one wave in registers: sorted
 // entry 64 k + lane is list position pos[k]. Keys are (24-bit depth rank << 8 | position).
@@ -891,7 +886,7 @@ __device__ __forceinline__ void enqueue_pixels(const FrameBufs &b, uint32_t slot
 	uint32_t base = 0;
 	if(lane == 0)
 		base = atomicAdd(&b.ctrl[kCtrlFallbackCount], (uint32_t)__popcll(sel));
-	base = __shfl(base, 0, 64);
+	base = wave_read(base, 0);
 	if(mine) {
 		const uint32_t i = base + (uint32_t)__popcll(sel & ((1ull << lane) - 1ull));
 		if(i < b.fallback_cap)
@@ -1453,7 +1448,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	}
 	lo = wave_min_u32(lo);
 	hi = wave_max_u32(hi);
-	mine = __shfl(wave_inclusive_add(mine), 63, 64);
+	mine = wave_read(wave_inclusive_add(mine), 63);
 	if(lane_s == 0)
 		s_lo[wave_s] = lo, s_hi[wave_s] = hi, s_wsum[1][wave_s] = mine;
 	__syncthreads();
@@ -1481,7 +1476,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 			const uint32_t j = ch * 256 + e * 64 + lane_s;
 			v[e] = j < m ? (grid.rank(s_key[j]) << pb) | j : ~0u;
 		}
-		bitonic_regs_from<4>(v, ch * 256);
+		bitonic_regs<4>(v, (ch & 1u) ? ~0u : 0u); // (alternating chunks for the next level)
 #pragma unroll
 		for(int e = 0; e < 4; e++)
 			s_key[ch * 256 + e * 64 + lane_s] = v[e];
@@ -1506,7 +1501,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 #pragma unroll
 			for(int e = 0; e < 4; e++)
 				v[e] = s_key[ch * 256 + e * 64 + lane_s];
-			bitonic_regs_steps<4>(v, ch * 256, k, 128);
+			bitonic_merge<4, 128>(v, ((ch * 256) & k) ? ~0u : 0u);
 #pragma unroll
 			for(int e = 0; e < 4; e++)
 				s_key[ch * 256 + e * 64 + lane_s] = v[e];
@@ -1690,31 +1685,41 @@ __global__ __launch_bounds__(kSortThreads) void high_finalize_long_kernel_batch(
 // the off-diagonal s x s blocks: the lower lane keeps its columns with (j & s) == 0 and
 // takes the partner's as columns j + s, the upper lane keeps its columns with (j & s) != 0
 // and takes the partner's, shifted down by s (Hacker's Delight, 7-3, one row per lane).
+// Stages 32 and 16 are row swaps of whole words and of packed halves; stage 8 picks bytes; the
+// others rotate the partner's word into place and merge it under a column mask, both chosen by
+// the lane's bit s.
 __device__ __forceinline__ uint64_t transpose64(uint64_t row) {
-	const int lane = lane_id();
-	{ // s = 32: whole 32-bit words
-		uint32_t lo = (uint32_t)row, hi = (uint32_t)(row >> 32);
-		const bool upper = (lane & 32) != 0;
-		const uint32_t got = __shfl_xor(upper ? lo : hi, 32, 64);
-		lo = upper ? got : lo;
-		hi = upper ? hi : got;
-		row = ((uint64_t)hi << 32) | lo;
-	}
-	constexpr uint64_t kM0[5] = {0x0000ffff0000ffffull, 0x00ff00ff00ff00ffull,
-								 0x0f0f0f0f0f0f0f0full, 0x3333333333333333ull,
-								 0x5555555555555555ull};
-	// Selects only (the lane condition is a wave-constant lane mask; the column masks and
-	// shifts are constants), so nothing lane-dependent stays live between calls.
+	int lane = lane_id();
+	// The lane's selectors are made here on every call (a dozen instructions): kept across the
+	// slice loops they cost a wave per SIMD (fp32 block_raster_big 130 registers instead of 128,
+	// 241 us instead of 204 for 41 M fragments at 512 x 512).
+	asm volatile("" : "+v"(lane));
+	const auto w32 = __builtin_amdgcn_permlane32_swap((uint32_t)row, (uint32_t)(row >> 32), false, false);
+	const uint32_t l16 = __builtin_amdgcn_perm(w32[1], w32[0], 0x05040100u); // the low halves
+	const uint32_t h16 = __builtin_amdgcn_perm(w32[1], w32[0], 0x07060302u); // the high halves
+	const auto w16 = __builtin_amdgcn_permlane16_swap(l16, h16, false, false);
+	uint32_t w[2] = {__builtin_amdgcn_perm(w16[1], w16[0], 0x05040100u),
+					 __builtin_amdgcn_perm(w16[1], w16[0], 0x07060302u)};
+	const uint32_t sel8 = (lane & 8) ? 0x03070105u : 0x06020400u;
 #pragma unroll
-	for(int st = 0; st < 5; st++) {
-		const int sh = 16 >> st;
-		const bool upper = (lane & sh) != 0;
-		const uint64_t lo_cols = row & kM0[st], hi_cols = row & ~kM0[st];
-		const uint64_t got = shfl_xor64(upper ? lo_cols : hi_cols, sh);
-		const uint64_t moved = upper ? got >> sh : got << sh;
-		row = (upper ? hi_cols : lo_cols) | moved;
-	}
-	return row;
+	for(int k = 0; k < 2; k++)
+		w[k] = __builtin_amdgcn_perm(lane_xor<8>(w[k]), w[k], sel8);
+	auto stage = [&](auto sh, uint32_t cols) {
+		constexpr int s = decltype(sh)::value;
+		const uint32_t upper = (lane & s) ? ~0u : 0u;
+		const uint32_t keep = cols ^ upper;
+		const uint32_t ror = ((32u - s) ^ upper) - upper; // down by s (upper lanes), else up
+#pragma unroll
+		for(int k = 0; k < 2; k++) {
+			const uint32_t p = lane_xor<s>(w[k]);
+			const uint32_t moved = __builtin_amdgcn_alignbit(p, p, ror);
+			w[k] = (w[k] & keep) | (moved & ~keep);
+		}
+	};
+	stage(std::integral_constant<int, 4>{}, 0x0f0f0f0fu);
+	stage(std::integral_constant<int, 2>{}, 0x33333333u);
+	stage(std::integral_constant<int, 1>{}, 0x55555555u);
+	return ((uint64_t)w[1] << 32) | w[0];
 }
 
 // Transposes the coverage masks of a slice (64-bit pixel masks, one per entry) into
@@ -1931,7 +1936,7 @@ __device__ __forceinline__ void finish_pixels(const FrameConst &c, const FrameBu
 	const bool on_screen = px < c.width && py < c.height;
 	write_pixel(c, b, px, py, acc, count);
 	enqueue_pixels(b, slot, bad && on_screen, px, py, false);
-	const uint32_t frags = __shfl(wave_inclusive_add(on_screen ? count : 0u), 63, 64);
+	const uint32_t frags = wave_read(wave_inclusive_add(on_screen ? count : 0u), 63);
 	if(lane == 0) {
 		atomicAdd(stat_stripe(b.ctrl, 0, slot % kStatStripes), frags);
 		if(m)
@@ -2240,7 +2245,7 @@ __device__ Accum blend_sorted(const FrameConst &c, const FrameBufs &b, const uin
 		}
 		const uint32_t cnt = min(64u, n - base);
 		for(uint32_t j = 0; j < cnt; j++) {
-			const SampleColor<FP32> c2 = col.shfl((int)j);
+			const SampleColor<FP32> c2 = col.read((int)j);
 			if(c2.contributes())
 				acc.blend(c2, additive);
 		}
@@ -2282,7 +2287,7 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 it
 				off = 0xffffffffu;
 			}
 		}
-		off = __shfl(off, 0, 64);
+		off = wave_read(off, 0);
 		if(off == 0xffffffffu)
 			return; // the frame reports an overflow and is rendered again
 		uint64_t *g = b.spill + off;
@@ -2317,7 +2322,7 @@ __device__ __forceinline__ void fallback_kernel_body(const FrameConst &c, const 
 		uint32_t v[2] = {*stat_stripe(b.ctrl, 0, threadIdx.x), *stat_stripe(b.ctrl, 1, threadIdx.x)};
 #pragma unroll
 		for(int k = 0; k < 2; k++) {
-			v[k] = __shfl(wave_inclusive_add(v[k]), 63, 64);
+			v[k] = wave_read(wave_inclusive_add(v[k]), 63);
 			if(threadIdx.x == 0 && v[k])
 				atomicAdd(&((lucid_info *)b.info)->stats[k], v[k]);
 		}
@@ -2986,7 +2991,7 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 				off = 0xffffffffu;
 			}
 		}
-		off = __shfl(off, 0, 64);
+		off = wave_read(off, 0);
 		if(off == 0xffffffffu)
 			return;
 		uint64_t *gk = b.spill + off;
@@ -3019,9 +3024,9 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 		const uint32_t cnt = min(64u, n - base);
 		for(uint32_t j = 0; j < cnt; j++) {
 			BwdSample s;
-			s.r = __shfl(smp.r, (int)j, 64), s.g = __shfl(smp.g, (int)j, 64);
-			s.b = __shfl(smp.b, (int)j, 64), s.a = __shfl(smp.a, (int)j, 64);
-			if(__shfl((int)ok, (int)j, 64))
+			s.r = wave_read(smp.r, (int)j), s.g = wave_read(smp.g, (int)j);
+			s.b = wave_read(smp.b, (int)j), s.a = wave_read(smp.a, (int)j);
+			if(wave_read((uint32_t)ok, (int)j))
 				tot.add(s.r, s.g, s.b, s.a);
 		}
 	}
@@ -3043,7 +3048,7 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 			base_row = 0xffffffffu;
 		}
 	}
-	base_row = __shfl(base_row, 0, 64);
+	base_row = wave_read(base_row, 0);
 	if(base_row == 0xffffffffu)
 		return;
 	const size_t row0 = (size_t)b.ctrl[kCtrlBwdRows] + base_row;
@@ -3062,12 +3067,12 @@ __device__ void bwd_fallback_pixel(const FrameConst &c, const FrameBufs &b, cons
 			mine[k] = 0.0f;
 		for(uint32_t j = 0; j < cnt; j++) {
 			BwdSample s;
-			s.r = __shfl(smp.r, (int)j, 64), s.g = __shfl(smp.g, (int)j, 64);
-			s.b = __shfl(smp.b, (int)j, 64), s.a = __shfl(smp.a, (int)j, 64);
-			s.b0 = __shfl(smp.b0, (int)j, 64), s.b1 = __shfl(smp.b1, (int)j, 64);
-			s.dr = __shfl(smp.dr, (int)j, 64), s.dg = __shfl(smp.dg, (int)j, 64);
-			s.db = __shfl(smp.db, (int)j, 64), s.da = __shfl(smp.da, (int)j, 64);
-			if(__shfl((int)ok, (int)j, 64)) {
+			s.r = wave_read(smp.r, (int)j), s.g = wave_read(smp.g, (int)j);
+			s.b = wave_read(smp.b, (int)j), s.a = wave_read(smp.a, (int)j);
+			s.b0 = wave_read(smp.b0, (int)j), s.b1 = wave_read(smp.b1, (int)j);
+			s.dr = wave_read(smp.dr, (int)j), s.dg = wave_read(smp.dg, (int)j);
+			s.db = wave_read(smp.db, (int)j), s.da = wave_read(smp.da, (int)j);
+			if(wave_read((uint32_t)ok, (int)j)) {
 				float out[kGradWords];
 				bwd_fragment(t, q, gsel[0], gsel[1], gsel[2], s, out);
 				if((uint32_t)lane == j) {

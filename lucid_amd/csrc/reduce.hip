@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_tile_sums_kernel(const uint
 #pragma unroll
 	for(int k = 0; k < kScanItems; k++) // coalesced: item k of the tile's k-th row
 		sum += scan_load(in, n, base + (size_t)k * kScanThreads + threadIdx.x);
-	sum = __shfl(wave_inclusive_add(sum), 63, 64);
+	sum = wave_read(wave_inclusive_add(sum), 63);
 	if(lane_id() == 0)
 		s_wave[threadIdx.x >> 6] = sum;
 	__syncthreads();

@@ -405,7 +405,7 @@ __device__ __forceinline__ void setup_kernel_body(const FrameConst &c, const Fra
 	uint32_t base = 0;
 	if(lane_id() == 0 && large)
 		base = atomicAdd(large_cursor(b.ctrl, stripe), (uint32_t)__popcll(large));
-	base = __shfl(base, 0, 64);
+	base = wave_read(base, 0);
 	if(kind == 1) {
 		uint32_t rank = (uint32_t)__popcll(large & ((1ull << lane_id()) - 1ull));
 		b.large_list[(size_t)stripe * large_stripe_cap((uint32_t)c.num_quads) + base + rank] = q;

@@ -41,3 +41,12 @@ def test_promotion_threshold(oracle_mod, n):
     sc = scenes.block_stack(48, 40, n, center_px=(12, 12), size_px=6.0, seed=n)
     r, gpu, ref = _render_both(sc, oracle_mod)
     _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("n", [64, 65, 128, 129, 512, 513, 2048, 2049, 4097])
+def test_sort_lengths(oracle_mod, n):
+    """n triangles over one block, at the lengths where its sort takes another path: one, two and
+    four keys per lane, one 256-key chunk, several, and the long-list pass."""
+    sc = scenes.block_stack(48, 40, n, center_px=(12, 12), size_px=6.0, seed=n)
+    r, gpu, ref = _render_both(sc, oracle_mod)
+    _check(sc, gpu, ref, oracle_mod)

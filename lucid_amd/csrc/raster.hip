@@ -139,31 +139,54 @@ __device__ __forceinline__ LitChannel lit_channel(float x, float f, float fp) {
 // blended by its fraction; within a level, bilinear weights at u = s * size - 0.5 with the
 // texel indices wrapped (repeat). s is reduced to [0, 1] first (repeat is periodic).
 
-// First texel of `level`: the offsets are kernel arguments, picked with selects (no dynamic
-// indexing of an argument array).
-__device__ __forceinline__ uint32_t tex_level_offset(const TexDesc &t, int level) {
-	uint32_t off = 0;
+//
+// The mip levels of both atlases sit in a small LDS table (fill_tex_table), one row per atlas
+// and level: a lane picks its level's size and texels with two LDS loads. Selecting them from
+// the kernel arguments instead took a chain of fifteen compares and selects per level and atlas.
+// The filtering is bound by VALU issue (about 70 operations per level go into the bilinear
+// filter itself); 96 textured planes at 1024 x 768 (26 M fragments): 316 -> 256 us for the
+// block rasteriser.
+constexpr int kTexTable = 2 * 2 * kMaxTexLevels; // two uint4 per level, opaque atlas first
+// Row of a level: {width, height as floats, width, height}, {texels (64 bits), number of levels of
+// the atlas, its last level as a float}.
+
+__device__ __forceinline__ void fill_tex_table(const FrameBufs &b, uint4 *s_tex) {
+	const int i = threadIdx.x;
+	if(i < 2 * kMaxTexLevels) {
+		const int level = i % kMaxTexLevels;
+		const bool second = i >= kMaxTexLevels;
+		uint32_t off = 0; // (the offsets are kernel arguments: no dynamic indexing)
 #pragma unroll
-	for(int i = 1; i < kMaxTexLevels; i++)
-		off = level == i ? t.offset[i] : off;
-	return off;
+		for(int l = 1; l < kMaxTexLevels; l++)
+			off = level == l ? (second ? b.tex[1].offset[l] : b.tex[0].offset[l]) : off;
+		const int w = max(1, (second ? b.tex[1].width : b.tex[0].width) >> level);
+		const int h = max(1, (second ? b.tex[1].height : b.tex[0].height) >> level);
+		const int levels = second ? b.tex[1].levels : b.tex[0].levels;
+		const uint64_t at = (uint64_t)((second ? b.tex[1].texels : b.tex[0].texels) + off);
+		s_tex[2 * i] = make_uint4(f2bits((float)w), f2bits((float)h), (uint32_t)w, (uint32_t)h);
+		s_tex[2 * i + 1] = make_uint4((uint32_t)at, (uint32_t)(at >> 32), (uint32_t)levels,
+									  f2bits((float)(levels - 1)));
+	}
 }
 
-__device__ __forceinline__ float4 tex_bilinear(const TexDesc &t, int level, float s, float v) {
-	const int w = max(1, t.width >> level), h = max(1, t.height >> level);
-	const uint32_t *texels = t.texels + tex_level_offset(t, level);
-	const float su = s - floorf(s), sv = v - floorf(v);
-	const float u = su * (float)w - 0.5f, uv = sv * (float)h - 0.5f;
+// The level of table rows l: su, sv are the texture coordinates reduced to [0, 1].
+__device__ __forceinline__ float4 tex_bilinear(const uint4 *l, float su, float sv) {
+	const uint4 d = l[0], at = l[1];
+	const int w = (int)d.z, h = (int)d.w;
+	const uint32_t *texels = (const uint32_t *)(((uint64_t)at.y << 32) | at.x);
+	const float u = su * bits2f(d.x) - 0.5f, uv = sv * bits2f(d.y) - 0.5f;
 	const float fu = floorf(u), fv = floorf(uv);
 	const float au = u - fu, av = uv - fv;
 	int x0 = (int)fu, y0 = (int)fv; // in [-1, size - 1]
 	x0 = x0 < 0 ? w - 1 : x0;
 	y0 = y0 < 0 ? h - 1 : y0;
-	const int x1 = x0 + 1 == w ? 0 : x0 + 1, y1 = y0 + 1 == h ? 0 : y0 + 1;
-	const float4 c00 = decode_rgba8(texels[(uint32_t)y0 * (uint32_t)w + (uint32_t)x0]);
-	const float4 c10 = decode_rgba8(texels[(uint32_t)y0 * (uint32_t)w + (uint32_t)x1]);
-	const float4 c01 = decode_rgba8(texels[(uint32_t)y1 * (uint32_t)w + (uint32_t)x0]);
-	const float4 c11 = decode_rgba8(texels[(uint32_t)y1 * (uint32_t)w + (uint32_t)x1]);
+	const int x1 = x0 + 1 == w ? 0 : x0 + 1;
+	const uint32_t row0 = (uint32_t)y0 * (uint32_t)w;
+	const uint32_t row1 = y0 + 1 == h ? 0u : row0 + (uint32_t)w;
+	const uint32_t t00 = texels[row0 + (uint32_t)x0], t10 = texels[row0 + (uint32_t)x1];
+	const uint32_t t01 = texels[row1 + (uint32_t)x0], t11 = texels[row1 + (uint32_t)x1];
+	const float4 c00 = decode_rgba8(t00), c10 = decode_rgba8(t10);
+	const float4 c01 = decode_rgba8(t01), c11 = decode_rgba8(t11);
 	const float bu = 1.0f - au, bv = 1.0f - av;
 	float4 r;
 	r.x = (c00.x * bu + c10.x * au) * bv + (c01.x * bu + c11.x * au) * av;
@@ -173,21 +196,24 @@ __device__ __forceinline__ float4 tex_bilinear(const TexDesc &t, int level, floa
 	return r;
 }
 
-__device__ float4 texture_grad(const TexDesc &t, float s, float v, float dsx, float dvx, float dsy,
-							   float dvy) {
-	const float fw = (float)t.width, fh = (float)t.height;
+// tab: the atlas's rows of the table.
+__device__ __forceinline__ float4 texture_grad(const uint4 *tab, float s, float v, float dsx,
+											   float dvx, float dsy, float dvy) {
+	const uint4 top = tab[0], meta = tab[1];
+	const float fw = bits2f(top.x), fh = bits2f(top.y);
 	const float ux = dsx * fw, vx = dvx * fh, uy = dsy * fw, vy = dvy * fh;
-	const float rho = fmx(sqrtf(ux * ux + vx * vx), sqrtf(uy * uy + vy * vy));
+	// the larger of the two lengths: the square root is monotonic, so one is enough
+	const float rho = sqrtf(fmx(ux * ux + vx * vx, uy * uy + vy * vy));
 	const float lambda = log2f(rho);
-	if(!(lambda > 0.0f)) // magnification (or a degenerate footprint): level 0
-		return tex_bilinear(t, 0, s, v);
-	const float d = fmn(lambda, (float)(t.levels - 1));
+	// magnification (or a degenerate footprint): level 0
+	const float d = lambda > 0.0f ? fmn(lambda, bits2f(meta.w)) : 0.0f;
 	const float fl = floorf(d);
 	const int lo = (int)fl;
 	const float delta = d - fl;
-	float4 r = tex_bilinear(t, lo, s, v);
+	const float su = s - floorf(s), sv = v - floorf(v);
+	float4 r = tex_bilinear(tab + 2 * lo, su, sv);
 	if(delta > 0.0f) {
-		const float4 h = tex_bilinear(t, min(lo + 1, t.levels - 1), s, v);
+		const float4 h = tex_bilinear(tab + 2 * min(lo + 1, (int)meta.z - 1), su, sv);
 		const float nd = 1.0f - delta;
 		r.x = r.x * nd + h.x * delta;
 		r.y = r.y * nd + h.y * delta;
@@ -201,9 +227,9 @@ __device__ float4 texture_grad(const TexDesc &t, float s, float v, float dsx, fl
 // derivatives from the planes one pixel right and one pixel down, the texture coordinate
 // and its derivatives from the triangle's corner coordinates, the instance's uv rectangle,
 // then the opaque (alpha 1) or transparent atlas. bary0/1: before the offsets are removed.
-__device__ __forceinline__ float4 albedo_sample(const FrameBufs &b, const uint4 *q, float inv_ray,
-												float e0, float e1, float bary0, float bary1,
-												float bp0, float bp1) {
+__device__ __forceinline__ float4 albedo_sample(const FrameBufs &b, const uint4 *s_tex,
+												const uint4 *q, float inv_ray, float e0, float e1,
+												float bary0, float bary1, float bp0, float bp1) {
 	const uint32_t flags = q[0].w & 0xffffu, inst = q[0].w >> 16, t = q[6].z;
 	const float dex = bits2f(q[0].x), dey = bits2f(q[0].y);
 	const float ray_posx = __builtin_amdgcn_rcpf(inv_ray + dex);
@@ -228,7 +254,7 @@ __device__ __forceinline__ float4 albedo_sample(const FrameBufs &b, const uint4 
 		dvx = dvx * rc.w, dvy = dvy * rc.w;
 	}
 	const bool opaque = (flags & LUCID_INST_TEX_OPAQUE) != 0;
-	float4 col = texture_grad(opaque ? b.tex[0] : b.tex[1], s, v, dsx, dvx, dsy, dvy);
+	float4 col = texture_grad(s_tex + (opaque ? 0 : 2 * kMaxTexLevels), s, v, dsx, dvx, dsy, dvy);
 	col.w = opaque ? 1.0f : col.w;
 	return col;
 }
@@ -261,7 +287,7 @@ struct ShadeState {
 
 template <bool TEX>
 __device__ __forceinline__ bool shade_prepare(const FrameConst &c, const FrameBufs &b,
-											  const uint4 *q, float px, float py, float inv_ray,
+											  const uint4 *s_tex, const uint4 *q, float px, float py, float inv_ray,
 											  ShadeState &st) {
 	const uint32_t flags = q[0].w & 0xffffu;
 	const uint4 b0 = q[1], b1 = q[2];
@@ -275,7 +301,7 @@ __device__ __forceinline__ bool shade_prepare(const FrameConst &c, const FrameBu
 	if constexpr(TEX) {
 		if(flags & LUCID_INST_HAS_ALBEDO_TEXTURE) {
 			textured = true;
-			tex = albedo_sample(b, q, inv_ray, e0, e1, bary0, bary1, bits2f(b0.w), bits2f(b1.w));
+			tex = albedo_sample(b, s_tex, q, inv_ray, e0, e1, bary0, bary1, bits2f(b0.w), bits2f(b1.w));
 		}
 	}
 	bary0 = bary0 - bits2f(b0.w);
@@ -358,11 +384,11 @@ __device__ __forceinline__ bool shade_prepare(const FrameConst &c, const FrameBu
 // of finalShading (funcs.glsl:261-271), then RGBA8 quantisation unless FP32.
 template <bool FP32, bool TEX>
 __device__ __forceinline__ SampleColor<FP32> shade_record(const FrameConst &c, const FrameBufs &b,
-														  const uint4 *q, float px, float py,
-														  float inv_ray) {
+														  const uint4 *s_tex, const uint4 *q,
+														  float px, float py, float inv_ray) {
 	ShadeState st;
 	SampleColor<FP32> out;
-	if(!shade_prepare<TEX>(c, b, q, px, py, inv_ray, st)) {
+	if(!shade_prepare<TEX>(c, b, s_tex, q, px, py, inv_ray, st)) {
 		out.zero();
 		return out;
 	}
@@ -387,11 +413,11 @@ __device__ __forceinline__ SampleColor<FP32> shade_record(const FrameConst &c, c
 // Shades triangle t at a pixel straight from the setup records (exact fallback path).
 template <bool FP32, bool TEX>
 __device__ __forceinline__ SampleColor<FP32> shade_sample(const FrameConst &c, const FrameBufs &b,
-														  uint32_t t, float px, float py,
-														  float inv_ray) {
+														  const uint4 *s_tex, uint32_t t,
+														  float px, float py, float inv_ray) {
 	uint4 q[kRecQuads];
 	load_shading_record(b, t, q);
-	return shade_record<FP32, TEX>(c, b, q, px, py, inv_ray);
+	return shade_record<FP32, TEX>(c, b, s_tex, q, px, py, inv_ray);
 }
 
 __device__ __forceinline__ uint64_t pixel_key(float inv_ray, uint32_t t) {
@@ -1873,8 +1899,9 @@ __device__ __forceinline__ void walk_bits(uint64_t (&bm)[W], Visit &&visit) {
 // carries no test of the blend options; otherwise they are read per sample.
 template <bool FP32, int W, int MODE, bool OVER, class PS>
 __device__ __forceinline__ void walk_pixel_t(const FrameConst &c, const FrameBufs &b,
-											 const uint4 *s_rec, uint64_t (&bm)[W], float px,
-											 float py, PS &ps, bool additive_opt) {
+											 const uint4 *s_rec, const uint4 *s_tex,
+											 uint64_t (&bm)[W], float px, float py, PS &ps,
+											 bool additive_opt) {
 	const bool unsorted = !OVER && (c.opts & LUCID_OPT_UNSORTED) != 0;
 	const bool additive = !OVER && additive_opt;
 	if constexpr(is_flat(MODE)) {
@@ -1898,7 +1925,7 @@ __device__ __forceinline__ void walk_pixel_t(const FrameConst &c, const FrameBuf
 		const uint4 *rec = s_rec + e * kRecQuads;
 		const uint4 q0 = rec[0];
 		const float inv = record_inv_depth(q0, px, py);
-		const SampleColor<FP32> col = shade_record<FP32, TEX>(c, b, rec, px, py, inv);
+		const SampleColor<FP32> col = shade_record<FP32, TEX>(c, b, s_tex, rec, px, py, inv);
 		if(col.contributes()) {
 			if(unsorted)
 				ps.acc.blend(col, additive); // list order, no depth order
@@ -1910,12 +1937,13 @@ __device__ __forceinline__ void walk_pixel_t(const FrameConst &c, const FrameBuf
 
 template <bool FP32, int W, int MODE, class PS>
 __device__ __forceinline__ void walk_pixel(const FrameConst &c, const FrameBufs &b,
-										   const uint4 *s_rec, uint64_t (&bm)[W], float px,
-										   float py, PS &ps, bool additive) {
+										   const uint4 *s_rec, const uint4 *s_tex,
+										   uint64_t (&bm)[W], float px, float py, PS &ps,
+										   bool additive) {
 	if(!additive && !(c.opts & LUCID_OPT_UNSORTED))
-		walk_pixel_t<FP32, W, MODE, true>(c, b, s_rec, bm, px, py, ps, false);
+		walk_pixel_t<FP32, W, MODE, true>(c, b, s_rec, s_tex, bm, px, py, ps, false);
 	else
-		walk_pixel_t<FP32, W, MODE, false>(c, b, s_rec, bm, px, py, ps, additive);
+		walk_pixel_t<FP32, W, MODE, false>(c, b, s_rec, s_tex, bm, px, py, ps, additive);
 }
 
 template <int W>
@@ -1976,6 +2004,10 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	}
 	if(b.ctrl[kCtrlRecorded])
 		return; // the recording pass A renders this block
+	constexpr bool TEX = MODE == kShadeTextured;
+	__shared__ uint4 s_tex[TEX ? kTexTable : 1];
+	if constexpr(TEX)
+		fill_tex_table(b, s_tex); // (one wave: the syncs before the first walk cover it)
 	const uint4 *list = b.blk_lists + sl.x;
 	uint64_t msk_all[4];
 	uint32_t tri_all[4];
@@ -2037,7 +2069,7 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 		if(opaque)
 			continue; // counted, not shaded
 		wave_sync_lds();
-		walk_pixel<FP32, W, MODE>(c, b, s_rec, bm, (float)px, (float)py, ps, additive);
+		walk_pixel<FP32, W, MODE>(c, b, s_rec, s_tex, bm, (float)px, (float)py, ps, additive);
 		wave_sync_lds(); // every lane is done with this slice's records
 		opaque = threshold && all_below_alpha_threshold(ps.acc.tr);
 	}
@@ -2099,6 +2131,12 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 	const int px0 = bin_x + bx * 8, py0 = bin_y + by * 8;
 	const int px = px0 + (lane & 7), py = py0 + (lane >> 3);
 	const bool additive = (c.opts & (1u << 5)) != 0;
+	constexpr bool TEX = MODE == kShadeTextured;
+	__shared__ uint4 s_tex[TEX ? kTexTable : 1];
+	if constexpr(TEX) {
+		fill_tex_table(b, s_tex);
+		__syncthreads();
+	}
 	if((uint32_t)wave < nw) {
 		const uint32_t e0 = hdr[1 + wave], e1 = hdr[2 + wave];
 		PixelState<FP32, MODE == kShadeFlatNarrow ? kNarrowBigWindow : kWindow> ps;
@@ -2124,7 +2162,7 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 			if(opaque)
 				continue; // counted, not shaded
 			wave_sync_lds();
-			walk_pixel<FP32, W, MODE>(c, b, s_rec[wave], bm, (float)px, (float)py, ps, additive);
+			walk_pixel<FP32, W, MODE>(c, b, s_rec[wave], s_tex, bm, (float)px, (float)py, ps, additive);
 			wave_sync_lds(); // every lane is done with this slice's records
 			// the range's own transmittance bounds the pixel's (earlier ranges only lower it)
 			opaque = threshold && all_below_alpha_threshold(ps.acc.tr);
@@ -2226,8 +2264,9 @@ __device__ uint32_t gather_pixel_keys(const FrameBufs &b, const uint4 *list, uin
 // Blends n sorted keys front to back: 64 samples are shaded in parallel, then composited
 // in order.
 template <bool FP32, bool TEX>
-__device__ Accum blend_sorted(const FrameConst &c, const FrameBufs &b, const uint64_t *keys,
-							  uint32_t n, float px, float py, bool global_src) {
+__device__ Accum blend_sorted(const FrameConst &c, const FrameBufs &b, const uint4 *s_tex,
+							  const uint64_t *keys, uint32_t n, float px, float py,
+							  bool global_src) {
 	const int lane = lane_id();
 	const bool additive = (c.opts & (1u << 5)) != 0;
 	Accum acc;
@@ -2241,7 +2280,7 @@ __device__ Accum blend_sorted(const FrameConst &c, const FrameBufs &b, const uin
 															  __HIP_MEMORY_SCOPE_AGENT)
 										  : keys[i];
 			const uint32_t t = (uint32_t)k;
-			col = shade_sample<FP32, TEX>(c, b, t, px, py, sample_inv_depth(b, t, px, py));
+			col = shade_sample<FP32, TEX>(c, b, s_tex, t, px, py, sample_inv_depth(b, t, px, py));
 		}
 		const uint32_t cnt = min(64u, n - base);
 		for(uint32_t j = 0; j < cnt; j++) {
@@ -2256,8 +2295,8 @@ __device__ Accum blend_sorted(const FrameConst &c, const FrameBufs &b, const uin
 // Exact path for one queued pixel: gathers its fragments from the block list, sorts the
 // keys (LDS bitonic up to kFallbackCap, else a global spill), shades and blends in order.
 template <bool FP32, bool TEX>
-__device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 item,
-							   uint64_t *s_keys) {
+__device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, const uint4 *s_tex,
+							   uint4 item, uint64_t *s_keys) {
 	const int lane = lane_id();
 	const uint32_t slot = item.x;
 	const int px = (int)item.y, py = (int)item.z;
@@ -2275,7 +2314,7 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 it
 			s_keys[i] = ~0ull;
 		wave_sync_lds();
 		bitonic_lds_wave(s_keys, P);
-		acc = blend_sorted<FP32, TEX>(c, b, s_keys, n, fx, fy, false);
+		acc = blend_sorted<FP32, TEX>(c, b, s_tex, s_keys, n, fx, fy, false);
 	} else {
 		// deep pixel: sort its keys in a global spill region
 		const uint32_t P = next_pow2(n);
@@ -2297,7 +2336,7 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, uint4 it
 		__threadfence();
 		__builtin_amdgcn_wave_barrier();
 		bitonic_global_wave(g, P);
-		acc = blend_sorted<FP32, TEX>(c, b, g, n, fx, fy, true);
+		acc = blend_sorted<FP32, TEX>(c, b, s_tex, g, n, fx, fy, true);
 	}
 	if(lane == 0) {
 		write_pixel(c, b, px, py, acc, n);
@@ -2328,10 +2367,15 @@ __device__ __forceinline__ void fallback_kernel_body(const FrameConst &c, const 
 		}
 	}
 	const uint32_t nq = min(b.ctrl[kCtrlFallbackCount], b.fallback_cap);
+	__shared__ uint4 s_tex[TEX ? kTexTable : 1];
+	if constexpr(TEX) {
+		fill_tex_table(b, s_tex);
+		__syncthreads();
+	}
 	const uint32_t waves = wg.count * (kFallbackThreads / 64);
 	const uint32_t w = wg.id * (kFallbackThreads / 64) + (threadIdx.x >> 6);
 	for(uint32_t qi = w; qi < nq; qi += waves)
-		fallback_pixel<FP32, TEX>(c, b, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
+		fallback_pixel<FP32, TEX>(c, b, s_tex, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
 }
 
 template <bool FP32, bool TEX>
@@ -2381,7 +2425,7 @@ struct BwdSample {
 __device__ __forceinline__ bool shade_grad(const FrameConst &c, const FrameBufs &b, const uint4 *q,
 										   float px, float py, float inv_ray, BwdSample &o) {
 	ShadeState st;
-	if(!shade_prepare<false>(c, b, q, px, py, inv_ray, st)) {
+	if(!shade_prepare<false>(c, b, nullptr, q, px, py, inv_ray, st)) {
 		o.zero();
 		return false;
 	}
@@ -2622,7 +2666,7 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 			walk_bits(bm, [&](int e) {
 				const uint4 *rec = s_rec[wave] + e * kRecQuads;
 				const float inv = record_inv_depth(rec[0], fx, fy);
-				const SampleColor<true> col = shade_record<true, false>(c, b, rec, fx, fy, inv);
+				const SampleColor<true> col = shade_record<true, false>(c, b, nullptr, rec, fx, fy, inv);
 				if(col.contributes()) {
 					BwdColor bc;
 					bc.r = col.col.x, bc.g = col.col.y, bc.b = col.col.z, bc.a = col.col.w;

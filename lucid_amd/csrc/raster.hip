@@ -10,9 +10,9 @@
 //   high_prep / high_finalize  allocation for high bins; long block lists are sorted by
 //                centroid depth (LDS bitonic, whole work-group) and split into depth ranges so
 //                that several waves share a dense block.
-//   block_raster one wave per block: sorts short lists itself in registers, expands coverage
-//                masks into dense 64-sample chunks, shades, routes samples to pixel lanes and
-//                blends front to back (block_raster_big: one wave per part of a sorted block).
+//   block_raster one wave per block: sorts short lists itself in registers, turns the coverage
+//                masks into per-pixel entry bitmaps, shades and blends front to back; pre-sorted
+//                blocks take one wave per depth range.
 //   fallback     exact per-pixel sort for pixels whose speculative order was violated.
 //
 // Exact ordering: triangles of a block are pre-sorted by the depth at their covered-pixel
@@ -1348,7 +1348,7 @@ __global__ __launch_bounds__(kRowgenThreads) void rowgen_high_kernel_batch(const
 constexpr int kSliceWords = 1;
 constexpr int kSliceEntries = 64 * kSliceWords;
 constexpr uint32_t kTieRun = 32; // longest run of equal block ranks put in exact order
-constexpr int kBigWaves = 4; // waves of block_raster_big_kernel / the backward block kernels
+constexpr int kBigWaves = 4; // waves of block_raster_kernel / the backward block kernels
 
 // Pre-sorted block layout in the sorted pool (offsets in words from an even base):
 //   [0] number of waves W, [1 .. W + 1] first entry of each wave's range (then m),
@@ -1670,7 +1670,7 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 }
 
 __global__ __launch_bounds__(kSortThreads) void high_finalize_kernel(FrameConst c, FrameBufs b) {
-	high_finalize_kernel_body<kMidSortCap>(c, b, WgPos{bin_run_id(blockIdx.x, gridDim.x), gridDim.x});
+	high_finalize_kernel_body<kMidSortCap>(c, b, WgPos{bin_run_id<16>(blockIdx.x, gridDim.x), gridDim.x});
 }
 
 // The long-list pass over the blocks queued by the first: work-group w of `count` takes
@@ -1691,7 +1691,7 @@ __global__ __launch_bounds__(kSortThreads) void high_finalize_long_kernel(FrameC
 __global__ __launch_bounds__(kSortThreads) void high_finalize_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
-	const uint32_t wg = bin_run_id(blockIdx.x, gridDim.x);
+	const uint32_t wg = bin_run_id<16>(blockIdx.x, gridDim.x);
 	const uint32_t f = batch_frame(sb, wg);
 	const FrameDesc &d = sb.frames[f];
 	high_finalize_kernel_body<kMidSortCap>(d.c, d.b, WgPos{wg - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
@@ -1717,7 +1717,7 @@ __global__ __launch_bounds__(kSortThreads) void high_finalize_long_kernel_batch(
 __device__ __forceinline__ uint64_t transpose64(uint64_t row) {
 	int lane = lane_id();
 	// The lane's selectors are made here on every call (a dozen instructions): kept across the
-	// slice loops they cost a wave per SIMD (fp32 block_raster_big 130 registers instead of 128,
+	// slice loops they cost a wave per SIMD (fp32 pre-sorted blocks 130 registers instead of 128,
 	// 241 us instead of 204 for 41 M fragments at 512 x 512).
 	asm volatile("" : "+v"(lane));
 	const auto w32 = __builtin_amdgcn_permlane32_swap((uint32_t)row, (uint32_t)(row >> 32), false, false);
@@ -1776,6 +1776,8 @@ __device__ __forceinline__ void transpose_masks(const uint64_t (&msk)[W], int nw
 constexpr int kFlatQuads = 5; // f0 depth plane | triangle id; f1-f3 r, g, b planes; f4 alpha
 constexpr bool is_flat(int mode) { return mode == kShadeFlat || mode == kShadeFlatNarrow; }
 constexpr int rec_quads(int mode) { return is_flat(mode) ? kFlatQuads : kRecQuads; }
+// LDS of one wave's slice of 64 W records
+template <int W, int MODE> constexpr int slice_quads() { return 64 * W * rec_quads(MODE); }
 
 __device__ __forceinline__ void make_flat_record(const uint4 *src, uint4 *dst) {
 	const uint4 q0 = src[0], q1 = src[1], q2 = src[2], q3 = src[3], q4 = src[4], q5 = src[5],
@@ -1974,14 +1976,12 @@ __device__ __forceinline__ void finish_pixels(const FrameConst &c, const FrameBu
 
 // One wave per block whose list fits the register sort (every low bin, most high blocks):
 // sorts the list by centroid depth in registers, then walks every pixel through it slice by
-// slice (each slice's shading records staged in LDS).
+// slice (each slice's shading records staged in LDS: s_rec, the wave's own).
 template <bool FP32, int W, int MODE>
-__device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
-		return;
-	__shared__ uint4 s_rec[(64 * W) * rec_quads(MODE)];
+__device__ __forceinline__ void raster_sorted_block(const FrameConst &c, const FrameBufs &b,
+													uint32_t slot, uint4 *s_rec,
+													const uint4 *s_tex) {
 	const int lane = lane_id();
-	const uint32_t slot = wg.id;
 	const int bin = slot >> 4, blk = slot & 15, by = blk >> 2, bx = blk & 3;
 	const int bin_x = (bin % c.bin_count_x) * kBinSize, bin_y = (bin / c.bin_count_x) * kBinSize;
 	const int px0 = bin_x + bx * 8, py0 = bin_y + by * 8;
@@ -1989,7 +1989,7 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	const uint32_t flags = b.blk_flags[slot];
 	const uint32_t level = flags & kSlotLevelMask;
 	if(flags & (kSlotWhole | kSlotPromoted | kSlotPresorted))
-		return; // fallback kernel, overflowed frame, or block_raster_big
+		return; // fallback kernel, overflowed frame, or the pre-sorted blocks' work-groups
 	Accum bg;
 	bg.init();
 	if(level == LUCID_BIN_LEVEL_EMPTY) {
@@ -2004,10 +2004,6 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	}
 	if(b.ctrl[kCtrlRecorded])
 		return; // the recording pass A renders this block
-	constexpr bool TEX = MODE == kShadeTextured;
-	__shared__ uint4 s_tex[TEX ? kTexTable : 1];
-	if constexpr(TEX)
-		fill_tex_table(b, s_tex); // (one wave: the syncs before the first walk cover it)
 	const uint4 *list = b.blk_lists + sl.x;
 	uint64_t msk_all[4];
 	uint32_t tri_all[4];
@@ -2024,7 +2020,8 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	} else {
 		// the sort leaves the masks and triangle ids by list position in the (not yet used)
 		// slice staging area; the lanes read them back in depth order
-		static_assert(sizeof(s_rec) >= kRegSortCap * (sizeof(uint64_t) + sizeof(uint32_t)),
+		static_assert(slice_quads<W, MODE>() * sizeof(uint4) >=
+						  kRegSortCap * (sizeof(uint64_t) + sizeof(uint32_t)),
 					  "the sort's masks and ids fit the staging area");
 		uint64_t *s_msk = reinterpret_cast<uint64_t *>(s_rec);
 		uint32_t *s_tri = reinterpret_cast<uint32_t *>(s_msk + kRegSortCap);
@@ -2077,34 +2074,21 @@ __device__ __forceinline__ void block_raster_kernel_body(const FrameConst &c, co
 	finish_pixels(c, b, ps.acc, ps.w.bad, count, px, py, slot, m);
 }
 
-template <bool FP32, int W, int MODE>
-__global__ __launch_bounds__(64) void block_raster_kernel(FrameConst c, FrameBufs b) {
-	block_raster_kernel_body<FP32, W, MODE>(c, b, WgPos{bin_run_id(blockIdx.x, gridDim.x), gridDim.x});
-}
-template <bool FP32, int W, int MODE>
-__global__ __launch_bounds__(64) void block_raster_kernel_batch(const FrameDesc *__restrict__ frames,
-		const uint32_t *__restrict__ pre, uint32_t num_frames) {
-	const StageBatch sb{frames, pre, num_frames};
-	const uint32_t wg = bin_run_id(blockIdx.x, gridDim.x);
-	const uint32_t f = batch_frame(sb, wg);
-	const FrameDesc &d = sb.frames[f];
-	block_raster_kernel_body<FP32, W, MODE>(d.c, d.b, WgPos{wg - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
-}
-
 // Pre-sorted lists longer than one register sort: one work-group per block. Wave w takes
 // the contiguous depth range [start[w], start[w + 1]) of the sorted list (ranges balanced
 // by sample count), walks it slice by slice with one ordering window per pixel, and leaves
 // a partial composite; wave 0 chains the partials front to back. A pixel is exact iff each
 // range's blended keys increase and every range starts behind the previous one's last key.
 template <bool FP32, int W, int MODE>
-__device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
-		return;
+__device__ __forceinline__ void raster_presorted_block(const FrameConst &c, const FrameBufs &b,
+													   uint32_t id,
+													   uint4 (&s_rec)[kBigWaves][slice_quads<W, MODE>()],
+													   const uint4 *s_tex) {
 	const lucid_info *info = (const lucid_info *)b.info;
-	const uint32_t hslot = wg.id >> 4;
+	const uint32_t hslot = id >> 4;
 	if(hslot >= (uint32_t)info->bin_level_counts[LUCID_BIN_LEVEL_HIGH])
 		return;
-	const int blk = wg.id & 15, by = blk >> 2, bx = blk & 3;
+	const int blk = id & 15, by = blk >> 2, bx = blk & 3;
 	const int bin = (int)b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + hslot];
 	const uint32_t slot = (uint32_t)bin * 16 + blk;
 	const uint32_t flags = b.blk_flags[slot];
@@ -2118,7 +2102,6 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 		uint64_t first[64], last[64];
 		uint32_t cnt[64]; // fragments | 0x80000000 when the range's order is not exact
 	};
-	__shared__ uint4 s_rec[kBigWaves][(64 * W) * rec_quads(MODE)];
 	static_assert(sizeof(RangeEnd) <= sizeof(s_rec[0]), "a range's end state fits its staging");
 	auto range_end = [&](int w) -> RangeEnd & { return *reinterpret_cast<RangeEnd *>(&s_rec[w][0]); };
 	const int wave = threadIdx.x >> 6, lane = lane_id();
@@ -2131,12 +2114,6 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 	const int px0 = bin_x + bx * 8, py0 = bin_y + by * 8;
 	const int px = px0 + (lane & 7), py = py0 + (lane >> 3);
 	const bool additive = (c.opts & (1u << 5)) != 0;
-	constexpr bool TEX = MODE == kShadeTextured;
-	__shared__ uint4 s_tex[TEX ? kTexTable : 1];
-	if constexpr(TEX) {
-		fill_tex_table(b, s_tex);
-		__syncthreads();
-	}
 	if((uint32_t)wave < nw) {
 		const uint32_t e0 = hdr[1 + wave], e1 = hdr[2 + wave];
 		PixelState<FP32, MODE == kShadeFlatNarrow ? kNarrowBigWindow : kWindow> ps;
@@ -2202,18 +2179,77 @@ __device__ __forceinline__ void block_raster_big_kernel_body(const FrameConst &c
 	finish_pixels(c, b, acc, bad, count, px, py, slot, m);
 }
 
+// Register-sorted blocks alone (one wave each) and pre-sorted blocks alone.
+template <bool FP32, int W, int MODE>
+__device__ __forceinline__ void block_raster_body(const FrameConst &c, const FrameBufs &b,
+												  uint32_t id) {
+	__shared__ uint4 s_rec[slice_quads<W, MODE>()];
+	__shared__ uint4 s_tex[MODE == kShadeTextured ? kTexTable : 1];
+	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
+		return;
+	if constexpr(MODE == kShadeTextured)
+		fill_tex_table(b, s_tex); // (one wave: the syncs before the first walk cover it)
+	raster_sorted_block<FP32, W, MODE>(c, b, id, s_rec, s_tex);
+}
+template <bool FP32, int W, int MODE>
+__device__ __forceinline__ void block_raster_big_body(const FrameConst &c, const FrameBufs &b,
+													  uint32_t id) {
+	__shared__ uint4 s_rec[kBigWaves][slice_quads<W, MODE>()];
+	__shared__ uint4 s_tex[MODE == kShadeTextured ? kTexTable : 1];
+	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
+		return;
+	if constexpr(MODE == kShadeTextured) {
+		fill_tex_table(b, s_tex);
+		__syncthreads();
+	}
+	raster_presorted_block<FP32, W, MODE>(c, b, id, s_rec, s_tex);
+}
+template <bool FP32, int W, int MODE>
+__global__ __launch_bounds__(64) void block_raster_kernel(FrameConst c, FrameBufs b) {
+	block_raster_body<FP32, W, MODE>(c, b, bin_run_id<16>(blockIdx.x, gridDim.x));
+}
+template <bool FP32, int W, int MODE>
+__global__ __launch_bounds__(64) void block_raster_kernel_batch(const FrameDesc *__restrict__ frames,
+		const uint32_t *__restrict__ pre, uint32_t num_frames) {
+	const StageBatch sb{frames, pre, num_frames};
+	const uint32_t wg = bin_run_id<16>(blockIdx.x, gridDim.x);
+	const uint32_t f = batch_frame(sb, wg);
+	const FrameDesc &d = sb.frames[f];
+	block_raster_body<FP32, W, MODE>(d.c, d.b, wg - sb.pre[f]);
+}
 template <bool FP32, int W, int MODE>
 __global__ __launch_bounds__(kBigWaves * 64) void block_raster_big_kernel(FrameConst c, FrameBufs b) {
-	block_raster_big_kernel_body<FP32, W, MODE>(c, b, WgPos{bin_run_id(blockIdx.x, gridDim.x), gridDim.x});
+	block_raster_big_body<FP32, W, MODE>(c, b, bin_run_id<16>(blockIdx.x, gridDim.x));
 }
 template <bool FP32, int W, int MODE>
 __global__ __launch_bounds__(kBigWaves * 64) void block_raster_big_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
-	const uint32_t wg = bin_run_id(blockIdx.x, gridDim.x);
+	const uint32_t wg = bin_run_id<16>(blockIdx.x, gridDim.x);
 	const uint32_t f = batch_frame(sb, wg);
 	const FrameDesc &d = sb.frames[f];
-	block_raster_big_kernel_body<FP32, W, MODE>(d.c, d.b, WgPos{wg - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
+	block_raster_big_body<FP32, W, MODE>(d.c, d.b, wg - sb.pre[f]);
+}
+
+// Both kinds in one launch, for frames of few blocks (kFusedRasterBins): the first 16 work-groups
+// per bin take the pre-sorted blocks, the others four register-sorted blocks each (one wave a
+// block, on its own quarter of the LDS), which fill the CUs that run out of the long ones. As two
+// launches each ends with a nearly empty chip. fp32 samples: four waves per SIMD, as apart.
+constexpr int kFusedRasterBins = 1024;
+static_assert(kBigWaves == 4, "a bin's 16 blocks are four work-groups of register-sorted blocks");
+template <bool FP32, int MODE>
+__global__ __launch_bounds__(kBigWaves * 64, FP32 ? 4 : 1) void block_raster_fused_kernel(FrameConst c, FrameBufs b) {
+	static_assert(MODE != kShadeTextured, "no texture table here");
+	__shared__ uint4 s_rec[kBigWaves][slice_quads<1, MODE>()];
+	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
+		return;
+	const uint32_t big = (uint32_t)c.bin_count * 16, w = blockIdx.x;
+	if(w < big) {
+		raster_presorted_block<FP32, 1, MODE>(c, b, bin_run_id<16>(w, big), s_rec, nullptr);
+	} else {
+		const uint32_t id = bin_run_id<4>(w - big, gridDim.x - big), wave = threadIdx.x >> 6;
+		raster_sorted_block<FP32, 1, MODE>(c, b, id * kBigWaves + wave, s_rec[wave], nullptr);
+	}
 }
 
 // ------------------------------------------------------------------ exact fallback
@@ -3156,6 +3192,35 @@ static void launch_high_finalize(const FrameConst &c, const FrameBufs &b, hipStr
 	hipLaunchKernelGGL(high_finalize_long_kernel, dim3(256), dim3(kSortThreads), 0, stream, c, b);
 }
 
+template <bool FP32, int W, int MODE>
+static void launch_block_raster_apart(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
+	hipLaunchKernelGGL((block_raster_kernel<FP32, W, MODE>), dim3(c.bin_count * 16), dim3(64), 0, stream,
+					   c, b);
+	hipLaunchKernelGGL((block_raster_big_kernel<FP32, W, MODE>), dim3(c.bin_count * 16),
+					   dim3(kBigWaves * 64), 0, stream, c, b);
+}
+
+// Frames of up to kFusedRasterBins bins take one launch (two -> one: 767 x 431 particles 336
+// bins, 79 -> 64 us; 1280 x 720 lit mesh, 920 bins, 104 -> 99 us; 512 x 512 preview, 18 -> 15 us).
+// Larger ones fill the chip either way, and the register-sorted blocks are better off as
+// work-groups of their own (1080p soup, 2040 bins, 198 -> 199 us; 1440p mesh, 3600 bins, 336 ->
+// 365 us), as are textured ones, whose blocks differ most in length (768 bins, 261 -> 269 us).
+template <bool FP32, int MODE>
+static void launch_block_raster(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
+	if constexpr(MODE != kShadeTextured) {
+		if(c.slice_words == 1 && c.bin_count <= kFusedRasterBins) {
+			hipLaunchKernelGGL((block_raster_fused_kernel<FP32, MODE>),
+							   dim3(c.bin_count * (16 + 16 / kBigWaves)), dim3(kBigWaves * 64), 0, stream,
+							   c, b);
+			return;
+		}
+	}
+	if(c.slice_words == 2)
+		launch_block_raster_apart<FP32, 2, MODE>(c, b, stream);
+	else
+		launch_block_raster_apart<FP32, 1, MODE>(c, b, stream);
+}
+
 template <bool FP32, int MODE>
 static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 							hipEvent_t *ev) {
@@ -3169,17 +3234,7 @@ static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t
 	launch_high_finalize(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[1], stream);
-	if(c.slice_words == 2) {
-		hipLaunchKernelGGL((block_raster_kernel<FP32, 2, MODE>), dim3(c.bin_count * 16), dim3(64), 0,
-						   stream, c, b);
-		hipLaunchKernelGGL((block_raster_big_kernel<FP32, 2, MODE>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b);
-	} else {
-		hipLaunchKernelGGL((block_raster_kernel<FP32, 1, MODE>), dim3(c.bin_count * 16), dim3(64), 0,
-						   stream, c, b);
-		hipLaunchKernelGGL((block_raster_big_kernel<FP32, 1, MODE>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b);
-	}
+	launch_block_raster<FP32, MODE>(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[2], stream);
 	hipLaunchKernelGGL((fallback_kernel<FP32, TEX>), dim3(1024), dim3(kFallbackThreads), 0, stream,
@@ -3320,17 +3375,7 @@ hipError_t launch_raster_recording(const FrameConst &c, const FrameBufs &b, cons
 	else
 		hipLaunchKernelGGL((bwd_pass_a_kernel<true, kWindow>), dim3(c.bin_count * 16),
 						   dim3(kBigWaves * 64), 0, stream, c, b, g);
-	if(c.slice_words == 2) {
-		hipLaunchKernelGGL((block_raster_kernel<true, 2, kShadeGeneral>), dim3(c.bin_count * 16), dim3(64), 0,
-						   stream, c, b);
-		hipLaunchKernelGGL((block_raster_big_kernel<true, 2, kShadeGeneral>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b);
-	} else {
-		hipLaunchKernelGGL((block_raster_kernel<true, 1, kShadeGeneral>), dim3(c.bin_count * 16), dim3(64), 0,
-						   stream, c, b);
-		hipLaunchKernelGGL((block_raster_big_kernel<true, 1, kShadeGeneral>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b);
-	}
+	launch_block_raster<true, kShadeGeneral>(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[2], stream);
 	hipLaunchKernelGGL((fallback_kernel<true, false>), dim3(1024), dim3(kFallbackThreads), 0, stream,

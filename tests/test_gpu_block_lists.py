@@ -50,3 +50,20 @@ def test_sort_lengths(oracle_mod, n):
     sc = scenes.block_stack(48, 40, n, center_px=(12, 12), size_px=6.0, seed=n)
     r, gpu, ref = _render_both(sc, oracle_mod)
     _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("opts", [0, _lib.OPT_FP32_SAMPLES])
+@pytest.mark.parametrize("w,h", [(1024, 1024), (1025, 1024)])
+def test_raster_launch_threshold(oracle_mod, w, h, opts):
+    """Frames at and just beyond the bin count up to which both kinds of blocks share a launch
+    (1024 bins), with register-sorted and pre-sorted blocks: two stacks of different heights."""
+    a = scenes.block_stack(w, h, 90, center_px=(500, 300), size_px=30.0, seed=1)
+    b = scenes.block_stack(w, h, 1500, center_px=(w - 9, h - 9), size_px=9.0, seed=2)
+    n = a.num_verts
+    sc = scenes.block_stack(w, h, 1590, seed=3)
+    sc.positions = np.concatenate([a.positions, b.positions])
+    sc.colors_rgb = np.concatenate([a.colors_rgb, b.colors_rgb])
+    sc.tri_alpha = np.concatenate([a.tri_alpha, b.tri_alpha])
+    assert n + b.num_verts == sc.num_verts
+    r, gpu, ref = _render_both(sc, oracle_mod, opts=opts)
+    _check(sc, gpu, ref, oracle_mod)

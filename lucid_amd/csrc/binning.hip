@@ -177,125 +177,110 @@ __global__ __launch_bounds__(kBinThreads) void bin_count_kernel_batch(const Fram
 	bin_count_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
 }
 
-// Per bin: totals over work-groups and each work-group's exclusive offset inside the bin.
-// Exclusive scan of the per-work-group bin histograms down each (kind, bin) column, and the
-// column totals (the bin counts). A work-group takes 16 columns; its 16 row-parts each sum
-// a run of rows with independent loads, an LDS scan joins the parts, then each part writes
-// its exclusive prefixes.
-constexpr int kScanCols = 16, kScanParts = 16;
-__device__ __forceinline__ void bin_wg_scan_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	const int NB = c.bin_count, nw = c.num_bin_wgs;
-	const int col_l = threadIdx.x % kScanCols, part = threadIdx.x / kScanCols;
-	const int col = wg.id * kScanCols + col_l; // 0 .. 2 NB: quads then tris
-	const int rows = (nw + kScanParts - 1) / kScanParts; // <= 16: num_bin_wgs <= 256
-	const int w0 = part * rows, w1 = min(nw, w0 + rows);
-	__shared__ uint32_t s_part[kScanParts][kScanCols];
-	uint32_t sum = 0;
-	if(col < 2 * NB)
-		for(int w = w0; w < w1; w++)
-			sum += b.wg_hist[(size_t)w * 2 * NB + col];
-	s_part[part][col_l] = sum;
-	__syncthreads();
-	if(part == 0) {
-		uint32_t run = 0;
-		for(int p = 0; p < kScanParts; p++) {
-			uint32_t v = s_part[p][col_l];
-			s_part[p][col_l] = run;
-			run += v;
-		}
-		if(col < 2 * NB) {
-			const int k = col / NB, bin = col - k * NB;
-			uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
-			counts[(k == 0 ? LUCID_COUNTS_QUAD_COUNTS : LUCID_COUNTS_TRI_COUNTS) * NB + bin] = run;
-		}
-	}
-	__syncthreads();
-	if(col >= 2 * NB)
-		return;
-	// all loads first (independent), then the stores: a part spans at most kMaxRows rows
-	constexpr int kMaxRows = 16;
-	uint32_t v[kMaxRows];
-#pragma unroll
-	for(int j = 0; j < kMaxRows; j++)
-		v[j] = w0 + j < w1 ? b.wg_hist[(size_t)(w0 + j) * 2 * NB + col] : 0u;
-	uint32_t run = s_part[part][col_l];
-#pragma unroll
-	for(int j = 0; j < kMaxRows; j++) {
-		if(w0 + j < w1)
-			b.wg_hist[(size_t)(w0 + j) * 2 * NB + col] = run;
-		run += v[j];
-	}
-}
+constexpr int kScanCols = 16, kScanParts = 16, kScanThreads = kScanCols * kScanParts;
 
-__global__ __launch_bounds__(kScanCols * kScanParts) void bin_wg_scan_kernel(FrameConst c, FrameBufs b) {
-	bin_wg_scan_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
-}
-__global__ __launch_bounds__(kScanCols * kScanParts) void bin_wg_scan_kernel_batch(const FrameDesc *__restrict__ frames,
-		const uint32_t *__restrict__ pre, uint32_t num_frames) {
-	const StageBatch sb{frames, pre, num_frames};
-	const uint32_t f = batch_frame(sb, blockIdx.x);
-	const FrameDesc &d = sb.frames[f];
-	bin_wg_scan_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
-}
-
-// bin_categorizer.glsl: exclusive offsets over bins, bin levels and level lists.
-__device__ __forceinline__ void bin_categorize_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
+// bin_categorizer.glsl: exclusive offsets over bins, bin levels and level lists; and the list
+// space of every high bin (16 lists of its triangle count each, which row generation fills).
+// One work-group; a wave takes a run of consecutive bins, 64 at a time: sums, one scan over the
+// waves, then the offsets.
+__device__ __forceinline__ void categorize_bins(const FrameConst &c, const FrameBufs &b) {
 	const int NB = c.bin_count;
 	uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
 	lucid_info *info = (lucid_info *)b.info;
-	__shared__ uint32_t s_wave[16][4];
-	__shared__ uint32_t s_carry[4];
-	if(threadIdx.x < 4)
-		s_carry[threadIdx.x] = 0;
+	const uint32_t *qcs = counts + LUCID_COUNTS_QUAD_COUNTS * NB, *tcs = counts + LUCID_COUNTS_TRI_COUNTS * NB;
+	constexpr int kWaves = kScanThreads / 64;
+	__shared__ uint32_t s_wave[kWaves][5];
+	const int wave = threadIdx.x >> 6, lane = lane_id();
+	const int run = (NB + 64 * kWaves - 1) / (64 * kWaves) * 64;
+	const int b0 = wave * run, b1 = min(NB, b0 + run);
+	// the counts of kAhead steps, whose loads are in flight together
+	constexpr int kAhead = 8;
+	uint32_t q[kAhead], t[kAhead];
+	auto load = [&](int i) {
+#pragma unroll
+		for(int j = 0; j < kAhead; j++) {
+			const int bin = i + j * 64 + lane;
+			q[j] = bin < b1 ? agent_load(qcs + bin) : 0u;
+			t[j] = bin < b1 ? agent_load(tcs + bin) : 0u;
+		}
+	};
+	// quads, triangles, low bins, high bins, triangles of the high bins
+	auto values = [&](uint32_t qc, uint32_t tc, uint32_t (&v)[5]) {
+		const uint32_t n = tc + 2 * qc;
+		const bool high = n >= (uint32_t)kLowLevelLimit;
+		v[0] = qc, v[1] = tc;
+		v[2] = n > 0 && !high ? 1u : 0u;
+		v[3] = high ? 1u : 0u;
+		v[4] = high ? n : 0u;
+	};
+	uint32_t ex[5] = {0u, 0u, 0u, 0u, 0u}, total[5];
+	for(int i = b0; i < b1; i += 64 * kAhead) {
+		load(i);
+#pragma unroll
+		for(int j = 0; j < kAhead; j++) {
+			uint32_t v[5];
+			values(q[j], t[j], v);
+#pragma unroll
+			for(int k = 0; k < 5; k++)
+				ex[k] += v[k];
+		}
+	}
+#pragma unroll
+	for(int k = 0; k < 5; k++) {
+		const uint32_t sum = wave_read(wave_inclusive_add(ex[k]), 63);
+		if(lane == 0)
+			s_wave[wave][k] = sum;
+	}
 	__syncthreads();
-	int wave = threadIdx.x >> 6;
-	for(int base = 0; base < NB; base += 1024) {
-		int bin = base + threadIdx.x;
-		uint32_t qc = bin < NB ? counts[LUCID_COUNTS_QUAD_COUNTS * NB + bin] : 0u;
-		uint32_t tc = bin < NB ? counts[LUCID_COUNTS_TRI_COUNTS * NB + bin] : 0u;
-		uint32_t ntris = tc + 2 * qc;
-		uint32_t vals[4] = {qc, tc, (bin < NB && ntris > 0 && ntris < (uint32_t)kLowLevelLimit) ? 1u : 0u,
-							(bin < NB && ntris >= (uint32_t)kLowLevelLimit) ? 1u : 0u};
-		uint32_t inc[4];
 #pragma unroll
-		for(int k = 0; k < 4; k++) {
-			inc[k] = wave_inclusive_add(vals[k]);
-			if(lane_id() == 63)
-				s_wave[wave][k] = inc[k];
+	for(int k = 0; k < 5; k++) {
+		total[k] = ex[k] = 0;
+#pragma unroll
+		for(int w = 0; w < kWaves; w++) {
+			ex[k] += w < wave ? s_wave[w][k] : 0u;
+			total[k] += s_wave[w][k];
 		}
-		__syncthreads();
-		if(threadIdx.x < 4) {
-			uint32_t run = s_carry[threadIdx.x];
-			for(int w = 0; w < 16; w++) {
-				uint32_t v = s_wave[w][threadIdx.x];
-				s_wave[w][threadIdx.x] = run;
-				run += v;
+	}
+	const uint64_t list0 = (uint64_t)NB * 16 * kRegSortCap;
+	const bool fits = list0 + 16ull * total[4] <= b.blk_lists_cap;
+	for(int i = b0; i < b1; i += 64 * kAhead) {
+		load(i);
+#pragma unroll
+		for(int j = 0; j < kAhead; j++) {
+			const int bin = i + j * 64 + lane;
+			uint32_t v[5], at[5];
+			values(q[j], t[j], v);
+#pragma unroll
+			for(int k = 0; k < 5; k++) {
+				const uint32_t inc = wave_inclusive_add(v[k]);
+				at[k] = ex[k] + inc - v[k];
+				ex[k] += wave_read(inc, 63);
 			}
-			s_carry[threadIdx.x] = run;
+			if(bin < b1) {
+				counts[LUCID_COUNTS_QUAD_OFFSETS * NB + bin] = at[0];
+				counts[LUCID_COUNTS_QUAD_OFFSETS_TEMP * NB + bin] = at[0] + v[0];
+				counts[LUCID_COUNTS_TRI_OFFSETS * NB + bin] = at[1];
+				counts[LUCID_COUNTS_TRI_OFFSETS_TEMP * NB + bin] = at[1] + v[1];
+				if(v[2])
+					counts[LUCID_COUNTS_LOW_BINS * NB + at[2]] = (uint32_t)bin;
+				if(v[3]) {
+					counts[LUCID_COUNTS_HIGH_BINS * NB + at[3]] = (uint32_t)bin;
+					b.blk_slot[(size_t)bin * 16] = make_uint2((uint32_t)(list0 + 16ull * at[4]), 0u);
+				}
+			}
 		}
-		__syncthreads();
-		if(bin < NB) {
-			uint32_t ex[4];
-#pragma unroll
-			for(int k = 0; k < 4; k++)
-				ex[k] = s_wave[wave][k] + inc[k] - vals[k];
-			counts[LUCID_COUNTS_QUAD_OFFSETS * NB + bin] = ex[0];
-			counts[LUCID_COUNTS_QUAD_OFFSETS_TEMP * NB + bin] = ex[0] + qc;
-			counts[LUCID_COUNTS_TRI_OFFSETS * NB + bin] = ex[1];
-			counts[LUCID_COUNTS_TRI_OFFSETS_TEMP * NB + bin] = ex[1] + tc;
-			if(vals[2])
-				counts[LUCID_COUNTS_LOW_BINS * NB + ex[2]] = (uint32_t)bin;
-			if(vals[3])
-				counts[LUCID_COUNTS_HIGH_BINS * NB + ex[3]] = (uint32_t)bin;
-		}
-		__syncthreads();
 	}
 	if(threadIdx.x == 0) {
-		uint32_t nq = s_carry[0], nt = s_carry[1], nlow = s_carry[2], nhigh = s_carry[3];
+		const uint32_t nq = total[0], nt = total[1], nlow = total[2], nhigh = total[3];
 		b.ctrl[kCtrlTotalBinQuads] = nq;
 		b.ctrl[kCtrlTotalBinTris] = nt;
-		if(nq > b.bin_quads_cap || nt > b.bin_tris_cap)
-			atomicOr(&b.ctrl[kCtrlOverflow], 1u);
+		b.ctrl[kCtrlFixedHigh] = nhigh;
+		// the size the host grows the lists to after an overflow (promoted bins add theirs)
+		b.ctrl[kCtrlListCursor] = (uint32_t)min(16ull * total[4], 0xffffffffull);
+		const uint32_t ovf = (nq > b.bin_quads_cap || nt > b.bin_tris_cap ? kOvfBinLists : 0u) |
+							 (fits ? 0u : kOvfLists);
+		if(ovf)
+			atomicOr(&b.ctrl[kCtrlOverflow], ovf);
 		info->bin_level_counts[LUCID_BIN_LEVEL_EMPTY] = (int32_t)((uint32_t)NB - nlow - nhigh);
 		info->bin_level_counts[LUCID_BIN_LEVEL_LOW] = (int32_t)nlow;
 		info->bin_level_counts[LUCID_BIN_LEVEL_HIGH] = (int32_t)nhigh;
@@ -308,15 +293,68 @@ __device__ __forceinline__ void bin_categorize_kernel_body(const FrameConst &c, 
 	}
 }
 
-__global__ __launch_bounds__(1024) void bin_categorize_kernel(FrameConst c, FrameBufs b) {
-	bin_categorize_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
+// Per bin: totals over work-groups and each work-group's exclusive offset inside the bin.
+// Exclusive scan of the per-work-group bin histograms down each (kind, bin) column, and the
+// column totals (the bin counts). A work-group takes 16 columns; its 16 row-parts each sum
+// a run of rows with independent loads, an LDS scan joins the parts, then each part writes
+// its exclusive prefixes. The last work-group to store its bin counts categorises the bins.
+__device__ __forceinline__ void bin_wg_scan_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
+	const int NB = c.bin_count, nw = c.num_bin_wgs;
+	const int col_l = threadIdx.x % kScanCols, part = threadIdx.x / kScanCols;
+	const int col = wg.id * kScanCols + col_l; // 0 .. 2 NB: quads then tris
+	const int rows = (nw + kScanParts - 1) / kScanParts; // <= 16: num_bin_wgs <= 256
+	const int w0 = part * rows, w1 = min(nw, w0 + rows);
+	__shared__ uint32_t s_part[kScanParts][kScanCols];
+	// all loads first (independent), then the stores: a part spans at most kMaxRows rows
+	constexpr int kMaxRows = 16;
+	uint32_t v[kMaxRows], sum = 0;
+	const bool live = col < 2 * NB;
+#pragma unroll
+	for(int j = 0; j < kMaxRows; j++)
+		v[j] = live && w0 + j < w1 ? b.wg_hist[(size_t)(w0 + j) * 2 * NB + col] : 0u;
+#pragma unroll
+	for(int j = 0; j < kMaxRows; j++)
+		sum += v[j];
+	s_part[part][col_l] = sum;
+	// the high bins' list lengths start at 0 (16 per bin: the grid has two threads for each)
+	const uint32_t id = wg.id * kScanThreads + threadIdx.x;
+	if(id < (uint32_t)NB * 16)
+		b.blk_count[id] = 0u;
+	__syncthreads();
+	if(part == 0) {
+		uint32_t run = 0;
+		for(int p = 0; p < kScanParts; p++) {
+			uint32_t v = s_part[p][col_l];
+			s_part[p][col_l] = run;
+			run += v;
+		}
+		if(live) {
+			const int k = col / NB, bin = col - k * NB;
+			uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
+			agent_store(&counts[(k == 0 ? LUCID_COUNTS_QUAD_COUNTS : LUCID_COUNTS_TRI_COUNTS) * NB + bin], run);
+		}
+	}
+	const bool last = last_work_group(&b.ctrl[kCtrlScanDone], 1u, wg.count);
+	uint32_t run = s_part[part][col_l];
+#pragma unroll
+	for(int j = 0; j < kMaxRows; j++) {
+		if(live && w0 + j < w1)
+			b.wg_hist[(size_t)(w0 + j) * 2 * NB + col] = run;
+		run += v[j];
+	}
+	if(last)
+		categorize_bins(c, b);
 }
-__global__ __launch_bounds__(1024) void bin_categorize_kernel_batch(const FrameDesc *__restrict__ frames,
+
+__global__ __launch_bounds__(kScanThreads) void bin_wg_scan_kernel(FrameConst c, FrameBufs b) {
+	bin_wg_scan_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
+}
+__global__ __launch_bounds__(kScanThreads) void bin_wg_scan_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
 	const uint32_t f = batch_frame(sb, blockIdx.x);
 	const FrameDesc &d = sb.frames[f];
-	bin_categorize_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
+	bin_wg_scan_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
 }
 
 // bin_dispatcher.glsl: replay the work-group's slice into its reserved ranges.
@@ -387,9 +425,7 @@ hipError_t launch_binning_batch(const BatchPlan &p, hipStream_t stream) {
 	hipLaunchKernelGGL(bin_count_kernel_batch, dim3(p.total[kBsBinCount]), dim3(kBinThreads),
 					   p.bin_lds, stream, p.frames, p.stage_pre(kBsBinCount), p.num_frames);
 	hipLaunchKernelGGL(bin_wg_scan_kernel_batch, dim3(p.total[kBsBinScan]),
-					   dim3(kScanCols * kScanParts), 0, stream, p.frames, p.stage_pre(kBsBinScan), p.num_frames);
-	hipLaunchKernelGGL(bin_categorize_kernel_batch, dim3(p.total[kBsBinCategorize]), dim3(1024), 0,
-					   stream, p.frames, p.stage_pre(kBsBinCategorize), p.num_frames);
+					   dim3(kScanThreads), 0, stream, p.frames, p.stage_pre(kBsBinScan), p.num_frames);
 	hipLaunchKernelGGL(bin_dispatch_kernel_batch, dim3(p.total[kBsBinDispatch]), dim3(kBinThreads),
 					   p.bin_lds, stream, p.frames, p.stage_pre(kBsBinDispatch), p.num_frames);
 	return hipGetLastError();
@@ -399,8 +435,7 @@ hipError_t launch_binning(const FrameConst &c, const FrameBufs &b, hipStream_t s
 	size_t lds = (size_t)2 * c.bin_count * sizeof(uint32_t);
 	hipLaunchKernelGGL(bin_count_kernel, dim3(c.num_bin_wgs), dim3(kBinThreads), lds, stream, c, b);
 	hipLaunchKernelGGL(bin_wg_scan_kernel, dim3((2 * c.bin_count + kScanCols - 1) / kScanCols),
-					   dim3(kScanCols * kScanParts), 0, stream, c, b);
-	hipLaunchKernelGGL(bin_categorize_kernel, dim3(1), dim3(1024), 0, stream, c, b);
+					   dim3(kScanThreads), 0, stream, c, b);
 	hipLaunchKernelGGL(bin_dispatch_kernel, dim3(c.num_bin_wgs), dim3(kBinThreads), lds, stream, c,
 					   b);
 	return hipGetLastError();

@@ -47,6 +47,8 @@ enum CtrlWord : int {
 	kCtrlWords = 16,
 	// device-only words (not copied to the host) up to kStatStripeBase:
 	kCtrlBigSorts = 16, // blocks queued in big_queue for the long-list sort pass
+	kCtrlScanDone = 17, // work-groups of bin_wg_scan that have stored their bin counts
+	kCtrlFixedHigh = 18, // high bins before row generation adds the promoted ones
 };
 
 // Frame statistics summed per block (fragments, list entries) go to kStatStripes counters
@@ -135,7 +137,8 @@ constexpr uint32_t kSlotWhole = 1u << 10;    // list too long: every pixel takes
 constexpr uint32_t kSlotPartShift = 12;      // log2 of the waves sharing a pre-sorted block
 constexpr int kRegSortCap = 256;  // lists sorted in registers by the raster wave itself
 constexpr int kBigSortCap = 8192; // lists sorted in LDS by high_finalize_kernel
-constexpr int kRowgenSplit = 8;   // work-groups per high bin in rowgen_high
+constexpr int kRowgenThreads = 256;       // work-group of the high bins' (and a batch's) row generation
+constexpr int kRowgenSplitThreads = 2048; // threads that share a high bin's row generation
 
 enum ColorMode : int { kColorNone = 0, kColorRGBA8 = 1, kColorF32 = 2 };
 
@@ -230,6 +233,9 @@ struct FrameBufs {
 	uint8_t *image;
 	float *image_f;
 	uint32_t *frag_counts;
+	// pinned host memory (kCtrlWords) that the frame's last kernel copies the control words to;
+	// null: the host copies them itself
+	uint32_t *host_status;
 };
 
 // ------------------------------------------------------------------ batched launches
@@ -269,10 +275,8 @@ enum BatchStage : int {
 	kBsSetup,
 	kBsBinCount,
 	kBsBinScan,
-	kBsBinCategorize,
 	kBsBinDispatch,
 	kBsRowgenLow,
-	kBsHighPrep,
 	kBsRowgenHigh,
 	kBsHighFinalize,
 	kBsHighFinalizeLong, // persistent: a few work-groups per frame over its queue
@@ -331,7 +335,6 @@ struct BatchPlan {
 	bool fp32;
 	int mode; // ShadeMode of the block kernels: textured if a frame is, flat if every frame is
 	int slice_words;
-	uint32_t *status; // device, kCtrlWords per frame: each frame's control words after it
 	__host__ const uint32_t *stage_pre(int s) const { return pre + (size_t)s * (num_frames + 1); }
 };
 
@@ -522,6 +525,29 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 }
 
 __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
+
+// Words that pass between the work-groups of one launch: loads and stores at the memory that all
+// XCDs share, past their own L2s.
+__device__ __forceinline__ uint32_t agent_load(const uint32_t *p) {
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void agent_store(uint32_t *p, uint32_t v) {
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Adds `mine` to `done` (a word that the frame cleared); true in every thread of the work-group
+// whose part completes the `total`. That work-group may agent_load what the others agent_store'd or changed by
+// atomics before: these are complete once each wave has waited for its memory operations, so no
+// cache has to be written back (a release fence of whole L2s, 512 waves of them, took 60 us).
+// Called by whole work-groups.
+__device__ __forceinline__ bool last_work_group(uint32_t *done, uint32_t mine, uint32_t total) {
+	__shared__ uint32_t s_last;
+	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+	__syncthreads();
+	if(threadIdx.x == 0)
+		s_last = __hip_atomic_fetch_add(done, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine == total;
+	__syncthreads();
+	return s_last != 0;
+}
 
 // Index of the k-th (0-based) set bit of m (k < popcount(m)).
 __device__ __forceinline__ int select_bit64(uint64_t m, uint32_t k) {

@@ -145,7 +145,8 @@ struct lucid_renderer {
 	std::vector<lucid_vec4> host_uv_rects;
 	bool uv_rects_null = true;
 
-	uint32_t *status = nullptr; // pinned copy of the control words of the last frame
+	uint32_t *status = nullptr; // pinned: the last frame's control words (its last kernel fills it)
+	uint32_t *status_dev = nullptr; // the same memory, as the GPU addresses it
 	hipEvent_t done = nullptr;
 	static constexpr int kStages = 6;
 	hipEvent_t stage_ev[kStages + 1] = {};
@@ -373,7 +374,9 @@ int lucid_create(const lucid_create_info *ci, lucid_renderer **out) {
 	chk(r->blk_lists.reserve(r->blk_lists_cap * 16));
 	r->sorted_cap = 1u << 22;
 	chk(r->sorted_pool.reserve(r->sorted_cap * 4));
-	chk(hipHostMalloc((void **)&r->status, kCtrlWords * 4, hipHostMallocDefault));
+	chk(hipHostMalloc((void **)&r->status, kCtrlWords * 4, hipHostMallocMapped | hipHostMallocCoherent));
+	if(rc == LUCID_OK)
+		chk(hipHostGetDevicePointer((void **)&r->status_dev, r->status, 0));
 	chk(hipEventCreateWithFlags(&r->done, hipEventDisableTiming));
 	r->timers = (ci->opts & LUCID_OPT_TIMERS) != 0;
 	if(r->timers)
@@ -628,6 +631,7 @@ int prepare_frame(lucid_renderer *r, const lucid_frame_inputs *in, const lucid_f
 	b.image = out ? out->image_rgba8 : nullptr;
 	b.image_f = out ? out->image_rgba32f : nullptr;
 	b.frag_counts = out ? out->frag_counts : nullptr;
+	b.host_status = r->status_dev;
 	nq_out = nq;
 	return LUCID_OK;
 }
@@ -774,9 +778,7 @@ int lucid_render_ex(lucid_renderer *r, const lucid_frame_inputs *in,
 		LUCID_CHECK(launch_raster_recording(c, b, g, stream, r->timers ? r->stage_ev + 3 : nullptr));
 	else
 		LUCID_CHECK(launch_raster(c, b, stream, r->timers ? r->stage_ev + 3 : nullptr));
-	LUCID_CHECK(hipMemcpyAsync(r->status, r->ctrl.ptr, kCtrlWords * 4, hipMemcpyDeviceToHost,
-							   stream));
-	LUCID_CHECK(hipEventRecord(r->done, stream));
+	LUCID_CHECK(hipEventRecord(r->done, stream)); // (the last kernel fills r->status)
 	r->frame_pending = true;
 	r->last_num_quads = nq;
 	r->last_stream = stream;
@@ -1034,8 +1036,9 @@ struct lucid_batch {
 	std::vector<lucid_renderer *> rs;
 	std::vector<FrameDesc> frames;   // the frames of the recorded launch (host copy)
 	std::vector<uint32_t> pre;       // kBsCount x (n + 1) work-group prefixes
-	DevBuf frames_dev, pre_dev, status_dev;
-	uint32_t *status = nullptr;      // pinned: kCtrlWords per frame after the last launch
+	DevBuf frames_dev, pre_dev;
+	uint32_t *status = nullptr;      // pinned: kCtrlWords per frame, filled by each frame's last kernel
+	uint32_t *status_dev = nullptr;  // the same memory, as the GPU addresses it
 	BatchPlan plan = {};
 	hipEvent_t done = nullptr;
 	hipStream_t capture_stream = nullptr;
@@ -1072,11 +1075,9 @@ void stage_wgs(const FrameConst &c, uint32_t w[kBsCount]) {
 	w[kBsSetup] = c.num_quads > 0 ? ((uint32_t)c.num_quads + kSetupThreads - 1) / kSetupThreads : 0;
 	w[kBsBinCount] = (uint32_t)c.num_bin_wgs;
 	w[kBsBinScan] = (2 * nb + kScanColsHost - 1) / kScanColsHost;
-	w[kBsBinCategorize] = 1;
 	w[kBsBinDispatch] = (uint32_t)c.num_bin_wgs;
 	w[kBsRowgenLow] = nb;
-	w[kBsHighPrep] = 1;
-	w[kBsRowgenHigh] = nb * kRowgenSplit;
+	w[kBsRowgenHigh] = nb * (kRowgenSplitThreads / kRowgenThreads);
 	w[kBsHighFinalize] = nb * 16;
 	w[kBsHighFinalizeLong] = kBatchLongSortWgs;
 	w[kBsBlockRaster] = nb * 16;
@@ -1084,23 +1085,19 @@ void stage_wgs(const FrameConst &c, uint32_t w[kBsCount]) {
 	w[kBsFallback] = kBatchFallbackWgs;
 }
 
-// Records the batch's launches into one graph: one launch per stage for all frames, then
-// the frames' control words to pinned host memory.
+// Records the batch's launches into one graph: one launch per stage for all frames.
 int capture_batch(lucid_batch *bt) {
 	if(bt->exec)
 		(void)hipGraphExecDestroy(bt->exec), bt->exec = nullptr;
 	if(bt->graph)
 		(void)hipGraphDestroy(bt->graph), bt->graph = nullptr;
 	hipStream_t s = bt->capture_stream;
-	const size_t n = bt->rs.size();
 	LUCID_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
 	hipError_t err = launch_setup_batch(bt->plan, s);
 	if(err == hipSuccess)
 		err = launch_binning_batch(bt->plan, s);
 	if(err == hipSuccess)
 		err = launch_raster_batch(bt->plan, s);
-	if(err == hipSuccess)
-		err = hipMemcpyAsync(bt->status, bt->plan.status, n * kCtrlWords * 4, hipMemcpyDeviceToHost, s);
 	hipGraph_t g = nullptr;
 	hipError_t end = hipStreamEndCapture(s, &g);
 	if(err != hipSuccess || end != hipSuccess) {
@@ -1134,12 +1131,12 @@ int lucid_batch_create(lucid_renderer *const *renderers, int n, lucid_batch **ou
 	if(hipSetDevice(bt->device) != hipSuccess ||
 	   hipStreamCreateWithFlags(&bt->capture_stream, hipStreamNonBlocking) != hipSuccess ||
 	   hipEventCreateWithFlags(&bt->done, hipEventDisableTiming) != hipSuccess ||
-	   hipHostMalloc((void **)&bt->status, (size_t)n * kCtrlWords * 4, hipHostMallocDefault) != hipSuccess)
+	   hipHostMalloc((void **)&bt->status, (size_t)n * kCtrlWords * 4,
+					 hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+	   hipHostGetDevicePointer((void **)&bt->status_dev, bt->status, 0) != hipSuccess)
 		rc = LUCID_ERR_HIP;
 	if(rc == LUCID_OK) {
-		rc = hip_status(bt->status_dev.reserve((size_t)n * kCtrlWords * 4));
-		if(rc == LUCID_OK)
-			rc = hip_status(bt->pre_dev.reserve((size_t)kBsCount * (n + 1) * 4));
+		rc = hip_status(bt->pre_dev.reserve((size_t)kBsCount * (n + 1) * 4));
 		if(rc == LUCID_OK)
 			rc = hip_status(bt->frames_dev.reserve((size_t)n * sizeof(FrameDesc)));
 	}
@@ -1189,6 +1186,7 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 		// every frame runs the block kernels of the first renderer's slice width (a tuning
 		// knob: results do not depend on it)
 		frames[i].c.slice_words = bt->rs[0]->tuning.slice_words;
+		frames[i].b.host_status = bt->status_dev + i * kCtrlWords;
 		tex = tex || frames[i].c.has_textures;
 		flat = flat && frame_shade_mode(frames[i].c) >= kShadeFlat; // flat records, either window
 		r->last_num_quads = nq;
@@ -1218,7 +1216,6 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 					: flat ? (bt->rs[0]->tuning.window == 1 ? kShadeFlatNarrow : kShadeFlat)
 						   : kShadeGeneral;
 	plan.slice_words = bt->rs[0]->tuning.slice_words;
-	plan.status = bt->status_dev.as<uint32_t>();
 	// the launches read the frames' constants and buffers from device memory, so a frame
 	// whose inputs change only needs them uploaded; the graph is recorded again only when a
 	// grid, the LDS size or a kernel choice changes

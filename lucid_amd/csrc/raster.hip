@@ -26,7 +26,6 @@
 
 namespace lucid {
 
-constexpr int kRowgenThreads = 256;
 constexpr int kSortThreads = 256;
 constexpr int kFallbackThreads = 256;
 constexpr int kWindow = 4;
@@ -955,11 +954,34 @@ template <int THREADS> union RowgenLds {
 	uint32_t sorted[kRowgenRound];
 	RowgenWave wave[THREADS / 64];
 };
-// rowgen_low's work-group: a low bin's triangles are few, so a single frame's bins take twice
-// the waves (each then scans one or two chunks); a batch has bins enough to fill the chip and
-// keeps to the smaller groups. 1280 x 720 lit mesh frame 26.2 -> 23.6 us with 512 threads, the
-// 32-frame batch 240 us with 256 and 271 us with 512.
-constexpr int kRowgenLowThreads = 512, kRowgenLowThreadsBatch = 256;
+struct RowgenCounts {
+	uint32_t cnt[8], off[8], nlive; // the counting sort
+	uint32_t blk_n[16];             // list lengths of a low bin
+};
+// The LDS that low and high bins share (in the launch that takes both, too). Three variables, not
+// one struct: accesses with indices known only at run time are then known not to overlap, and the
+// compiler keeps them in flight together (one struct: rowgen_high 5 - 10 % slower).
+template <int THREADS> __device__ __forceinline__ RowgenLds<THREADS> &rowgen_lds() {
+	__shared__ RowgenLds<THREADS> s;
+	return s;
+}
+__device__ __forceinline__ RowgenCounts &rowgen_counts() {
+	__shared__ RowgenCounts s;
+	return s;
+}
+__device__ __forceinline__ float *rowgen_inverses() { // [n] = 1 / n, n <= 64
+	__shared__ float s[65];
+	return s;
+}
+__device__ __forceinline__ void fill_inverses() {
+	if(threadIdx.x <= 64)
+		rowgen_inverses()[threadIdx.x] = 1.0f / (float)(threadIdx.x > 0 ? threadIdx.x : 1);
+}
+// Work-group size: a single frame's low bins take twice the waves, as a low bin's triangles are
+// few (each wave then scans one or two chunks); high bins, and a batch, which has bins enough to
+// fill the chip, keep to the smaller groups. Low bins: 1280 x 720 lit mesh frame 26.2 -> 23.6 us
+// with 512 threads, the 32-frame batch 240 us with 256 and 271 us with 512.
+constexpr int kRowgenLowThreads = 512;
 
 // What a lane scans: a triangle (~0: none), its scan parameters and depth plane.
 struct ScanTri {
@@ -1048,20 +1070,93 @@ __device__ __forceinline__ void rowgen_wave(const FrameBufs &b, RowgenWave &w, c
 	wave_sync_lds(); // the staging is used again
 }
 
-__device__ __forceinline__ void fill_inverses(float *s_inv) { // s_inv[n] = 1 / n, n <= 64
-	if(threadIdx.x <= 64)
-		s_inv[threadIdx.x] = 1.0f / (float)(threadIdx.x > 0 ? threadIdx.x : 1);
+// ------------------------------------------------------------------ high bins
+
+// Block lists of a high bin with the 4-row rule (raster_high.glsl:54-90): a triangle's scan
+// starts at the first row of its 4-row group (the start row fixes the scanline arithmetic).
+// Work-group `split` of `splits` that share the bin; block k's list starts at lst + k * nlevel.
+// A wave's row loop runs as long as its tallest triangle, so each work-group first sorts its
+// triangles by height (a counting sort over the 8 heights in 4-row groups, up to kRowgenRound
+// list positions at a time).
+template <int THREADS>
+__device__ __forceinline__ void rowgen_high_bin(const FrameBufs &b, int bin,
+												const BinInfo &bi, uint32_t lst, uint32_t split,
+												uint32_t splits) {
+	RowgenLds<THREADS> &s = rowgen_lds<THREADS>();
+	RowgenCounts &sh = rowgen_counts();
+	const int lane = lane_id(), wave = threadIdx.x >> 6;
+	const uint32_t first = lst + (uint32_t)(lane & 15) * bi.nlevel;
+	uint32_t *blk_n = b.blk_count + (size_t)bin * 16;
+	const uint32_t stride = THREADS * splits;
+	constexpr int kHeights = kBinSize / 4, kChunks = kRowgenRound / THREADS;
+	// first row group and height in row groups of triangle t in this bin
+	auto groups = [&](uint32_t yr, int &g0, int &g1) {
+		g0 = min(max((int)(yr & 0xffffu) - bi.bin_y, 0), kBinMask) >> 2;
+		g1 = min(max((int)(yr >> 16) - bi.bin_y, 0), kBinMask) >> 2;
+	};
+	// the work-group's list positions: chunks split, split + splits, ... of THREADS entries;
+	// culled triangles (every second one of a soup quad) are dropped
+	const uint32_t round_len = stride * kChunks;
+	for(uint32_t base = split * THREADS; base < bi.nlevel; base += round_len) {
+		if(threadIdx.x < kHeights)
+			sh.cnt[threadIdx.x] = 0;
+		__syncthreads();
+		uint32_t tk[kChunks];
+		int hk[kChunks];
+#pragma unroll
+		for(int k = 0; k < kChunks; k++) {
+			const uint32_t i = base + k * stride + threadIdx.x;
+			const uint32_t t = i < bi.nlevel ? bin_tri_at(b, i, bi.qc, bi.qo, bi.to) : 0xffffffffu;
+			int h = -1;
+			if(t != 0xffffffffu) {
+				int g0, g1;
+				groups(b.tri_scan[2 * (size_t)tri_rec(b, t)].w, g0, g1);
+				h = g1 > g0 ? g1 - g0 : 0;
+				atomicAdd(&sh.cnt[h], 1u);
+			}
+			tk[k] = t, hk[k] = h;
+		}
+		__syncthreads();
+		if(threadIdx.x == 0) {
+			uint32_t run = 0;
+			for(int h = 0; h < kHeights; h++)
+				sh.off[h] = run, run += sh.cnt[h];
+			sh.nlive = run;
+		}
+		__syncthreads();
+#pragma unroll
+		for(int k = 0; k < kChunks; k++)
+			if(hk[k] >= 0)
+				s.sorted[atomicAdd(&sh.off[hk[k]], 1u)] = tk[k];
+		__syncthreads();
+		const uint32_t n = sh.nlive;
+#pragma unroll
+		for(int k = 0; k < kChunks; k++)
+			tk[k] = k * THREADS + threadIdx.x < n ? s.sorted[k * THREADS + threadIdx.x] : 0xffffffffu;
+		__syncthreads(); // the staging takes the sorted list's place
+		for(int k = 0; k * THREADS + wave * 64 < (int)n; k++) {
+			const ScanTri tr = load_scan_tri(b, k == 0 ? tk[0] : k == 1 ? tk[1] : k == 2 ? tk[2 % kChunks] : tk[3 % kChunks]);
+			int g0 = 0, g1 = -1;
+			if(tr.t != 0xffffffffu)
+				groups(tr.s0.w, g0, g1);
+			rowgen_wave(b, s.wave[wave], rowgen_inverses(), bi.bin_x, bi.bin_y, tr, g0, g1, first, ~0u,
+						[&](uint32_t num) { return atomicAdd(&blk_n[lane], num); });
+		}
+		if(base + round_len < bi.nlevel)
+			__syncthreads(); // the next round reuses the sorted list
+	}
 }
 
-// ------------------------------------------------------------------ rowgen_low
+// ------------------------------------------------------------------ low bins
 
+// Block lists of a low bin, 256 positions each, with the 8-row rule (raster_low.glsl:39-79): the
+// scan starts at the first row of a band. A bin with a longer list is promoted: it joins the
+// high list, takes list space of its own and is generated again as a high bin.
 template <int THREADS>
-__device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	const int bin = wg.id;
-	const uint32_t overflow = b.ctrl[kCtrlOverflow]; // loaded beside the bin's counts
+__device__ __forceinline__ void rowgen_low_bin(const FrameConst &c, const FrameBufs &b, int bin) {
+	RowgenLds<THREADS> &s = rowgen_lds<THREADS>();
+	RowgenCounts &sh = rowgen_counts();
 	const BinInfo bi = load_bin(c, b, bin);
-	if(overflow & kOvfBinLists)
-		return;
 	uint32_t *flags = b.blk_flags + (size_t)bin * 16;
 	if(bi.nlevel == 0) {
 		if(threadIdx.x < 16)
@@ -1069,22 +1164,18 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 		return;
 	}
 	if(bi.nlevel >= (uint32_t)kLowLevelLimit)
-		return; // rowgen_high writes this bin's slots
+		return; // a high bin
 
 	constexpr int kChunks = kRowgenRound / THREADS; // list positions per thread
-	__shared__ RowgenLds<THREADS> s;
-	__shared__ float s_inv[65];
-	__shared__ uint32_t s_blk_n[16];
 	// The bin's live triangles (its list has fewer than kLowLevelLimit entries: one position
 	// per thread and chunk) are counting-sorted by their number of 8-row bands, so that the
 	// waves' row loops run about as long as each of their triangles needs.
 	static_assert(kLowLevelLimit <= kRowgenRound, "a low bin's list in one round");
-	__shared__ uint32_t s_nb[4], s_nb_off[4], s_nlive;
-	fill_inverses(s_inv);
+	fill_inverses();
 	if(threadIdx.x < 16)
-		s_blk_n[threadIdx.x] = 0;
+		sh.blk_n[threadIdx.x] = 0;
 	if(threadIdx.x < 4)
-		s_nb[threadIdx.x] = 0;
+		sh.cnt[threadIdx.x] = 0;
 	__syncthreads();
 	uint32_t tk[kChunks];
 	int hk[kChunks];
@@ -1102,7 +1193,7 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 			int lo_by, hi_by;
 			bands(b.tri_scan[2 * (size_t)tri_rec(b, t)].w, lo_by, hi_by);
 			h = hi_by > lo_by ? hi_by - lo_by : 0;
-			atomicAdd(&s_nb[h], 1u);
+			atomicAdd(&sh.cnt[h], 1u);
 		}
 		tk[k] = t, hk[k] = h;
 	}
@@ -1110,235 +1201,122 @@ __device__ __forceinline__ void rowgen_low_kernel_body(const FrameConst &c, cons
 	if(threadIdx.x == 0) {
 		uint32_t run = 0;
 		for(int h = 0; h < 4; h++)
-			s_nb_off[h] = run, run += s_nb[h];
-		s_nlive = run;
+			sh.off[h] = run, run += sh.cnt[h];
+		sh.nlive = run;
 	}
 	__syncthreads();
 #pragma unroll
 	for(int k = 0; k < kChunks; k++)
 		if(hk[k] >= 0)
-			s.sorted[atomicAdd(&s_nb_off[hk[k]], 1u)] = tk[k];
+			s.sorted[atomicAdd(&sh.off[hk[k]], 1u)] = tk[k];
 	__syncthreads();
-	const uint32_t nlive = s_nlive;
+	const uint32_t nlive = sh.nlive;
 	const int lane = lane_id(), wave = threadIdx.x >> 6;
 #pragma unroll
 	for(int k = 0; k < kChunks; k++)
 		tk[k] = k * THREADS + threadIdx.x < nlive ? s.sorted[k * THREADS + threadIdx.x] : 0xffffffffu;
 	__syncthreads(); // the staging takes the sorted list's place
 	const uint32_t first = ((uint32_t)bin * 16 + (uint32_t)(lane & 15)) * kRegSortCap;
-	// 8-row rule (raster_low.glsl:39-79): the scan starts at the first row of a band
 	for(int k = 0; k * THREADS + wave * 64 < (int)nlive; k++) {
 		const ScanTri tr = load_scan_tri(b, k == 0 ? tk[0] : k == 1 ? tk[1] : k == 2 ? tk[2 % kChunks] : tk[3 % kChunks]);
 		int lo_by = 0, hi_by = -1;
 		if(tr.t != 0xffffffffu)
 			bands(tr.s0.w, lo_by, hi_by);
-		rowgen_wave(b, s.wave[wave], s_inv, bi.bin_x, bi.bin_y, tr, lo_by * 2, hi_by * 2 + 1, first,
-					(uint32_t)kRegSortCap, [&](uint32_t n) { return atomicAdd(&s_blk_n[lane], n); });
+		rowgen_wave(b, s.wave[wave], rowgen_inverses(), bi.bin_x, bi.bin_y, tr, lo_by * 2, hi_by * 2 + 1, first,
+					(uint32_t)kRegSortCap, [&](uint32_t n) { return atomicAdd(&sh.blk_n[lane], n); });
 	}
 	__syncthreads();
 	bool promote = false;
 	for(int k = 0; k < 16; k++)
-		promote |= s_blk_n[k] > (uint32_t)kMaxBlockTris;
-	if(promote) {
-		if(threadIdx.x == 0) {
-			lucid_info *info = (lucid_info *)b.info;
-			uint32_t id = atomicAdd((uint32_t *)&info->bin_level_counts[LUCID_BIN_LEVEL_HIGH], 1u);
-			b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + id] = (uint32_t)bin;
+		promote |= sh.blk_n[k] > (uint32_t)kMaxBlockTris;
+	if(!promote) {
+		if(threadIdx.x < 16) {
+			b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(first, sh.blk_n[threadIdx.x]);
+			flags[threadIdx.x] = LUCID_BIN_LEVEL_LOW;
 		}
-		if(threadIdx.x < 16)
-			flags[threadIdx.x] = kSlotPromoted;
 		return;
 	}
-	if(threadIdx.x < 16) {
-		b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(first, s_blk_n[threadIdx.x]);
-		flags[threadIdx.x] = LUCID_BIN_LEVEL_LOW;
+	__syncthreads(); // blk_n is read
+	if(threadIdx.x == 0) {
+		lucid_info *info = (lucid_info *)b.info;
+		uint32_t id = atomicAdd((uint32_t *)&info->bin_level_counts[LUCID_BIN_LEVEL_HIGH], 1u);
+		b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + id] = (uint32_t)bin;
+		const uint32_t off = atomicAdd(&b.ctrl[kCtrlListCursor], 16u * bi.nlevel);
+		const uint64_t lst = (uint64_t)c.bin_count * 16 * kRegSortCap + off;
+		const bool ok = lst + 16ull * bi.nlevel <= b.blk_lists_cap;
+		if(!ok)
+			atomicOr(&b.ctrl[kCtrlOverflow], kOvfLists);
+		sh.blk_n[0] = (uint32_t)lst, sh.blk_n[1] = ok ? 1u : 0u;
 	}
-}
-
-__global__ __launch_bounds__(kRowgenLowThreads) void rowgen_low_kernel(FrameConst c, FrameBufs b) {
-	rowgen_low_kernel_body<kRowgenLowThreads>(c, b, WgPos{blockIdx.x, gridDim.x});
-}
-__global__ __launch_bounds__(kRowgenLowThreadsBatch) void rowgen_low_kernel_batch(const FrameDesc *__restrict__ frames,
-		const uint32_t *__restrict__ pre, uint32_t num_frames) {
-	const StageBatch sb{frames, pre, num_frames};
-	const uint32_t f = batch_frame(sb, blockIdx.x);
-	const FrameDesc &d = sb.frames[f];
-	rowgen_low_kernel_body<kRowgenLowThreadsBatch>(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
-}
-
-// ------------------------------------------------------------------ high bins
-
-// Allocates the list space of every high bin (promotions included) with an exclusive scan
-// over the high list, and clears the counters rowgen_high accumulates into.
-__device__ __forceinline__ void high_prep_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
-		return;
-	const lucid_info *info = (const lucid_info *)b.info;
-	const uint32_t nh = (uint32_t)info->bin_level_counts[LUCID_BIN_LEVEL_HIGH];
-	const uint32_t *high = b.info + LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count;
-	__shared__ uint32_t s_wave[16];
-	__shared__ uint32_t s_carry;
-	__shared__ uint32_t s_ex[1024], s_n[1024]; // per bin of the chunk: earlier tris, its tris
-	__shared__ uint32_t s_bad[1024 / 32];      // per bin of the chunk: allocation failed
-	if(threadIdx.x == 0)
-		s_carry = 0;
 	__syncthreads();
-	const uint64_t list0 = (uint64_t)c.bin_count * 16 * kRegSortCap;
-	const int wave = threadIdx.x >> 6;
-	for(uint32_t base = 0; base < nh; base += 1024) {
-		uint32_t i = base + threadIdx.x;
-		int bin = i < nh ? (int)high[i] : 0;
-		uint32_t n = i < nh ? load_bin(c, b, bin).nlevel : 0u;
-		uint32_t inc = wave_inclusive_add(n);
-		if(lane_id() == 63)
-			s_wave[wave] = inc;
-		__syncthreads();
-		if(threadIdx.x == 0) {
-			uint32_t run = s_carry;
-			for(int w = 0; w < 16; w++) {
-				uint32_t v = s_wave[w];
-				s_wave[w] = run;
-				run += v;
-			}
-			s_carry = run;
-		}
-		__syncthreads();
-		bool bad = false;
-		if(i < nh) {
-			uint64_t ex = (uint64_t)s_wave[wave] + inc - n; // tris of earlier high bins
-			uint64_t lst = list0 + 16 * ex;
-			bool ok = lst + 16ull * n <= b.blk_lists_cap;
-			if(!ok)
-				atomicOr(&b.ctrl[kCtrlOverflow], kOvfLists);
-			bad = !ok; // (ex then need not fit 32 bits: the bin's slots are not used)
-			if(i == nh - 1) // the size the host grows the lists to after an overflow
-				b.ctrl[kCtrlListCursor] = (uint32_t)min(16ull * (ex + n), 0xffffffffull);
-			s_ex[threadIdx.x] = (uint32_t)ex;
-			s_n[threadIdx.x] = n;
-		}
-		if((threadIdx.x & 31) == 0)
-			s_bad[threadIdx.x >> 5] = 0;
-		__syncthreads();
-		if(bad)
-			atomicOr(&s_bad[threadIdx.x >> 5], 1u << (threadIdx.x & 31));
-		__syncthreads();
-		// the chunk's block slots, 16 consecutive ones per bin, one per thread and step
-		const uint32_t nb = min(nh - base, 1024u);
-		for(uint32_t p = threadIdx.x; p < nb * 16; p += 1024) {
-			const uint32_t k = p >> 4, blk = p & 15;
-			const uint32_t bin = high[base + k], n = s_n[k];
-			const uint64_t ex = s_ex[k], lst = list0 + 16 * ex;
-			b.blk_slot[(size_t)bin * 16 + blk] = make_uint2((uint32_t)(lst + (uint64_t)blk * n), 0u);
-			b.blk_count[(size_t)bin * 16 + blk] = 0;
-			b.blk_flags[(size_t)bin * 16 + blk] = (s_bad[k >> 5] >> (k & 31)) & 1u ? kSlotPromoted : 0u;
-		}
-		__syncthreads();
+	const uint32_t lst = sh.blk_n[0];
+	const bool ok = sh.blk_n[1] != 0u;
+	if(threadIdx.x < 16) {
+		b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(lst + threadIdx.x * bi.nlevel, 0u);
+		flags[threadIdx.x] = ok ? 0u : kSlotPromoted; // (no space: the frame reports an overflow)
 	}
+	if(ok)
+		rowgen_high_bin<THREADS>(b, bin, bi, lst, 0u, 1u);
 }
 
-__global__ __launch_bounds__(1024) void high_prep_kernel(FrameConst c, FrameBufs b) {
-	high_prep_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
+// Work-group id of the kRowgenSplitThreads / THREADS that share each high bin.
+template <int THREADS>
+__device__ __forceinline__ void rowgen_high_body(const FrameConst &c, const FrameBufs &b, uint32_t id) {
+	constexpr uint32_t kSplits = kRowgenSplitThreads / THREADS;
+	const uint32_t slot = id / kSplits, split = id % kSplits;
+	const uint32_t overflow = b.ctrl[kCtrlOverflow];
+	if((overflow & kOvfBinLists) || slot >= b.ctrl[kCtrlFixedHigh])
+		return;
+	const int bin = (int)b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + slot];
+	const BinInfo bi = load_bin(c, b, bin);
+	const uint32_t lst = b.blk_slot[(size_t)bin * 16].x;
+	// (a low bin that is promoted meanwhile may set kOvfLists: such a frame is rendered again)
+	const bool fits = !(overflow & kOvfLists);
+	if(split == 0 && threadIdx.x < 16) {
+		if(threadIdx.x > 0)
+			b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(lst + threadIdx.x * bi.nlevel, 0u);
+		b.blk_flags[(size_t)bin * 16 + threadIdx.x] = fits ? 0u : kSlotPromoted;
+	}
+	if(!fits)
+		return;
+	fill_inverses();
+	rowgen_high_bin<THREADS>(b, bin, bi, lst, split, kSplits);
 }
-__global__ __launch_bounds__(1024) void high_prep_kernel_batch(const FrameDesc *__restrict__ frames,
+template <int THREADS>
+__device__ __forceinline__ void rowgen_low_body(const FrameConst &c, const FrameBufs &b, uint32_t id) {
+	const uint32_t overflow = b.ctrl[kCtrlOverflow];
+	if(!(overflow & kOvfBinLists))
+		rowgen_low_bin<THREADS>(c, b, (int)id);
+}
+
+// Low (and empty) bins and high bins apart, and in one launch: the high bins' work-groups first
+// (the longest), then the low ones', which fill the chip as the high ones run out.
+__global__ __launch_bounds__(kRowgenLowThreads) void rowgen_low_kernel(FrameConst c, FrameBufs b) {
+	rowgen_low_body<kRowgenLowThreads>(c, b, blockIdx.x);
+}
+__global__ __launch_bounds__(kRowgenThreads) void rowgen_high_kernel(FrameConst c, FrameBufs b) {
+	rowgen_high_body<kRowgenThreads>(c, b, blockIdx.x);
+}
+__global__ __launch_bounds__(kRowgenLowThreads) void rowgen_fused_kernel(FrameConst c, FrameBufs b) {
+	const uint32_t high = (uint32_t)c.bin_count * (kRowgenSplitThreads / kRowgenLowThreads);
+	if(blockIdx.x < high)
+		rowgen_high_body<kRowgenLowThreads>(c, b, blockIdx.x);
+	else
+		rowgen_low_body<kRowgenLowThreads>(c, b, blockIdx.x - high);
+}
+__global__ __launch_bounds__(kRowgenThreads) void rowgen_low_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
 	const uint32_t f = batch_frame(sb, blockIdx.x);
 	const FrameDesc &d = sb.frames[f];
-	high_prep_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
-}
-
-// Block lists of a high bin with the 4-row rule (raster_high.glsl:54-90): a triangle's scan
-// starts at the first row of its 4-row group (the start row fixes the scanline arithmetic).
-// kRowgenSplit work-groups share a bin. A wave's row loop runs as long as its tallest
-// triangle, so each work-group first sorts its triangles by height (a counting sort over the
-// 8 heights in 4-row groups, up to kRowgenRound list chunks at a time).
-__device__ __forceinline__ void rowgen_high_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfLists))
-		return;
-	const lucid_info *info = (const lucid_info *)b.info;
-	const uint32_t slot = wg.id / kRowgenSplit;
-	const int split = wg.id % kRowgenSplit;
-	if(slot >= (uint32_t)info->bin_level_counts[LUCID_BIN_LEVEL_HIGH])
-		return;
-	const uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
-	const int bin = (int)counts[LUCID_COUNTS_HIGH_BINS * c.bin_count + slot];
-	const BinInfo bi = load_bin(c, b, bin);
-	const int lane = lane_id(), wave = threadIdx.x >> 6;
-	const uint32_t first = b.blk_slot[(size_t)bin * 16 + (lane & 15)].x;
-	uint32_t *blk_n = b.blk_count + (size_t)bin * 16;
-	const uint32_t stride = kRowgenThreads * kRowgenSplit;
-	constexpr int kHeights = kBinSize / 4, kChunks = kRowgenRound / kRowgenThreads;
-	__shared__ RowgenLds<kRowgenThreads> s;
-	__shared__ float s_inv[65];
-	__shared__ uint32_t s_cnt[kHeights], s_off[kHeights], s_n;
-	fill_inverses(s_inv);
-	// first row group and height in row groups of triangle t in this bin
-	auto groups = [&](uint32_t yr, int &g0, int &g1) {
-		g0 = min(max((int)(yr & 0xffffu) - bi.bin_y, 0), kBinMask) >> 2;
-		g1 = min(max((int)(yr >> 16) - bi.bin_y, 0), kBinMask) >> 2;
-	};
-	// the work-group's list positions: chunks split, split + kRowgenSplit, ... of
-	// kRowgenThreads entries; culled triangles (every second one of a soup quad) are dropped
-	const uint32_t round_len = stride * kChunks;
-	for(uint32_t base = split * kRowgenThreads; base < bi.nlevel; base += round_len) {
-		if(threadIdx.x < kHeights)
-			s_cnt[threadIdx.x] = 0;
-		__syncthreads();
-		uint32_t tk[kChunks];
-		int hk[kChunks];
-#pragma unroll
-		for(int k = 0; k < kChunks; k++) {
-			const uint32_t i = base + k * stride + threadIdx.x;
-			const uint32_t t = i < bi.nlevel ? bin_tri_at(b, i, bi.qc, bi.qo, bi.to) : 0xffffffffu;
-			int h = -1;
-			if(t != 0xffffffffu) {
-				int g0, g1;
-				groups(b.tri_scan[2 * (size_t)tri_rec(b, t)].w, g0, g1);
-				h = g1 > g0 ? g1 - g0 : 0;
-				atomicAdd(&s_cnt[h], 1u);
-			}
-			tk[k] = t, hk[k] = h;
-		}
-		__syncthreads();
-		if(threadIdx.x == 0) {
-			uint32_t run = 0;
-			for(int h = 0; h < kHeights; h++)
-				s_off[h] = run, run += s_cnt[h];
-			s_n = run;
-		}
-		__syncthreads();
-#pragma unroll
-		for(int k = 0; k < kChunks; k++)
-			if(hk[k] >= 0)
-				s.sorted[atomicAdd(&s_off[hk[k]], 1u)] = tk[k];
-		__syncthreads();
-		const uint32_t n = s_n;
-#pragma unroll
-		for(int k = 0; k < kChunks; k++)
-			tk[k] = k * kRowgenThreads + threadIdx.x < n ? s.sorted[k * kRowgenThreads + threadIdx.x] : 0xffffffffu;
-		__syncthreads(); // the staging takes the sorted list's place
-		for(int k = 0; k * kRowgenThreads + wave * 64 < (int)n; k++) {
-			const ScanTri tr = load_scan_tri(b, k == 0 ? tk[0] : k == 1 ? tk[1] : k == 2 ? tk[2] : tk[3]);
-			int g0 = 0, g1 = -1;
-			if(tr.t != 0xffffffffu)
-				groups(tr.s0.w, g0, g1);
-			rowgen_wave(b, s.wave[wave], s_inv, bi.bin_x, bi.bin_y, tr, g0, g1, first, ~0u,
-						[&](uint32_t num) { return atomicAdd(&blk_n[lane], num); });
-		}
-		if(base + round_len < bi.nlevel)
-			__syncthreads(); // the next round reuses the sorted list
-	}
-}
-
-__global__ __launch_bounds__(kRowgenThreads) void rowgen_high_kernel(FrameConst c, FrameBufs b) {
-	rowgen_high_kernel_body(c, b, WgPos{blockIdx.x, gridDim.x});
+	rowgen_low_body<kRowgenThreads>(d.c, d.b, blockIdx.x - sb.pre[f]);
 }
 __global__ __launch_bounds__(kRowgenThreads) void rowgen_high_kernel_batch(const FrameDesc *__restrict__ frames,
 		const uint32_t *__restrict__ pre, uint32_t num_frames) {
 	const StageBatch sb{frames, pre, num_frames};
 	const uint32_t f = batch_frame(sb, blockIdx.x);
 	const FrameDesc &d = sb.frames[f];
-	rowgen_high_kernel_body(d.c, d.b, WgPos{blockIdx.x - sb.pre[f], sb.pre[f + 1] - sb.pre[f]});
+	rowgen_high_body<kRowgenThreads>(d.c, d.b, blockIdx.x - sb.pre[f]);
 }
 
 // Entries (triangles of one block in depth order) are handed to the rasteriser in slices
@@ -2376,13 +2354,8 @@ __device__ void fallback_pixel(const FrameConst &c, const FrameBufs &b, const ui
 	}
 	if(lane == 0) {
 		write_pixel(c, b, px, py, acc, n);
-		lucid_info *info = (lucid_info *)b.info;
-		atomicAdd(&b.ctrl[kCtrlFallbackPixels], 1u);
-		// stats[2]: pixels resolved by the exact per-pixel sort (the reference counts the
-		// pixels its 3-deep window gets wrong there, shading.glsl:258-265)
-		atomicAdd(&info->stats[2], 1u);
-		if(whole)
-			atomicAdd(&info->stats[0], n); // these pixels skipped the block rasteriser
+		if(whole) // these pixels skipped the block rasteriser
+			atomicAdd(&((lucid_info *)b.info)->stats[0], n);
 	}
 }
 
@@ -2412,6 +2385,30 @@ __device__ __forceinline__ void fallback_kernel_body(const FrameConst &c, const 
 	const uint32_t w = wg.id * (kFallbackThreads / 64) + (threadIdx.x >> 6);
 	for(uint32_t qi = w; qi < nq; qi += waves)
 		fallback_pixel<FP32, TEX>(c, b, s_tex, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
+	// The pixels are counted once per work-group (an atomic each, on two words of the whole frame,
+	// took 130 of the kernel's 157 us for 17 k pixels of 32 fragments); the work-group that
+	// completes the count ends the frame. With an empty queue that is the first one.
+	constexpr uint32_t kItems = kFallbackThreads / 64;
+	if(nq ? wg.id * kItems >= nq : wg.id != 0)
+		return;
+	if(nq) {
+		uint32_t mine = 0;
+		for(uint32_t k = 0; k < kItems; k++) {
+			const uint32_t q0 = wg.id * kItems + k;
+			mine += q0 < nq ? (nq - q0 + waves - 1) / waves : 0u;
+		}
+		if(!last_work_group(&b.ctrl[kCtrlFallbackPixels], mine, nq))
+			return;
+		// stats[2]: pixels resolved by the exact per-pixel sort (the reference counts the
+		// pixels its 3-deep window gets wrong there, shading.glsl:258-265)
+		if(threadIdx.x == 0)
+			((lucid_info *)b.info)->stats[2] = nq;
+	}
+	// The control words go to pinned host memory, where the host reads them once the frame's
+	// event has completed (a copy command of 64 bytes: 4 us of the GPU, and its submission).
+	if(b.host_status && threadIdx.x < (uint32_t)kCtrlWords)
+		__hip_atomic_store(&b.host_status[threadIdx.x], agent_load(&b.ctrl[threadIdx.x]), __ATOMIC_RELAXED,
+						   __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <bool FP32, bool TEX>
@@ -3184,6 +3181,21 @@ __global__ __launch_bounds__(kFallbackThreads) void bwd_fallback_kernel(FrameCon
 		bwd_fallback_pixel(c, b, g, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
 }
 
+// Row generation of small frames (kFusedRasterBins) in one launch, where two would each end with
+// a nearly empty chip (767 x 431 particles 33 + gap -> 24 us, 1280 x 720 lit mesh 49 + gap -> 44);
+// larger ones fill it and do better apart, with the high bins' smaller groups (1440p mesh 310 us
+// apart, 350 in one launch).
+static void launch_rowgen(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
+	constexpr int kHigh = kRowgenSplitThreads / kRowgenThreads, kHighFused = kRowgenSplitThreads / kRowgenLowThreads;
+	if(c.bin_count <= kFusedRasterBins) {
+		hipLaunchKernelGGL(rowgen_fused_kernel, dim3(c.bin_count * (kHighFused + 1)), dim3(kRowgenLowThreads),
+						   0, stream, c, b);
+		return;
+	}
+	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
+	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kHigh), dim3(kRowgenThreads), 0, stream, c, b);
+}
+
 // Block bookkeeping and the pre-sort of long lists (up to kMidSortCap entries), then the
 // queued lists longer than that (one work-group per CU).
 static void launch_high_finalize(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
@@ -3225,12 +3237,9 @@ template <bool FP32, int MODE>
 static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 							hipEvent_t *ev) {
 	constexpr bool TEX = MODE == kShadeTextured;
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
+	launch_rowgen(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[0], stream);
-	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);
-	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kRowgenSplit), dim3(kRowgenThreads), 0,
-					   stream, c, b);
 	launch_high_finalize(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[1], stream);
@@ -3246,12 +3255,10 @@ static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t
 template <bool FP32, int W, int MODE>
 static void launch_raster_batch_t(const BatchPlan &p, hipStream_t stream) {
 	constexpr bool TEX = MODE == kShadeTextured;
-	hipLaunchKernelGGL(rowgen_low_kernel_batch, dim3(p.total[kBsRowgenLow]), dim3(kRowgenLowThreadsBatch), 0,
+	hipLaunchKernelGGL(rowgen_low_kernel_batch, dim3(p.total[kBsRowgenLow]), dim3(kRowgenThreads), 0,
 					   stream, p.frames, p.stage_pre(kBsRowgenLow), p.num_frames);
-	hipLaunchKernelGGL(high_prep_kernel_batch, dim3(p.total[kBsHighPrep]), dim3(1024), 0, stream,
-					   p.frames, p.stage_pre(kBsHighPrep), p.num_frames);
-	hipLaunchKernelGGL(rowgen_high_kernel_batch, dim3(p.total[kBsRowgenHigh]),
-					   dim3(kRowgenThreads), 0, stream, p.frames, p.stage_pre(kBsRowgenHigh), p.num_frames);
+	hipLaunchKernelGGL(rowgen_high_kernel_batch, dim3(p.total[kBsRowgenHigh]), dim3(kRowgenThreads), 0,
+					   stream, p.frames, p.stage_pre(kBsRowgenHigh), p.num_frames);
 	hipLaunchKernelGGL(high_finalize_kernel_batch, dim3(p.total[kBsHighFinalize]),
 					   dim3(kSortThreads), 0, stream, p.frames, p.stage_pre(kBsHighFinalize), p.num_frames);
 	hipLaunchKernelGGL(high_finalize_long_kernel_batch, dim3(p.total[kBsHighFinalizeLong]),
@@ -3266,17 +3273,9 @@ static void launch_raster_batch_t(const BatchPlan &p, hipStream_t stream) {
 					   dim3(kFallbackThreads), 0, stream, p.frames, p.stage_pre(kBsFallback), p.num_frames);
 }
 
-// Each frame's control words, for the host's overflow check (one copy per batch).
-__global__ __launch_bounds__(64) void batch_status_kernel(const FrameDesc *frames, uint32_t n,
-														 uint32_t *status) {
-	const uint32_t f = blockIdx.x;
-	if(f < n && threadIdx.x < (uint32_t)kCtrlWords)
-		status[(size_t)f * kCtrlWords + threadIdx.x] = frames[f].b.ctrl[threadIdx.x];
-}
-
 // Row generation, sorting, block rasterisation and the exact fallback of every frame of a
 // batch: one launch per stage, kernels chosen by the batch's sample format, slice width and
-// shading mode; then the frames' control words into p.status.
+// shading mode.
 template <int W>
 static void launch_raster_batch_w(const BatchPlan &p, hipStream_t stream) {
 	if(p.fp32)
@@ -3297,12 +3296,10 @@ hipError_t launch_raster_batch(const BatchPlan &p, hipStream_t stream) {
 		launch_raster_batch_w<2>(p, stream);
 	else
 		launch_raster_batch_w<1>(p, stream);
-	hipLaunchKernelGGL(batch_status_kernel, dim3(p.num_frames), dim3(64), 0, stream, p.frames,
-					   p.num_frames, p.status);
 	return hipGetLastError();
 }
 
-// events (optional, 4): after rowgen_low, after the high-bin row generation and sorting,
+// events (optional, 4): after the row generation, after the sorting of long block lists,
 // after block rasterisation, after the fallback kernel.
 hipError_t launch_raster(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 						 hipEvent_t *events) {
@@ -3328,10 +3325,7 @@ hipError_t launch_raster(const FrameConst &c, const FrameBufs &b, hipStream_t st
 // recomputed, not stored), then the gradient row allocation.
 hipError_t launch_backward_prepare(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								   hipStream_t stream) {
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
-	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);
-	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kRowgenSplit), dim3(kRowgenThreads), 0,
-					   stream, c, b);
+	launch_rowgen(c, b, stream);
 	launch_high_finalize(c, b, stream);
 	hipLaunchKernelGGL(grad_row_scan_kernel<false>, dim3(1), dim3(1024), 0, stream, c, b, g);
 	return hipGetLastError();
@@ -3358,12 +3352,9 @@ __global__ __launch_bounds__(64) void record_gate_kernel(FrameBufs b, BwdBufs g)
 // (which then render only what the recording pass does not).
 hipError_t launch_raster_recording(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								   hipStream_t stream, hipEvent_t *ev) {
-	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
+	launch_rowgen(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[0], stream);
-	hipLaunchKernelGGL(high_prep_kernel, dim3(1), dim3(1024), 0, stream, c, b);
-	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kRowgenSplit), dim3(kRowgenThreads), 0,
-					   stream, c, b);
 	launch_high_finalize(c, b, stream);
 	hipLaunchKernelGGL(grad_row_scan_kernel<false>, dim3(1), dim3(1024), 0, stream, c, b, g);
 	hipLaunchKernelGGL(record_gate_kernel, dim3(1), dim3(64), 0, stream, b, g);

@@ -67,3 +67,37 @@ def test_raster_launch_threshold(oracle_mod, w, h, opts):
     assert n + b.num_verts == sc.num_verts
     r, gpu, ref = _render_both(sc, oracle_mod, opts=opts)
     _check(sc, gpu, ref, oracle_mod)
+
+
+def _stacks(w, h, per_bin, counts, seed):
+    """`counts[i]` triangles over one block in the middle of bin i (row-major, 32 x 32 pixels)."""
+    rng = np.random.default_rng(seed)
+    bins = np.repeat(np.arange(len(counts)), counts)
+    nbx = (w + 31) // 32
+    c = np.stack([bins % nbx, bins // nbx], -1)[:, None] * 32.0 + 12.0
+    off = np.array([[-3.0, -3.0], [4.0, -3.0], [-3.0, 4.0]]) + rng.uniform(-0.4, 0.4, (len(bins), 3, 2))
+    ndc = (c + off + 0.5) / np.array([w, h]) * 2.0 - 1.0
+    n = len(bins)
+    return scenes.soup_scene(w, h, ndc, rng.uniform(1.0, 90.0, n), rng.uniform(0, 1, (n, 3, 3)),
+                             rng.uniform(0.05, 0.4, n), name=f"stacks_{w}x{h}_{per_bin}")
+
+
+def test_promoted_bins_overflow_the_lists(oracle_mod):
+    """512 promoted bins, whose list space (16 lists of 1000 positions each) is more than a new
+    renderer has: the frame is rendered again with larger lists."""
+    sc = _stacks(1024, 512, 500, np.full(512, 500), seed=5)
+    r, gpu, ref = _render_both(sc, oracle_mod)
+    assert gpu["stats"]["high_bins"] >= 512
+    _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("w,h", [(2080, 1056), (1000, 37), (2500, 300)])
+def test_many_bins(oracle_mod, w, h):
+    """More bins than one step of the categorising work-group takes (2048), and rows of bins that
+    end inside a step; empty, low, promoted and high bins mixed."""
+    rng = np.random.default_rng(w)
+    nb = ((w + 31) // 32) * (h // 32)
+    counts = rng.choice([0, 1, 7, 300, 520], nb, p=[0.5, 0.2, 0.25, 0.03, 0.02])
+    sc = _stacks(w, h, "mixed", counts, seed=w)
+    r, gpu, ref = _render_both(sc, oracle_mod)
+    _check(sc, gpu, ref, oracle_mod)

@@ -154,7 +154,7 @@ struct FrameConst {
 	uint32_t presort_min;      // high-bin blocks with more entries are pre-sorted (<= kRegSortCap)
 	uint32_t samples_per_wave; // target samples per wave of a pre-sorted block
 	int slice_words;           // block rasteriser slice width: 1 or 2 words of 64 entries
-	int window;                // ordering window of flat-colour frames (tuning): 1 or 4
+	int window;                // ordering window (tuning): 1 (narrow) or 4
 	int color_mode;
 	int has_normals;
 	// 1 when an earlier frame of the renderer may still be running: the clear kernel then
@@ -165,6 +165,8 @@ struct FrameConst {
 	// ambient 1 and no sun light: every lighting factor of the frame is exactly 1, and
 	// finalShading's sRGB round trip L2S(S2L(x) * 1) is the identity
 	int identity_light;
+	// fp32 vertex colours on every instance, no instance colours or textures, identity_light
+	int plain_colors;
 	float vp[16]; // column-major view-projection matrix
 	float origin[3], dir0[3], dirx[3], diry[3], ray_dir0[3];
 	float ambient[3], sun_color[3], sun_dir[3];
@@ -313,17 +315,21 @@ __device__ __forceinline__ uint32_t batch_frame(const StageBatch &sb, uint32_t w
 // textures, or flat colour planes (RGBA8 samples, unit lighting, vertex colours absent or
 // fp32 with a per-triangle alpha, no textures: a sample's colour is then an affine function
 // of the pixel divided by the inverse depth).
-// kShadeFlatNarrow: flat records with the narrow ordering windows (tuning window 1).
-enum ShadeMode : int { kShadeGeneral = 0, kShadeTextured = 1, kShadeFlat = 2, kShadeFlatNarrow = 3 };
+// kShadePlain: the same frames with fp32 samples whose instances all have fp32 vertex colours
+// and no instance colour (the general shading's values, without its tests).
+// kShadeNarrow (a flag): narrow ordering windows (tuning window 1).
+enum ShadeMode : int { kShadeGeneral = 0, kShadeTextured = 1, kShadeFlat = 2, kShadePlain = 3, kShadeNarrow = 4 };
 
 inline int frame_shade_mode(const FrameConst &c) {
-	if(c.has_textures)
-		return kShadeTextured;
 	const bool fp32 = (c.opts & LUCID_OPT_FP32_SAMPLES) != 0;
 	const bool flat_colors = c.color_mode == kColorNone || c.color_mode == kColorF32;
-	if(fp32 || !c.identity_light || !flat_colors)
-		return kShadeGeneral;
-	return c.window == 1 ? kShadeFlatNarrow : kShadeFlat;
+	const int kind = c.has_textures ? kShadeTextured
+					 : fp32 ? (c.plain_colors ? kShadePlain : kShadeGeneral)
+							: (c.identity_light && flat_colors ? kShadeFlat : kShadeGeneral);
+	// the alpha threshold looks at the samples that have left the window, so its results depend
+	// on the slots: only flat frames take it with the narrow ones
+	const bool threshold = (c.opts & LUCID_OPT_ALPHA_THRESHOLD) != 0;
+	return kind | (c.window == 1 && (kind == kShadeFlat || !threshold) ? kShadeNarrow : 0);
 }
 
 struct BatchPlan {
@@ -333,7 +339,7 @@ struct BatchPlan {
 	uint32_t total[kBsCount]; // work-groups of each stage over all frames
 	size_t bin_lds;           // dynamic LDS of the bin kernels: the largest frame's
 	bool fp32;
-	int mode; // ShadeMode of the block kernels: textured if a frame is, flat if every frame is
+	int mode; // ShadeMode of the block kernels: textured if a frame is, flat or plain if every frame is
 	int slice_words;
 	__host__ const uint32_t *stage_pre(int s) const { return pre + (size_t)s * (num_frames + 1); }
 };

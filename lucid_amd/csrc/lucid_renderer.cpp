@@ -446,13 +446,14 @@ TexDesc tex_desc(const lucid_texture &t) {
 	return d;
 }
 
+// plain: every instance has vertex colours and none an instance colour or a texture.
 int validate_inputs(const lucid_frame_inputs *in, int *prefix, int64_t &nq, int &color_mode,
-					bool &textured) {
+					bool &textured, bool &plain) {
 	if(!in->config || in->num_instances < 0 || in->num_instances > kMaxInstances ||
 	   (in->num_instances > 0 && !in->instances))
 		return LUCID_ERR_INVALID_ARG;
 	nq = 0;
-	textured = false;
+	textured = false, plain = true;
 	bool has_colors_flag = false;
 	for(int i = 0; i < in->num_instances; i++) {
 		const lucid_instance_data &ins = in->instances[i];
@@ -468,6 +469,8 @@ int validate_inputs(const lucid_frame_inputs *in, int *prefix, int64_t &nq, int 
 		}
 		if(ins.flags & LUCID_INST_HAS_VERTEX_COLORS)
 			has_colors_flag = true;
+		plain = plain && (ins.flags & (LUCID_INST_HAS_VERTEX_COLORS | LUCID_INST_HAS_COLOR |
+									   LUCID_INST_HAS_ALBEDO_TEXTURE)) == LUCID_INST_HAS_VERTEX_COLORS;
 		prefix[i] = (int)nq;
 		nq += ins.num_quads;
 		if(nq >= kMaxQuads)
@@ -499,8 +502,8 @@ int prepare_frame(lucid_renderer *r, const lucid_frame_inputs *in, const lucid_f
 	std::vector<int> prefix(in->num_instances + 1, 0);
 	int64_t nq = 0;
 	int color_mode = kColorNone;
-	bool textured = false;
-	int ve = validate_inputs(in, prefix.data(), nq, color_mode, textured);
+	bool textured = false, plain = false;
+	int ve = validate_inputs(in, prefix.data(), nq, color_mode, textured, plain);
 	if(ve != LUCID_OK)
 		return ve;
 
@@ -585,6 +588,7 @@ int prepare_frame(lucid_renderer *r, const lucid_frame_inputs *in, const lucid_f
 
 	fill_const(r->width, r->height, r->opts, r->tuning, *in->config, nq, in->num_instances,
 			   color_mode, in->normals != nullptr, c);
+	c.plain_colors = plain && color_mode == kColorF32 && c.identity_light ? 1 : 0;
 	c.keep_overflow = r->frame_pending ? 1u : 0u;
 	c.has_textures = textured ? 1 : 0;
 	memset(&b, 0, sizeof(b));
@@ -1171,7 +1175,8 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 	}
 	const size_t n = bt->rs.size();
 	std::vector<FrameDesc> frames(n);
-	bool tex = false, flat = true;
+	bool tex = false, fast = true, narrow = true; // fast: flat or plain records for every frame
+	int fast_mode = kShadeGeneral;
 	for(size_t i = 0; i < n; i++) {
 		lucid_renderer *r = bt->rs[i];
 		if(r->frame_pending) {
@@ -1188,7 +1193,10 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 		frames[i].c.slice_words = bt->rs[0]->tuning.slice_words;
 		frames[i].b.host_status = bt->status_dev + i * kCtrlWords;
 		tex = tex || frames[i].c.has_textures;
-		flat = flat && frame_shade_mode(frames[i].c) >= kShadeFlat; // flat records, either window
+		const int mode = frame_shade_mode(frames[i].c);
+		narrow = narrow && (mode & kShadeNarrow);
+		fast_mode = mode & ~kShadeNarrow;
+		fast = fast && (fast_mode == kShadeFlat || fast_mode == kShadePlain);
 		r->last_num_quads = nq;
 		r->last_stream = stream;
 		r->retained.valid = r->retained.pending = false;
@@ -1212,9 +1220,9 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 	plan.num_frames = (uint32_t)n;
 	plan.bin_lds = bin_lds;
 	plan.fp32 = (bt->rs[0]->opts & LUCID_OPT_FP32_SAMPLES) != 0;
-	plan.mode = tex ? kShadeTextured
-					: flat ? (bt->rs[0]->tuning.window == 1 ? kShadeFlatNarrow : kShadeFlat)
-						   : kShadeGeneral;
+	// (one sample format: fast frames are all flat or all plain)
+	plan.mode = (tex ? kShadeTextured : fast ? fast_mode : kShadeGeneral) |
+				(narrow ? kShadeNarrow : 0);
 	plan.slice_words = bt->rs[0]->tuning.slice_words;
 	// the launches read the frames' constants and buffers from device memory, so a frame
 	// whose inputs change only needs them uploaded; the graph is recorded again only when a
@@ -1386,8 +1394,8 @@ int lucid_render_noalloc(int width, int height, uint32_t opts, const lucid_tunin
 	int color_mode = kColorNone;
 	if(in->num_instances < 0)
 		return LUCID_ERR_INVALID_ARG;
-	bool textured = false;
-	int ve = validate_inputs(in, prefix, nq, color_mode, textured);
+	bool textured = false, plain = false;
+	int ve = validate_inputs(in, prefix, nq, color_mode, textured, plain);
 	if(ve != LUCID_OK)
 		return ve;
 	if(nq > kNaMaxQuads)
@@ -1406,6 +1414,7 @@ int lucid_render_noalloc(int width, int height, uint32_t opts, const lucid_tunin
 	FrameConst c;
 	fill_const(width, height, opts & ~(uint32_t)LUCID_OPT_TIMERS, t, *in->config, nq,
 			   in->num_instances, color_mode, in->normals != nullptr, c);
+	c.plain_colors = plain && color_mode == kColorF32 && c.identity_light ? 1 : 0;
 	c.keep_overflow = 0u;
 	FrameBufs b;
 	memset(&b, 0, sizeof(b));

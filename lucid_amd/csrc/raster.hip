@@ -29,9 +29,12 @@ namespace lucid {
 constexpr int kSortThreads = 256;
 constexpr int kFallbackThreads = 256;
 constexpr int kWindow = 4;
-// Narrow ordering windows (tuning window 1): one slot in the register-sorted blocks and in
-// the pre-sorted ones (whose depth ranks keep 32 - log2 of the padded list length bits).
-constexpr int kNarrowWindow = 1, kNarrowBigWindow = 1;
+// Narrow ordering windows (tuning window 1): one slot for flat and plain records, in the
+// register-sorted blocks and in the pre-sorted ones (whose depth ranks keep 32 - log2 of the padded
+// list length bits); two for the general records of register-sorted blocks, where a pixel sent to
+// the exact sort costs more (4 -> 2 slots: 1280 x 720 lit mesh 98 -> 83 us, textured planes 254 ->
+// 237). The fp32 soup of 41 M fragments at 512 x 512: four slots 178 us, two 138, one 121.
+constexpr int kNarrowWindow = 1, kNarrowPlainWindow = 1, kNarrowGeneralWindow = 2;
 constexpr int kFallbackCap = 512; // fragments per pixel sorted in LDS by the fallback kernel
 
 // ------------------------------------------------------------------ shading
@@ -1752,7 +1755,20 @@ __device__ __forceinline__ void transpose_masks(const uint64_t (&msk)[W], int nw
 // is the same affine function (rounding differs by a few ulps, inside the 1/255 colour bar);
 // the depth key keeps its unfused evaluation. The instance colour is folded into the planes.
 constexpr int kFlatQuads = 5; // f0 depth plane | triangle id; f1-f3 r, g, b planes; f4 alpha
-constexpr bool is_flat(int mode) { return mode == kShadeFlat || mode == kShadeFlatNarrow; }
+constexpr int shade_kind(int mode) { return mode & ~kShadeNarrow; }
+constexpr bool is_flat(int mode) { return shade_kind(mode) == kShadeFlat; }
+constexpr bool is_plain(int mode) { return shade_kind(mode) == kShadePlain; }
+constexpr bool is_textured(int mode) { return shade_kind(mode) == kShadeTextured; }
+// Window slots of the register-sorted and the pre-sorted blocks. A pre-sorted pixel's depth ranges
+// are composited apart and then chained, which rounds differently from the exact sort: there the
+// general kinds keep four slots, so that no RGBA8 pixel changes to the exact sort by the tuning.
+constexpr int window_slots(int mode, bool presorted) {
+	return !(mode & kShadeNarrow) ? kWindow
+		   : is_flat(mode)		  ? kNarrowWindow
+		   : is_plain(mode)		  ? kNarrowPlainWindow
+		   : presorted			  ? kWindow
+								  : kNarrowGeneralWindow;
+}
 constexpr int rec_quads(int mode) { return is_flat(mode) ? kFlatQuads : kRecQuads; }
 // LDS of one wave's slice of 64 W records
 template <int W, int MODE> constexpr int slice_quads() { return 64 * W * rec_quads(MODE); }
@@ -1811,6 +1827,45 @@ __device__ __forceinline__ SampleColor<false> shade_flat(const uint4 *f, float p
 	return out;
 }
 
+// ------------------------------------------------------------------ plain records
+//
+// Frames with fp32 samples whose instances all have fp32 vertex colours, unit lighting and no
+// instance colour (kShadePlain) keep the general record's planes and colours (its first six
+// quads, the triangle id in place of the flags; still kRecQuads apart, as six quads would put
+// twice as many entries on one LDS bank) and evaluate the general shading without its tests of
+// instance flags and frame options: the same operations on the same values, bit for bit. These
+// kernels are bound by VALU issue: 41 M fragments at 512 x 512, forward raster 204 -> 121 us (with
+// the one-slot window), pass A 214 -> 179, pass B 534 -> 441 (with its eight rotated orders and
+// 12.5 KB of LDS instead of 15.5).
+constexpr int kPlainQuads = 6; // depth plane | triangle id; two barycentric planes; c0 | alpha; c1; c2
+
+struct PlainShade {
+	float b0, b1; // barycentrics
+	float x[3];   // interpolated colour, unclamped
+	float alpha;
+};
+__device__ __forceinline__ PlainShade shade_plain(const uint4 *q, float px, float py, float inv_ray) {
+	PlainShade o;
+	const uint4 p0 = q[1], p1 = q[2], q3 = q[3], q4 = q[4], q5 = q[5];
+	const float ray_pos = __builtin_amdgcn_rcpf(inv_ray);
+	const float e0 = bits2f(p0.x) * px + (bits2f(p0.y) * py + bits2f(p0.z));
+	const float e1 = bits2f(p1.x) * px + (bits2f(p1.y) * py + bits2f(p1.z));
+	o.b0 = e0 * ray_pos - bits2f(p0.w);
+	o.b1 = e1 * ray_pos - bits2f(p1.w);
+	const float w0 = (1.0f - o.b0) - o.b1;
+	o.x[0] = w0 * bits2f(q3.x) + (o.b0 * bits2f(q4.x) + o.b1 * bits2f(q5.x));
+	o.x[1] = w0 * bits2f(q3.y) + (o.b0 * bits2f(q4.y) + o.b1 * bits2f(q5.y));
+	o.x[2] = w0 * bits2f(q3.z) + (o.b0 * bits2f(q4.z) + o.b1 * bits2f(q5.z));
+	o.alpha = bits2f(q3.w);
+	return o;
+}
+__device__ __forceinline__ SampleColor<true> plain_sample(const uint4 *q, float px, float py, float inv_ray) {
+	const PlainShade p = shade_plain(q, px, py, inv_ray);
+	SampleColor<true> out;
+	out.col = make_float4(sat(p.x[0]), sat(p.x[1]), sat(p.x[2]), p.alpha);
+	return out;
+}
+
 // Stages the shading records of a slice in LDS: lane l writes entries l + 64 k.
 template <int W, int MODE = kShadeGeneral>
 __device__ __forceinline__ void stage_slice(const FrameConst &c, const FrameBufs &b,
@@ -1826,6 +1881,12 @@ __device__ __forceinline__ void stage_slice(const FrameConst &c, const FrameBufs
 			const uint4 *src = b.tri_shade + (size_t)kRecStride * tri_rec(b, tri[k]);
 			if constexpr(is_flat(MODE)) {
 				make_flat_record(src, s_rec + i * kFlatQuads);
+			} else if constexpr(is_plain(MODE)) {
+				const uint4 q0 = src[0];
+				s_rec[i * kRecQuads] = make_uint4(q0.x, q0.y, q0.z, tri[k]);
+#pragma unroll
+				for(int j = 1; j < kPlainQuads; j++)
+					s_rec[i * kRecQuads + j] = src[j];
 			} else {
 #pragma unroll
 				for(int j = 0; j < kRecQuads; j++)
@@ -1900,7 +1961,23 @@ __device__ __forceinline__ void walk_pixel_t(const FrameConst &c, const FrameBuf
 		});
 		return;
 	}
-	constexpr bool TEX = MODE == kShadeTextured;
+	if constexpr(is_plain(MODE)) {
+		static_assert(FP32, "plain records carry fp32 samples");
+		walk_bits(bm, [&](int e) {
+			const uint4 *rec = s_rec + e * kRecQuads;
+			const uint4 q0 = rec[0];
+			const float inv = record_inv_depth(q0, px, py);
+			const SampleColor<true> col = plain_sample(rec, px, py, inv);
+			if(col.contributes()) {
+				if(unsorted)
+					ps.acc.blend(col, additive);
+				else
+					ps.insert(pixel_key(inv, q0.w), col, additive);
+			}
+		});
+		return;
+	}
+	constexpr bool TEX = is_textured(MODE);
 	walk_bits(bm, [&](int e) {
 		const uint4 *rec = s_rec + e * kRecQuads;
 		const uint4 q0 = rec[0];
@@ -2018,7 +2095,7 @@ __device__ __forceinline__ void raster_sorted_block(const FrameConst &c, const F
 	}
 	const bool additive = (c.opts & (1u << 5)) != 0;
 	const bool threshold = alpha_threshold_on(c);
-	PixelState<FP32, MODE == kShadeFlatNarrow ? kNarrowWindow : kWindow> ps;
+	PixelState<FP32, window_slots(MODE, false)> ps;
 	ps.init();
 	uint32_t count = 0;
 	bool opaque = false; // every pixel of the block is nearly opaque (alpha threshold)
@@ -2094,7 +2171,7 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 	const bool additive = (c.opts & (1u << 5)) != 0;
 	if((uint32_t)wave < nw) {
 		const uint32_t e0 = hdr[1 + wave], e1 = hdr[2 + wave];
-		PixelState<FP32, MODE == kShadeFlatNarrow ? kNarrowBigWindow : kWindow> ps;
+		PixelState<FP32, window_slots(MODE, true)> ps;
 		ps.init();
 		uint32_t count = 0;
 		const bool threshold = alpha_threshold_on(c);
@@ -2162,10 +2239,10 @@ template <bool FP32, int W, int MODE>
 __device__ __forceinline__ void block_raster_body(const FrameConst &c, const FrameBufs &b,
 												  uint32_t id) {
 	__shared__ uint4 s_rec[slice_quads<W, MODE>()];
-	__shared__ uint4 s_tex[MODE == kShadeTextured ? kTexTable : 1];
+	__shared__ uint4 s_tex[is_textured(MODE) ? kTexTable : 1];
 	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
 		return;
-	if constexpr(MODE == kShadeTextured)
+	if constexpr(is_textured(MODE))
 		fill_tex_table(b, s_tex); // (one wave: the syncs before the first walk cover it)
 	raster_sorted_block<FP32, W, MODE>(c, b, id, s_rec, s_tex);
 }
@@ -2173,10 +2250,10 @@ template <bool FP32, int W, int MODE>
 __device__ __forceinline__ void block_raster_big_body(const FrameConst &c, const FrameBufs &b,
 													  uint32_t id) {
 	__shared__ uint4 s_rec[kBigWaves][slice_quads<W, MODE>()];
-	__shared__ uint4 s_tex[MODE == kShadeTextured ? kTexTable : 1];
+	__shared__ uint4 s_tex[is_textured(MODE) ? kTexTable : 1];
 	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
 		return;
-	if constexpr(MODE == kShadeTextured) {
+	if constexpr(is_textured(MODE)) {
 		fill_tex_table(b, s_tex);
 		__syncthreads();
 	}
@@ -2217,7 +2294,7 @@ constexpr int kFusedRasterBins = 1024;
 static_assert(kBigWaves == 4, "a bin's 16 blocks are four work-groups of register-sorted blocks");
 template <bool FP32, int MODE>
 __global__ __launch_bounds__(kBigWaves * 64, FP32 ? 4 : 1) void block_raster_fused_kernel(FrameConst c, FrameBufs b) {
-	static_assert(MODE != kShadeTextured, "no texture table here");
+	static_assert(!is_textured(MODE), "no texture table here");
 	__shared__ uint4 s_rec[kBigWaves][slice_quads<1, MODE>()];
 	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
 		return;
@@ -2588,6 +2665,7 @@ __device__ __forceinline__ BlockEntries bwd_block_entries(const FrameConst &c, c
 }
 
 // Loads and stages slice [s0, s0 + n) of the block's entries; returns the coverage masks.
+template <int MODE>
 __device__ __forceinline__ void bwd_stage(const FrameConst &c, const FrameBufs &b,
 										  const BlockEntries &ent, uint32_t s0, uint32_t n,
 										  uint4 *s_rec, uint64_t (&msk)[kSliceWords]) {
@@ -2599,7 +2677,7 @@ __device__ __forceinline__ void bwd_stage(const FrameConst &c, const FrameBufs &
 		msk[k] = i < n ? ent.mask[s0 + i] : 0ull;
 		t[k] = i < n ? ent.tri[s0 + i] : 0u;
 	}
-	stage_slice(c, b, t, n, s_rec);
+	stage_slice<kSliceWords, MODE>(c, b, t, n, s_rec);
 	wave_sync_lds();
 }
 
@@ -2626,7 +2704,8 @@ __device__ __forceinline__ bool bwd_fits(const FrameBufs &b, const BwdBufs &g) {
 // dL/dpixel), the BwdRecord of each (range, pixel) and the pixel's clamp/exact flags;
 // bwd_start_kernel turns them into start states when the backward runs.
 // WIN: slots of the ordering window (4, or 2 with the narrow-window tuning).
-template <bool RECORD, int WIN>
+// MODE: kShadePlain or kShadeGeneral.
+template <bool RECORD, int WIN, int MODE>
 __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c, FrameBufs b,
 																	 BwdBufs g) {
 	if(b.ctrl[kCtrlOverflow] & kOvfBinLists)
@@ -2682,7 +2761,7 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 		for(uint32_t s0 = ent.e0; s0 < ent.e1; s0 += kSliceEntries) {
 			const uint32_t n = min(ent.e1 - s0, (uint32_t)kSliceEntries);
 			uint64_t msk[kSliceWords];
-			bwd_stage(c, b, ent, s0, n, s_rec[wave], msk);
+			bwd_stage<MODE>(c, b, ent, s0, n, s_rec[wave], msk);
 			// the triangle of each gradient row (pass B fills the row itself)
 			for(uint32_t e = lane; e < n; e += 64)
 				g.row_tri[(size_t)row0 + s0 + e] = ent.tri[s0 + e];
@@ -2698,13 +2777,18 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 			};
 			walk_bits(bm, [&](int e) {
 				const uint4 *rec = s_rec[wave] + e * kRecQuads;
-				const float inv = record_inv_depth(rec[0], fx, fy);
-				const SampleColor<true> col = shade_record<true, false>(c, b, nullptr, rec, fx, fy, inv);
+				const uint4 q0 = rec[0];
+				const float inv = record_inv_depth(q0, fx, fy);
+				SampleColor<true> col;
+				if constexpr(is_plain(MODE))
+					col = plain_sample(rec, fx, fy, inv);
+				else
+					col = shade_record<true, false>(c, b, nullptr, rec, fx, fy, inv);
 				if(col.contributes()) {
 					BwdColor bc;
 					bc.r = col.col.x, bc.g = col.col.y, bc.b = col.col.z, bc.a = col.col.w;
 					bc.e = (uint32_t)e;
-					w.insert(pixel_key(inv, rec[6].z), bc, emit);
+					w.insert(pixel_key(inv, is_plain(MODE) ? q0.w : rec[6].z), bc, emit);
 				}
 			});
 			// the window empties at every slice end, so pass B only needs this slice staged
@@ -2846,13 +2930,13 @@ constexpr int kGradStride = kGradWords + 1; // odd stride against bank conflicts
 
 // One wave per (block, depth range); single-wave work-groups (no LDS is shared between
 // waves), so that more of them fit on a CU.
+// MODE: kShadePlain or kShadeGeneral.
+template <int MODE>
 __global__ __launch_bounds__(64) void bwd_pass_b_kernel(FrameConst c, FrameBufs b, BwdBufs g) {
 	if((b.ctrl[kCtrlOverflow] & kOvfBinLists) || !bwd_fits(b, g))
 		return;
 	__shared__ uint4 s_rec[kSliceEntries * kRecQuads];
 	__shared__ unsigned long long s_grad[kSliceEntries * kGradStride];
-	__shared__ uint32_t s_tri_all[kRegSortCap];
-	__shared__ uint64_t s_mask_all[kRegSortCap];
 	const int lane = lane_id();
 	const uint32_t slot = blockIdx.x / kBigWaves;
 	const int wave = (int)(blockIdx.x % kBigWaves);
@@ -2874,19 +2958,50 @@ __global__ __launch_bounds__(64) void bwd_pass_b_kernel(FrameConst c, FrameBufs 
 	const int px = (bin % c.bin_count_x) * kBinSize + bx * 8 + (lane & 7);
 	const int py = (bin / c.bin_count_x) * kBinSize + by * 8 + (lane >> 3);
 	const float fx = (float)px, fy = (float)py;
-	const BlockEntries ent = bwd_block_entries(c, b, slot, flags, sl, wave, s_tri_all, s_mask_all);
+	// The block's triangles in depth order: the pre-sorted pool, or the lane's entries of a register
+	// sort. (Kept in LDS, as pass A has them, they took 3 of the wave's 16 KB, and the kernel is
+	// short of waves: 10 per CU instead of 12.)
+	const uint32_t *sorted = nullptr;
+	uint32_t e0 = 0, e1 = sl.y, tri_all[4] = {0u, 0u, 0u, 0u};
+	if(flags & kSlotPresorted) {
+		const uint32_t *hdr = b.sorted_pool + b.blk_sorted[slot];
+		sorted = hdr + kSortedHeader;
+		e0 = hdr[1 + wave], e1 = hdr[2 + wave];
+	} else {
+		uint64_t *s_msk = reinterpret_cast<uint64_t *>(s_rec);
+		uint32_t *s_tri = reinterpret_cast<uint32_t *>(s_msk + kRegSortCap);
+		static_assert(sizeof(s_rec) >= kRegSortCap * 12, "the sort's ids and masks fit the staging area");
+		uint32_t pos[4];
+		sort_block_positions(b.blk_lists + sl.x, sl.y, pos, s_msk, s_tri);
+		wave_sync_lds();
+#pragma unroll
+		for(int j = 0; j < 4; j++)
+			if(j * 64 + lane < (int)sl.y)
+				tri_all[j] = s_tri[pos[j]];
+		wave_sync_lds(); // read before the first slice is staged over them
+	}
 	const uint32_t row0 = g.row_base[slot];
 	const BwdStart st = g.start[((size_t)g.range_base[slot] + wave) * 64 + lane];
 	double t = st.t, q = st.q;
 	const bool live = st.gr != 0.0f || st.gg != 0.0f || st.gb != 0.0f;
 	const int fix_k = grad_fixed_exp(c, bits2f(b.ctrl[kCtrlBwdGradMax]));
 	const double fix_scale = ldexp(1.0, fix_k);
-	const bool rot_b0 = (lane & 1) != 0, rot_b1 = (lane & 2) != 0;
-	const int rot = rot_b1 ? (rot_b0 ? 8 : 5) : (rot_b0 ? 3 : 0);
-	for(uint32_t s0 = ent.e0; s0 < ent.e1; s0 += kSliceEntries) {
-		const uint32_t n = min(ent.e1 - s0, (uint32_t)kSliceEntries);
-		uint64_t msk[kSliceWords];
-		bwd_stage(c, b, ent, s0, n, s_rec, msk);
+	// the lane's slots of the ten components: component k of the rotated order is added at kk[k]
+	const bool rot1 = (lane & 1) != 0, rot2 = (lane & 2) != 0, rot4 = (lane & 4) != 0;
+	const int rot = (rot1 ? 3 : 0) + (rot2 ? 5 : 0) + (rot4 ? 1 : 0);
+	static_assert(kSliceEntries == 64, "a lane stages one entry of a slice");
+	for(uint32_t s0 = e0; s0 < e1; s0 += kSliceEntries) {
+		const uint32_t n = min(e1 - s0, (uint32_t)kSliceEntries);
+		uint32_t tri[1] = {0u};
+		if(sorted) {
+			if((uint32_t)lane < n)
+				tri[0] = sorted[s0 + lane];
+		} else {
+#pragma unroll
+			for(uint32_t j = 0; j < 4; j++)
+				tri[0] = s0 == j * 64 ? tri_all[j] : tri[0];
+		}
+		stage_slice<kSliceWords, MODE>(c, b, tri, n, s_rec);
 		for(int i = lane; i < kSliceEntries * kGradStride; i += 64)
 			s_grad[i] = 0ull;
 		wave_sync_lds();
@@ -2901,23 +3016,42 @@ __global__ __launch_bounds__(64) void bwd_pass_b_kernel(FrameConst c, FrameBufs 
 			const uint4 *rec = s_rec + (uint32_t)e * kRecQuads;
 			const float inv = record_inv_depth(rec[0], fx, fy);
 			BwdSample smp;
-			shade_grad(c, b, rec, fx, fy, inv, smp);
+			if constexpr(is_plain(MODE)) {
+				const PlainShade p = shade_plain(rec, fx, fy, inv);
+				smp.b0 = p.b0, smp.b1 = p.b1;
+				smp.r = sat(p.x[0]), smp.g = sat(p.x[1]), smp.b = sat(p.x[2]), smp.a = p.alpha;
+				// (recorded samples have an alpha other than 0; the clamp passes the gradient on [0, 1])
+				smp.dr = p.x[0] >= 0.0f && p.x[0] <= 1.0f ? 1.0f : 0.0f;
+				smp.dg = p.x[1] >= 0.0f && p.x[1] <= 1.0f ? 1.0f : 0.0f;
+				smp.db = p.x[2] >= 0.0f && p.x[2] <= 1.0f ? 1.0f : 0.0f;
+				smp.da = 1.0f;
+			} else {
+				shade_grad(c, b, rec, fx, fy, inv, smp);
+			}
 			float out[kGradWords];
 			bwd_fragment(t, q, st.gr, st.gg, st.gb, smp, out);
 			if(live) {
-				// lanes add the ten components in four rotated orders (pixel column mod 4: by
-				// 0, 3, 5 or 8), so that pixels at the same entry in the same step seldom hit
-				// one address (integer sums: the order changes no bit). The order is picked with
-				// selects on two lane bits: an equality chain on lane & 3 would compile to a
-				// branchy switch per component.
+				// Lanes add the ten components in eight rotated orders (by pixel column: 0, 3, 5, 8, 1,
+				// 4, 6 and 9), so that pixels at the same entry in the same step seldom hit one
+				// address (integer sums: the order changes no bit). The rotation is three stages of
+				// selects on a lane bit each, as many as one four-way choice per component takes.
+				float r1[kGradWords], r2[kGradWords], r3[kGradWords];
+				// (by value: a choice between array elements would become one of addresses)
+				auto sel = [](bool p, float x, float y) { return p ? x : y; };
+#pragma unroll
+				for(int k = 0; k < kGradWords; k++)
+					r1[k] = sel(rot1, out[(k + 3) % kGradWords], out[k]);
+#pragma unroll
+				for(int k = 0; k < kGradWords; k++)
+					r2[k] = sel(rot2, r1[(k + 5) % kGradWords], r1[k]);
+#pragma unroll
+				for(int k = 0; k < kGradWords; k++)
+					r3[k] = sel(rot4, r2[(k + 1) % kGradWords], r2[k]);
 #pragma unroll
 				for(int k = 0; k < kGradWords; k++) {
-					const int k1 = (k + 3) % kGradWords, k2 = (k + 5) % kGradWords;
-					const int k3 = (k + 8) % kGradWords;
-					const float v = rot_b1 ? (rot_b0 ? out[k3] : out[k2]) : (rot_b0 ? out[k1] : out[k]);
 					const int kk0 = k + rot;
 					const int kk = kk0 >= kGradWords ? kk0 - kGradWords : kk0;
-					atomicAdd(&s_grad[(uint32_t)e * kGradStride + kk], to_fixed(v, fix_scale));
+					atomicAdd(&s_grad[(uint32_t)e * kGradStride + kk], to_fixed(r3[k], fix_scale));
 				}
 			}
 		}
@@ -3204,6 +3338,31 @@ static void launch_high_finalize(const FrameConst &c, const FrameBufs &b, hipStr
 	hipLaunchKernelGGL(high_finalize_long_kernel, dim3(256), dim3(kSortThreads), 0, stream, c, b);
 }
 
+// Calls f with the sample format and shading mode as compile-time constants.
+template <class F> static void with_shade_mode(bool fp32, int mode, F &&f) {
+	auto pick = [&](auto fmt, auto kind) {
+		if(mode & kShadeNarrow)
+			f(fmt, std::integral_constant<int, decltype(kind)::value | kShadeNarrow>{});
+		else
+			f(fmt, kind);
+	};
+	const std::integral_constant<int, kShadeGeneral> general;
+	const std::integral_constant<int, kShadeTextured> textured;
+	if(fp32) {
+		if(shade_kind(mode) == kShadePlain)
+			pick(std::true_type{}, std::integral_constant<int, kShadePlain>{});
+		else if(is_textured(mode))
+			pick(std::true_type{}, textured);
+		else
+			pick(std::true_type{}, general);
+	} else if(is_flat(mode))
+		pick(std::false_type{}, std::integral_constant<int, kShadeFlat>{});
+	else if(is_textured(mode))
+		pick(std::false_type{}, textured);
+	else
+		pick(std::false_type{}, general);
+}
+
 template <bool FP32, int W, int MODE>
 static void launch_block_raster_apart(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
 	hipLaunchKernelGGL((block_raster_kernel<FP32, W, MODE>), dim3(c.bin_count * 16), dim3(64), 0, stream,
@@ -3219,7 +3378,7 @@ static void launch_block_raster_apart(const FrameConst &c, const FrameBufs &b, h
 // 365 us), as are textured ones, whose blocks differ most in length (768 bins, 261 -> 269 us).
 template <bool FP32, int MODE>
 static void launch_block_raster(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
-	if constexpr(MODE != kShadeTextured) {
+	if constexpr(!is_textured(MODE)) {
 		if(c.slice_words == 1 && c.bin_count <= kFusedRasterBins) {
 			hipLaunchKernelGGL((block_raster_fused_kernel<FP32, MODE>),
 							   dim3(c.bin_count * (16 + 16 / kBigWaves)), dim3(kBigWaves * 64), 0, stream,
@@ -3236,7 +3395,7 @@ static void launch_block_raster(const FrameConst &c, const FrameBufs &b, hipStre
 template <bool FP32, int MODE>
 static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 							hipEvent_t *ev) {
-	constexpr bool TEX = MODE == kShadeTextured;
+	constexpr bool TEX = is_textured(MODE);
 	launch_rowgen(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[0], stream);
@@ -3254,7 +3413,7 @@ static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t
 
 template <bool FP32, int W, int MODE>
 static void launch_raster_batch_t(const BatchPlan &p, hipStream_t stream) {
-	constexpr bool TEX = MODE == kShadeTextured;
+	constexpr bool TEX = is_textured(MODE);
 	hipLaunchKernelGGL(rowgen_low_kernel_batch, dim3(p.total[kBsRowgenLow]), dim3(kRowgenThreads), 0,
 					   stream, p.frames, p.stage_pre(kBsRowgenLow), p.num_frames);
 	hipLaunchKernelGGL(rowgen_high_kernel_batch, dim3(p.total[kBsRowgenHigh]), dim3(kRowgenThreads), 0,
@@ -3278,17 +3437,9 @@ static void launch_raster_batch_t(const BatchPlan &p, hipStream_t stream) {
 // shading mode.
 template <int W>
 static void launch_raster_batch_w(const BatchPlan &p, hipStream_t stream) {
-	if(p.fp32)
-		p.mode == kShadeTextured ? launch_raster_batch_t<true, W, kShadeTextured>(p, stream)
-								 : launch_raster_batch_t<true, W, kShadeGeneral>(p, stream);
-	else if(p.mode == kShadeTextured)
-		launch_raster_batch_t<false, W, kShadeTextured>(p, stream);
-	else if(p.mode == kShadeFlat)
-		launch_raster_batch_t<false, W, kShadeFlat>(p, stream);
-	else if(p.mode == kShadeFlatNarrow)
-		launch_raster_batch_t<false, W, kShadeFlatNarrow>(p, stream);
-	else
-		launch_raster_batch_t<false, W, kShadeGeneral>(p, stream);
+	with_shade_mode(p.fp32, p.mode, [&](auto fp32, auto mode) {
+		launch_raster_batch_t<decltype(fp32)::value, W, decltype(mode)::value>(p, stream);
+	});
 }
 
 hipError_t launch_raster_batch(const BatchPlan &p, hipStream_t stream) {
@@ -3305,19 +3456,9 @@ hipError_t launch_raster(const FrameConst &c, const FrameBufs &b, hipStream_t st
 						 hipEvent_t *events) {
 	// frames with albedo textures take kernels built with the texture path (the others carry
 	// none of its code or registers); flat-colour frames take the colour-plane records
-	const bool fp32 = (c.opts & LUCID_OPT_FP32_SAMPLES) != 0;
-	const int mode = frame_shade_mode(c);
-	if(fp32)
-		mode == kShadeTextured ? launch_raster_t<true, kShadeTextured>(c, b, stream, events)
-							   : launch_raster_t<true, kShadeGeneral>(c, b, stream, events);
-	else if(mode == kShadeTextured)
-		launch_raster_t<false, kShadeTextured>(c, b, stream, events);
-	else if(mode == kShadeFlat)
-		launch_raster_t<false, kShadeFlat>(c, b, stream, events);
-	else if(mode == kShadeFlatNarrow)
-		launch_raster_t<false, kShadeFlatNarrow>(c, b, stream, events);
-	else
-		launch_raster_t<false, kShadeGeneral>(c, b, stream, events);
+	with_shade_mode((c.opts & LUCID_OPT_FP32_SAMPLES) != 0, frame_shade_mode(c), [&](auto fp32, auto mode) {
+		launch_raster_t<decltype(fp32)::value, decltype(mode)::value>(c, b, stream, events);
+	});
 	return hipGetLastError();
 }
 
@@ -3347,6 +3488,19 @@ __global__ __launch_bounds__(64) void record_gate_kernel(FrameBufs b, BwdBufs g)
 		b.ctrl[kCtrlRecorded] = (!(b.ctrl[kCtrlOverflow] & kOvfBinLists) && bwd_fits(b, g)) ? 1u : 0u;
 }
 
+template <bool RECORD>
+static void launch_pass_a(const FrameConst &c, const FrameBufs &b, const BwdBufs &g, hipStream_t stream) {
+	auto go = [&](auto kernel) {
+		hipLaunchKernelGGL(kernel, dim3(c.bin_count * 16), dim3(kBigWaves * 64), 0, stream, c, b, g);
+	};
+	if(c.window == 1) // narrow-window tuning: two slots
+		c.plain_colors ? go(bwd_pass_a_kernel<RECORD, 2, kShadePlain>)
+					   : go(bwd_pass_a_kernel<RECORD, 2, kShadeGeneral>);
+	else
+		c.plain_colors ? go(bwd_pass_a_kernel<RECORD, kWindow, kShadePlain>)
+					   : go(bwd_pass_a_kernel<RECORD, kWindow, kShadeGeneral>);
+}
+
 // Forward frame that also records pass A (fp32 samples): the raster stage of launch_raster
 // with the gradient row scan, the gate and the recording pass before the block kernels
 // (which then render only what the recording pass does not).
@@ -3360,13 +3514,11 @@ hipError_t launch_raster_recording(const FrameConst &c, const FrameBufs &b, cons
 	hipLaunchKernelGGL(record_gate_kernel, dim3(1), dim3(64), 0, stream, b, g);
 	if(ev)
 		(void)hipEventRecord(ev[1], stream);
-	if(c.window == 1)
-		hipLaunchKernelGGL((bwd_pass_a_kernel<true, 2>), dim3(c.bin_count * 16), dim3(kBigWaves * 64),
-						   0, stream, c, b, g);
-	else
-		hipLaunchKernelGGL((bwd_pass_a_kernel<true, kWindow>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b, g);
-	launch_block_raster<true, kShadeGeneral>(c, b, stream);
+	launch_pass_a<true>(c, b, g, stream);
+	with_shade_mode(true, frame_shade_mode(c), [&](auto, auto mode) {
+		if constexpr(!is_textured(decltype(mode)::value) && !is_flat(decltype(mode)::value))
+			launch_block_raster<true, decltype(mode)::value>(c, b, stream);
+	});
 	if(ev)
 		(void)hipEventRecord(ev[2], stream);
 	hipLaunchKernelGGL((fallback_kernel<true, false>), dim3(1024), dim3(kFallbackThreads), 0, stream,
@@ -3417,12 +3569,7 @@ hipError_t launch_backward_reuse(const FrameConst &c, const FrameBufs &b, const 
 // rows follow the block rows). After these every row's triangle is known.
 hipError_t launch_backward_order(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								 hipStream_t stream) {
-	if(c.window == 1) // narrow-window tuning: two slots
-		hipLaunchKernelGGL((bwd_pass_a_kernel<false, 2>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b, g);
-	else
-		hipLaunchKernelGGL((bwd_pass_a_kernel<false, kWindow>), dim3(c.bin_count * 16),
-						   dim3(kBigWaves * 64), 0, stream, c, b, g);
+	launch_pass_a<false>(c, b, g, stream);
 	hipLaunchKernelGGL(bwd_fallback_kernel, dim3(1024), dim3(kFallbackThreads), 0, stream, c, b, g);
 	return hipGetLastError();
 }
@@ -3430,8 +3577,12 @@ hipError_t launch_backward_order(const FrameConst &c, const FrameBufs &b, const 
 // Backward, third part: the block gradient rows (pass B replays the recorded order).
 hipError_t launch_backward_rows(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								hipStream_t stream) {
-	hipLaunchKernelGGL(bwd_pass_b_kernel, dim3(c.bin_count * 16 * kBigWaves), dim3(64), 0, stream, c,
-					   b, g);
+	if(c.plain_colors)
+		hipLaunchKernelGGL(bwd_pass_b_kernel<kShadePlain>, dim3(c.bin_count * 16 * kBigWaves), dim3(64), 0,
+						   stream, c, b, g);
+	else
+		hipLaunchKernelGGL(bwd_pass_b_kernel<kShadeGeneral>, dim3(c.bin_count * 16 * kBigWaves), dim3(64), 0,
+						   stream, c, b, g);
 	return hipGetLastError();
 }
 

@@ -12,6 +12,7 @@
 namespace lucid {
 
 constexpr int kBinThreads = 512;
+constexpr int kMaxBinRows = 2048 / kBinSize; // the renderer's largest height
 constexpr int kBinPrefetch = 8; // quad AABBs a thread loads before it counts or places them
 
 // loadScanlineParamsBin + scanlineStep (scanline.glsl:28-52, bin_counter.glsl:53-62)
@@ -96,6 +97,68 @@ __device__ __forceinline__ uint32_t large_at(const FrameBufs &b, const Slice &s,
 	return b.large_list[(size_t)k * s.lcap + (i - base)];
 }
 
+// Large triangle i of a work-group's slice (two per quad), with its scan at the first bin row.
+struct LargeTri {
+	bool culled;
+	uint32_t t;
+	int bsx, bex;
+	BinScan s;
+};
+__device__ __forceinline__ LargeTri load_large(const FrameBufs &b, const Slice &sl, uint32_t i) {
+	LargeTri lt;
+	const uint32_t q = large_at(b, sl, i >> 1), s = i & 1u, a = b.quad_aabb[q];
+	lt.culled = (a >> (30 + s)) & 1u;
+	lt.t = 2 * q + s;
+	lt.bsx = (int)(a & 0x7fu), lt.bex = (int)((a >> 14) & 0x7fu);
+	if(!lt.culled)
+		bin_scan_init(lt.s, b.tri_scan[2 * (size_t)tri_rec(b, lt.t)], b.tri_scan[2 * (size_t)tri_rec(b, lt.t) + 1]);
+	return lt;
+}
+// The bins [bmin, bmax] that the triangle covers in bin row `by` (an empty span outside its rows);
+// the scan advances row by row, as it does for all of them.
+__device__ __forceinline__ void row_span(const LargeTri &lt, int by, int &bmin, int &bmax) {
+	BinScan s = lt.s;
+	bmin = 1, bmax = 0;
+	if(by > s.max_by)
+		return;
+	for(int y = s.min_by; y <= by; y++)
+		bin_scan_step(s, bmin, bmax);
+	bmin = max(bmin, lt.bsx), bmax = min(bmax, lt.bex);
+}
+// A slice of few large triangles (scenes of a few screen-filling planes) takes a wave per triangle,
+// a lane per bin row; more of them take a thread each, which is better for the small spans of many.
+// 96 planes over 768 bins, a thread per triangle against a wave: bin_dispatch 27 -> 8 us, bin_count
+// 8.5 -> 6 (the thread walked 24 rows of up to 32 atomics in turn).
+constexpr uint32_t kFewLarge = 8 * (kBinThreads / 64);
+__device__ __forceinline__ bool few_large(const Slice &sl) { return (sl.l1 - sl.l0) * 2 <= kFewLarge; }
+// visit(triangle, bin row, first bin, last bin) for every bin row of the slice's large triangles.
+template <class F>
+__device__ __forceinline__ void large_rows(const FrameConst &c, const FrameBufs &b, const Slice &sl, F &&visit) {
+	if(few_large(sl)) {
+		static_assert(kMaxBinRows <= 64, "a lane per bin row");
+		for(uint32_t i = sl.l0 * 2 + (threadIdx.x >> 6); i < sl.l1 * 2; i += kBinThreads / 64) {
+			const LargeTri lt = load_large(b, sl, i);
+			const int by = lt.culled ? 0 : lt.s.min_by + lane_id();
+			if(lt.culled || by > lt.s.max_by)
+				continue;
+			int bmin, bmax;
+			row_span(lt, by, bmin, bmax);
+			visit(lt.t, by, bmin, bmax);
+		}
+		return;
+	}
+	for(uint32_t i = sl.l0 * 2 + threadIdx.x; i < sl.l1 * 2; i += kBinThreads) {
+		LargeTri lt = load_large(b, sl, i);
+		if(lt.culled)
+			continue;
+		for(int by = lt.s.min_by; by <= lt.s.max_by; by++) {
+			int bmin, bmax;
+			bin_scan_step(lt.s, bmin, bmax);
+			visit(lt.t, by, max(bmin, lt.bsx), min(bmax, lt.bex));
+		}
+	}
+}
+
 // bin_counter.glsl: per-work-group histograms of small quads and large tris.
 __device__ __forceinline__ void bin_count_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
 	extern __shared__ uint32_t s_hist[]; // [2][bin_count]
@@ -126,26 +189,13 @@ __device__ __forceinline__ void bin_count_kernel_body(const FrameConst &c, const
 		}
 	}
 	// large tris: per bin row +1/-1 marks (bin_counter.glsl:112-134)
-	for(uint32_t i = sl.l0 * 2 + threadIdx.x; i < sl.l1 * 2; i += kBinThreads) {
-		uint32_t q = large_at(b, sl, i >> 1), s = i & 1u;
-		uint32_t a = b.quad_aabb[q];
-		if((a >> (30 + s)) & 1u)
-			continue;
-		uint32_t t = 2 * q + s;
-		int bsx = (int)(a & 0x7fu), bex = (int)((a >> 14) & 0x7fu);
-		BinScan bs;
-		bin_scan_init(bs, b.tri_scan[2 * (size_t)tri_rec(b, t)], b.tri_scan[2 * (size_t)tri_rec(b, t) + 1]);
-		for(int by = bs.min_by; by <= bs.max_by; by++) {
-			int bmin, bmax;
-			bin_scan_step(bs, bmin, bmax);
-			bmin = max(bmin, bsx), bmax = min(bmax, bex);
-			if(bmax >= bmin) {
-				atomicAdd(&ht[by * NBX + bmin], 1u);
-				if(bmax + 1 < NBX)
-					atomicAdd(&ht[by * NBX + bmax + 1], 0xffffffffu);
-			}
+	large_rows(c, b, sl, [&](uint32_t, int by, int bmin, int bmax) {
+		if(bmax >= bmin) {
+			atomicAdd(&ht[by * NBX + bmin], 1u);
+			if(bmax + 1 < NBX)
+				atomicAdd(&ht[by * NBX + bmax + 1], 0xffffffffu);
 		}
-	}
+	});
 	__syncthreads();
 	// prefix over each bin row turns the marks into counts
 	int wave = threadIdx.x >> 6, nwaves = kBinThreads / 64;
@@ -391,21 +441,25 @@ __device__ __forceinline__ void bin_dispatch_kernel_body(const FrameConst &c, co
 					b.bin_quads[atomicAdd(&pq[by * NBX + bx], 1u)] = entry;
 		}
 	}
-	for(uint32_t i = sl.l0 * 2 + threadIdx.x; i < sl.l1 * 2; i += kBinThreads) {
-		uint32_t q = large_at(b, sl, i >> 1), s = i & 1u;
-		uint32_t a = b.quad_aabb[q];
-		if((a >> (30 + s)) & 1u)
-			continue;
-		uint32_t t = 2 * q + s;
-		int bsx = (int)(a & 0x7fu), bex = (int)((a >> 14) & 0x7fu);
-		BinScan bs;
-		bin_scan_init(bs, b.tri_scan[2 * (size_t)tri_rec(b, t)], b.tri_scan[2 * (size_t)tri_rec(b, t) + 1]);
-		for(int by = bs.min_by; by <= bs.max_by; by++) {
-			int bmin, bmax;
-			bin_scan_step(bs, bmin, bmax);
-			bmin = max(bmin, bsx), bmax = min(bmax, bex);
+	if(!few_large(sl)) {
+		large_rows(c, b, sl, [&](uint32_t t, int by, int bmin, int bmax) {
 			for(int bx = bmin; bx <= bmax; bx++)
 				b.bin_tris[atomicAdd(&pt[by * NBX + bx], 1u)] = t;
+		});
+		return;
+	}
+	// a wave per triangle: its bin rows' spans from the lanes, then a lane per bin of a row
+	const int lane = lane_id();
+	for(uint32_t i = sl.l0 * 2 + (threadIdx.x >> 6); i < sl.l1 * 2; i += kBinThreads / 64) {
+		const LargeTri lt = load_large(b, sl, i);
+		if(lt.culled)
+			continue;
+		int bmin, bmax;
+		row_span(lt, lt.s.min_by + lane, bmin, bmax);
+		for(int r = 0; r <= lt.s.max_by - lt.s.min_by; r++) {
+			const int x0 = (int)wave_read((uint32_t)bmin, r), x1 = (int)wave_read((uint32_t)bmax, r);
+			for(int bx = x0 + lane; bx <= x1; bx += 64)
+				b.bin_tris[atomicAdd(&pt[(lt.s.min_by + r) * NBX + bx], 1u)] = lt.t;
 		}
 	}
 }

@@ -109,10 +109,18 @@ __global__ void tri_group_sum_kernel(FrameConst c, const uint32_t *ctrl, const u
 // (0, 1 + s, 2 + s), quads addressed through the instances (quad_setup.glsl:136-160).
 // Writes the corner -> vertex map into `vkeys` and sets *changed when it differs from what
 // `vkeys` held (the vertex grouping of the previous backward pass is then stale).
+// Also clears what the later kernels add to: the rows per triangle (ntri + 1 counts) and, if there
+// is such an output, the vertex gradients (nzero words).
 __global__ void corner_check_kernel(FrameConst c, FrameBufs b, uint32_t ntri, uint32_t *vkeys,
-									uint32_t *changed) {
+									uint32_t *changed, uint32_t *counts, float *zero, size_t nzero) {
 	const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
 	bool diff = false;
+	if(t < ntri)
+		counts[t] = 0u;
+	if(t == 0)
+		counts[ntri] = 0u;
+	for(size_t i = t; i < nzero; i += (size_t)gridDim.x * blockDim.x)
+		zero[i] = 0.0f;
 	if(t < ntri) {
 		const uint32_t q = t >> 1, s = t & 1u;
 		int lo = 0, hi = c.num_instances - 1;
@@ -162,12 +170,6 @@ __global__ void vertex_segment_sum_kernel(const uint32_t *keys, const uint32_t *
 		grad_colors[(size_t)k * 3 + 1] = sum[1];
 		grad_colors[(size_t)k * 3 + 2] = sum[2];
 	}
-}
-
-__global__ void alpha_grad_kernel(const float *tri_grad, uint32_t ntri, float *grad_alpha) {
-	const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-	if(t < ntri)
-		grad_alpha[t] = tri_grad[(size_t)t * kGradWords + 9];
 }
 
 // Exclusive prefix sum of u32 counts in three launches: tile totals, their exclusive scan
@@ -278,6 +280,12 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t
 	}
 }
 
+// The control words to pinned host memory (read after the stream has been waited for).
+__global__ __launch_bounds__(64) void status_kernel(const uint32_t *ctrl, uint32_t *host) {
+	if(threadIdx.x < (uint32_t)kCtrlWords)
+		__hip_atomic_store(&host[threadIdx.x], ctrl[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 inline uint32_t scan_tiles(size_t n) { return (uint32_t)((n + kScanTile - 1) / kScanTile); }
 
 // out[i] = in[0] + ... + in[i - 1] for i < n; `temp` holds scan_tiles(n) words.
@@ -316,23 +324,20 @@ size_t reduce_temp_bytes(uint32_t npairs, uint32_t nscan) {
 
 // Corner -> vertex map of the frame's triangles into vkeys (3 per triangle); sets *changed
 // when it differs from the map already there.
-hipError_t reduce_check_corners(const FrameConst &c, const FrameBufs &b, uint32_t ntri,
-								uint32_t *vkeys, uint32_t *changed, hipStream_t stream) {
-	if(ntri)
-		hipLaunchKernelGGL(corner_check_kernel, grid_for(ntri), dim3(256), 0, stream, c, b, ntri,
-						   vkeys, changed);
+// The counts and the vertex gradients (if any) start at zero.
+hipError_t reduce_begin(const FrameConst &c, const FrameBufs &b, const ReduceBufs &r, uint32_t ntri,
+						uint32_t nverts, uint32_t *changed, float *grad_colors, hipStream_t stream) {
+	hipLaunchKernelGGL(corner_check_kernel, grid_for(std::max<size_t>(ntri, 1)), dim3(256), 0, stream, c, b,
+					   ntri, r.vkeys, changed, r.counts, grad_colors, grad_colors ? (size_t)nverts * 3 : 0);
 	return hipGetLastError();
 }
 
-hipError_t reduce_vertices(const ReduceBufs &r, uint32_t ntri, uint32_t nverts, bool regroup,
-						   float *grad_colors, float *grad_alpha, hipStream_t stream);
-
+static hipError_t sum_vertices(const ReduceBufs &r, uint32_t ntri, uint32_t nverts, bool regroup,
+							   float *grad_colors, hipStream_t stream);
 // Groups the gradient rows by triangle (counts, offsets, grouped row indices); the row
 // count is read on the device, `rows_cap` bounds the grid.
 hipError_t reduce_group_rows(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 							 const ReduceBufs &r, uint32_t ntri, hipStream_t stream) {
-	hipLaunchKernelGGL(zero_kernel, grid_for((size_t)ntri + 1), dim3(256), 0, stream, r.counts,
-					   (size_t)ntri + 1);
 	if(g.rows_cap)
 		hipLaunchKernelGGL(row_hist_kernel, grid_for(g.rows_cap), dim3(256), 0, stream, b.ctrl, g,
 						   ntri, r.counts);
@@ -352,38 +357,44 @@ hipError_t reduce_group_rows(const FrameConst &c, const FrameBufs &b, const BwdB
 // r.vcorners) depend only on the mesh: they are regrouped only when `regroup` is set.
 hipError_t reduce_sum(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 					  const ReduceBufs &r, uint32_t ntri, uint32_t nverts, bool regroup,
-					  float *grad_colors, float *grad_alpha, hipStream_t stream) {
+					  float *grad_colors, float *grad_alpha, uint32_t *host_status, hipStream_t stream) {
 	if(ntri)
 		hipLaunchKernelGGL(tri_group_sum_kernel, grid_for(ntri), dim3(256), 0, stream, c, b.ctrl,
 						   r.offsets, ntri, r.grouped, g.rows, r.tri_grad, grad_alpha);
-	// (the alpha gradients are written above)
-	return reduce_vertices(r, ntri, nverts, regroup, grad_colors, nullptr, stream);
+	const hipError_t e = sum_vertices(r, ntri, nverts, regroup, grad_colors, stream);
+	if(e != hipSuccess)
+		return e;
+	hipLaunchKernelGGL(status_kernel, dim3(1), dim3(64), 0, stream, b.ctrl, host_status);
+	return hipGetLastError();
 }
 
-// Per-vertex colour sums (and the alpha copy) from r.tri_grad.
-hipError_t reduce_vertices(const ReduceBufs &r, uint32_t ntri, uint32_t nverts, bool regroup,
-						   float *grad_colors, float *grad_alpha, hipStream_t stream) {
-	if(grad_colors) {
+// Per-vertex colour sums from r.tri_grad, added to the cleared grad_colors.
+static hipError_t sum_vertices(const ReduceBufs &r, uint32_t ntri, uint32_t nverts, bool regroup,
+							   float *grad_colors, hipStream_t stream) {
+	const uint32_t np = 3 * ntri;
+	if(!grad_colors || !np)
+		return hipGetLastError();
+	if(regroup) {
+		hipLaunchKernelGGL(iota_kernel, grid_for(np), dim3(256), 0, stream, r.viota, np);
+		size_t bytes = r.temp_bytes;
+		hipError_t e = rocprim::radix_sort_pairs(
+			r.temp, bytes, (const uint32_t *)r.vkeys, r.vsorted, (const uint32_t *)r.viota,
+			r.vcorners, np, 0, key_bits(nverts), stream);
+		if(e != hipSuccess)
+			return e;
+	}
+	hipLaunchKernelGGL(vertex_segment_sum_kernel, grid_for(np), dim3(256), 0, stream, r.vsorted, r.vcorners,
+					   np, r.tri_grad, nverts, grad_colors);
+	return hipGetLastError();
+}
+
+// The vertex sums again, with the corners grouped anew.
+hipError_t reduce_vertices(const ReduceBufs &r, uint32_t ntri, uint32_t nverts, float *grad_colors,
+						   hipStream_t stream) {
+	if(nverts)
 		hipLaunchKernelGGL(zero_kernel, grid_for((size_t)nverts * 3), dim3(256), 0, stream,
 						   (uint32_t *)grad_colors, (size_t)nverts * 3);
-		const uint32_t np = 3 * ntri;
-		if(regroup && np) {
-			hipLaunchKernelGGL(iota_kernel, grid_for(np), dim3(256), 0, stream, r.viota, np);
-			size_t bytes = r.temp_bytes;
-			hipError_t e = rocprim::radix_sort_pairs(
-				r.temp, bytes, (const uint32_t *)r.vkeys, r.vsorted, (const uint32_t *)r.viota,
-				r.vcorners, np, 0, key_bits(nverts), stream);
-			if(e != hipSuccess)
-				return e;
-		}
-		if(np)
-			hipLaunchKernelGGL(vertex_segment_sum_kernel, grid_for(np), dim3(256), 0, stream,
-							   r.vsorted, r.vcorners, np, r.tri_grad, nverts, grad_colors);
-	}
-	if(grad_alpha && ntri)
-		hipLaunchKernelGGL(alpha_grad_kernel, grid_for(ntri), dim3(256), 0, stream, r.tri_grad,
-						   ntri, grad_alpha);
-	return hipGetLastError();
+	return sum_vertices(r, ntri, nverts, true, grad_colors, stream);
 }
 
 } // namespace lucid

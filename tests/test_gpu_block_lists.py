@@ -101,3 +101,31 @@ def test_many_bins(oracle_mod, w, h):
     sc = _stacks(w, h, "mixed", counts, seed=w)
     r, gpu, ref = _render_both(sc, oracle_mod)
     _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("make", [
+    lambda: scenes.tilted_planes(2500, 2048, 3, seed=1),      # 79 x 64 bins, a wave per triangle
+    lambda: scenes.tilted_planes(2560, 40, 5, seed=2),
+    lambda: scenes.tilted_planes(40, 2000, 5, seed=3),
+    lambda: scenes.config0(seed=8, num_tris=300, width=1000, height=700),
+    lambda: scenes.config0(seed=9, num_tris=8192, width=700, height=500),
+    lambda: scenes.config0(seed=9, num_tris=30000, width=500, height=300),  # a thread per triangle
+])
+def test_large_triangles(oracle_mod, make):
+    """Triangles over more than four bins, a few and many per work-group of the binning kernels,
+    in frames of the most rows and columns of bins."""
+    sc = make()
+    r, gpu, ref = _render_both(sc, oracle_mod)
+    _check(sc, gpu, ref, oracle_mod)
+
+
+@pytest.mark.parametrize("opts", [0, _lib.OPT_FP32_SAMPLES])
+@pytest.mark.parametrize("n", [2, 33, 63, 64, 65, 130])
+def test_exact_pixel_lengths(oracle_mod, n, opts):
+    """Pixels of n intersecting planes, around the length up to which their keys are sorted in
+    registers (64)."""
+    sc = scenes.tilted_planes(90, 60, n, seed=n)
+    r, gpu, ref = _render_both(sc, oracle_mod, opts=opts)
+    if n >= 63:
+        assert gpu["stats"]["fallback_pixels"] > 0
+    _check(sc, gpu, ref, oracle_mod)

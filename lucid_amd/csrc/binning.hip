@@ -129,7 +129,10 @@ __device__ __forceinline__ void row_span(const LargeTri &lt, int by, int &bmin, 
 // a lane per bin row; more of them take a thread each, which is better for the small spans of many.
 // 96 planes over 768 bins, a thread per triangle against a wave: bin_dispatch 27 -> 8 us, bin_count
 // 8.5 -> 6 (the thread walked 24 rows of up to 32 atomics in turn).
-constexpr uint32_t kFewLarge = 8 * (kBinThreads / 64);
+// Only one triangle per wave: each is a chain of three dependent loads, which a thread per triangle
+// takes once for all of them (the 32-frame batch with up to 8 per wave: bin_count 62 -> 77 us,
+// bin_dispatch 84 -> 98).
+constexpr uint32_t kFewLarge = kBinThreads / 64;
 __device__ __forceinline__ bool few_large(const Slice &sl) { return (sl.l1 - sl.l0) * 2 <= kFewLarge; }
 // visit(triangle, bin row, first bin, last bin) for every bin row of the slice's large triangles.
 template <class F>
@@ -384,7 +387,7 @@ __device__ __forceinline__ void bin_wg_scan_kernel_body(const FrameConst &c, con
 			agent_store(&counts[(k == 0 ? LUCID_COUNTS_QUAD_COUNTS : LUCID_COUNTS_TRI_COUNTS) * NB + bin], run);
 		}
 	}
-	const bool last = last_work_group(&b.ctrl[kCtrlScanDone], 1u, wg.count);
+	const bool last = last_work_group(b.ctrl, kDoneScan, wg.id, wg.count);
 	uint32_t run = s_part[part][col_l];
 #pragma unroll
 	for(int j = 0; j < kMaxRows; j++) {

@@ -108,6 +108,8 @@ def test_many_bins(oracle_mod, w, h):
     lambda: scenes.tilted_planes(2560, 40, 5, seed=2),
     lambda: scenes.tilted_planes(40, 2000, 5, seed=3),
     lambda: scenes.config0(seed=8, num_tris=300, width=1000, height=700),
+    lambda: scenes.config0(seed=9, num_tris=1024, width=700, height=500),
+    lambda: scenes.config0(seed=9, num_tris=1025, width=700, height=500),  # two quads for some
     lambda: scenes.config0(seed=9, num_tris=8192, width=700, height=500),
     lambda: scenes.config0(seed=9, num_tris=30000, width=500, height=300),  # a thread per triangle
 ])

@@ -47,8 +47,7 @@ enum CtrlWord : int {
 	kCtrlWords = 16,
 	// device-only words (not copied to the host) up to kStatStripeBase:
 	kCtrlBigSorts = 16, // blocks queued in big_queue for the long-list sort pass
-	kCtrlScanDone = 17, // work-groups of bin_wg_scan that have stored their bin counts
-	kCtrlFixedHigh = 18, // high bins before row generation adds the promoted ones
+	kCtrlFixedHigh = 17, // high bins before row generation adds the promoted ones
 };
 
 // Frame statistics summed per block (fragments, list entries) go to kStatStripes counters
@@ -75,7 +74,15 @@ __device__ __forceinline__ uint32_t *sort_cursor(uint32_t *ctrl, uint32_t stripe
 constexpr int kLargeStripes = 16;
 constexpr int kSetupThreads = 256;
 constexpr int kLargeCursorBase = kSortCursorBase + kSortStripes * kStatStride;
-constexpr int kCtrlAllocWords = kLargeCursorBase + kLargeStripes * kStatStride;
+// Counters of the work-groups that are done (last_work_group), of the bin scan and of the exact
+// fallback: kDoneStripes words and one for the stripes that are complete, a line each.
+constexpr int kDoneStripes = 16;
+enum DoneCounter : int { kDoneScan = 0, kDoneFallback = 1, kDoneCounters = 2 };
+constexpr int kDoneBase = kLargeCursorBase + kLargeStripes * kStatStride;
+constexpr int kCtrlAllocWords = kDoneBase + kDoneCounters * (kDoneStripes + 1) * kStatStride;
+__device__ __forceinline__ uint32_t *done_counter(uint32_t *ctrl, int counter, uint32_t word) {
+	return ctrl + kDoneBase + (counter * (kDoneStripes + 1) + (int)word) * kStatStride;
+}
 __device__ __forceinline__ uint32_t *large_cursor(uint32_t *ctrl, uint32_t stripe) {
 	return ctrl + kLargeCursorBase + (int)stripe * kStatStride;
 }
@@ -540,17 +547,26 @@ __device__ __forceinline__ uint32_t agent_load(const uint32_t *p) {
 __device__ __forceinline__ void agent_store(uint32_t *p, uint32_t v) {
 	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// Adds `mine` to `done` (a word that the frame cleared); true in every thread of the work-group
-// whose part completes the `total`. That work-group may agent_load what the others agent_store'd or changed by
-// atomics before: these are complete once each wave has waited for its memory operations, so no
-// cache has to be written back (a release fence of whole L2s, 512 waves of them, took 60 us).
-// Called by whole work-groups.
-__device__ __forceinline__ bool last_work_group(uint32_t *done, uint32_t mine, uint32_t total) {
+// True in every thread of the last of `count` work-groups to get here, work-group `wg` of them
+// (`counter`: which set of the frame's cleared done counters). That work-group may agent_load what
+// the others agent_store'd or changed by atomics before: these are complete once each wave has
+// waited for its memory operations, so no cache has to be written back (a release fence of whole
+// L2s, 512 waves of them, took 60 us). Work-groups count in kDoneStripes words, whose last ones
+// count in another: atomics on one word take turns (2048 of them: 35 us). Called by whole
+// work-groups.
+__device__ __forceinline__ bool last_work_group(uint32_t *ctrl, int counter, uint32_t wg, uint32_t count) {
 	__shared__ uint32_t s_last;
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 	__syncthreads();
-	if(threadIdx.x == 0)
-		s_last = __hip_atomic_fetch_add(done, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine == total;
+	if(threadIdx.x == 0) {
+		const uint32_t stripe = wg % kDoneStripes, stripes = min(count, (uint32_t)kDoneStripes);
+		const uint32_t members = (count - stripe + kDoneStripes - 1) / kDoneStripes;
+		auto ended = [&](uint32_t word, uint32_t n) {
+			return __hip_atomic_fetch_add(done_counter(ctrl, counter, word), 1u, __ATOMIC_RELAXED,
+										  __HIP_MEMORY_SCOPE_AGENT) + 1u == n;
+		};
+		s_last = ended(stripe, members) && ended(kDoneStripes, stripes);
+	}
 	__syncthreads();
 	return s_last != 0;
 }

@@ -728,7 +728,6 @@ template <int E> __device__ __forceinline__ void bitonic_regs(uint32_t (&v)[E], 
 	bitonic_merge<E, 32 * E>(v, flip);
 }
 
-// Ascending bitonic sort of P (power of two) keys in LDS by one wave.
 // Sorts the wave's 64 keys, one per lane, ascending.
 template <int K, int J> __device__ __forceinline__ void bitonic64_steps(uint64_t &v) {
 	const uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
@@ -752,6 +751,7 @@ template <int K = 2> __device__ __forceinline__ void bitonic64_wave(uint64_t &v)
 		bitonic64_wave<K * 2>(v);
 }
 
+// Ascending bitonic sort of P (power of two) keys in LDS by one wave.
 __device__ void bitonic_lds_wave(uint64_t *key, uint32_t P) {
 	const int lane = lane_id();
 	for(uint32_t k = 2; k <= P; k <<= 1) {
@@ -921,6 +921,14 @@ __device__ __forceinline__ uint32_t bin_tri_at(const FrameBufs &b, uint32_t i, u
 		return 2 * (e & 0x0fffffffu) + s;
 	}
 	return b.bin_tris[to + (i - 2 * qc)];
+}
+
+// Keeps loads that a return could come before where they are written, in flight together: a block's
+// chain of early exits otherwise takes a memory latency for each.
+__device__ __forceinline__ void loaded_here() {}
+template <class T, class... R> __device__ __forceinline__ void loaded_here(T v, R... rest) {
+	asm volatile("" ::"v"(v));
+	loaded_here(rest...);
 }
 
 struct BinInfo {
@@ -1382,6 +1390,10 @@ __device__ __forceinline__ uint32_t sorted_mask_offset(uint32_t m) {
 // pre-sorts long lists. A long list is sorted once by centroid depth (LDS bitonic by the
 // whole work-group) and split into `parts` pixel-row groups, each a compacted list of the
 // entries that cover it, so that several waves can rasterise a dense block.
+// A work-group is a chain of memory and LDS latencies (VALU busy 0.4), so the loads that decide its
+// early exits are made together, the pool is asked for while the entries load, and a list of up to
+// 256 keys is sorted by all four waves: 32-frame batch 506 -> 471 us, 5.2 M mesh triangles 192 ->
+// 148, 1 M soup triangles 89 -> 80.
 // Two passes share the body: CAP = kMidSortCap does the slot bookkeeping of every block,
 // sorts the lists of up to kMidSortCap entries (8 KB of keys in LDS, so twice as many
 // work-groups per CU as with the full capacity) and queues the longer ones in big_queue;
@@ -1391,20 +1403,20 @@ constexpr uint32_t kMidSortCap = 2048;
 
 template <uint32_t CAP>
 __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, const FrameBufs &b, WgPos wg) {
-	if(b.ctrl[kCtrlOverflow] & (kOvfBinLists | kOvfLists))
-		return;
 	const lucid_info *info = (const lucid_info *)b.info;
 	const uint32_t hslot = wg.id >> 4;
 	const int blk = wg.id & 15, by = blk >> 2, bx = blk & 3;
-	if(hslot >= (uint32_t)info->bin_level_counts[LUCID_BIN_LEVEL_HIGH])
-		return;
 	const uint32_t *counts = b.info + LUCID_INFO_U32_SIZE;
-	const int bin = (int)counts[LUCID_COUNTS_HIGH_BINS * c.bin_count + hslot];
+	const uint32_t overflow = b.ctrl[kCtrlOverflow], nhigh = (uint32_t)info->bin_level_counts[LUCID_BIN_LEVEL_HIGH];
+	const int bin = (int)counts[LUCID_COUNTS_HIGH_BINS * c.bin_count + hslot]; // (hslot < bin_count)
+	loaded_here(overflow, nhigh, bin);
+	if((overflow & (kOvfBinLists | kOvfLists)) || hslot >= nhigh)
+		return;
 	const uint32_t slot = (uint32_t)bin * 16 + blk;
-	if(b.blk_flags[slot] & kSlotPromoted)
+	const uint32_t flags = b.blk_flags[slot], m = b.blk_count[slot], list0 = b.blk_slot[slot].x;
+	loaded_here(flags, m, list0);
+	if(flags & kSlotPromoted)
 		return; // allocation failed: the frame reports an overflow
-	const uint32_t m = b.blk_count[slot];
-	const uint32_t list0 = b.blk_slot[slot].x;
 	if(CAP == kMidSortCap && threadIdx.x == 0)
 		b.blk_slot[slot].y = m;
 	if(m <= c.presort_min) { // sorted in registers by the block rasteriser (<= kRegSortCap)
@@ -1450,11 +1462,34 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 	const bool unsorted = (c.opts & LUCID_OPT_UNSORTED) != 0; // the unsorted baseline
 	// the block's pool space (allocated first) for the sorted entries: header, triangle ids,
 	// masks
+	// (the answer is awaited after pass 1's loads are under way)
+	const uint32_t need = sorted_mask_offset(m) + 2 * m + 1; // + 1: even rounding of the base
+	const uint32_t stripe = slot % kSortStripes;
+	uint32_t off = 0;
+	if(threadIdx.x == 0)
+		off = atomicAdd(sort_cursor(b.ctrl, stripe), need);
+	// Keys are (depth rank << pb | list position). Pass 1 reads the entries once: depth keys
+	// (in s_key), sample counts and the block's key range.
+	uint32_t lo = ~0u, hi = 0u;
+	uint32_t mine = 0;
+#pragma unroll 2
+	for(uint32_t j = threadIdx.x; j < m; j += kSortThreads) {
+		const uint4 en = list[j];
+		const uint32_t smp = (uint32_t)__popc(en.z) + (uint32_t)__popc(en.w);
+		s_smp[j] = (uint8_t)smp;
+		mine += smp;
+		// the unsorted baseline: list order (rank 0, the position alone)
+		s_key[j] = unsorted ? j : en.y;
+		lo = min(lo, en.y);
+		hi = max(hi, en.y);
+	}
+	lo = wave_min_u32(lo);
+	hi = wave_max_u32(hi);
+	mine = wave_read(wave_inclusive_add(mine), 63);
+	if(lane_s == 0)
+		s_lo[wave_s] = lo, s_hi[wave_s] = hi, s_wsum[1][wave_s] = mine;
 	if(threadIdx.x == 0) {
-		const uint32_t need = sorted_mask_offset(m) + 2 * m + 1; // + 1: even rounding of the base
-		const uint32_t stripe = slot % kSortStripes;
 		const uint64_t region = (b.sorted_cap / kSortStripes) & ~1ull;
-		const uint32_t off = atomicAdd(sort_cursor(b.ctrl, stripe), need);
 		uint32_t base = 0xffffffffu;
 		if((uint64_t)off + need <= region) {
 			base = (uint32_t)(stripe * region + off);
@@ -1472,32 +1507,6 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 		return;
 	}
 	uint32_t *hdr = b.sorted_pool + s_base;
-	// Keys are (depth rank << pb | list position). Pass 1 reads the entries once: depth keys
-	// (in s_key), sample counts and the block's key range.
-	uint32_t lo = ~0u, hi = 0u;
-	uint32_t mine = 0;
-	for(uint32_t ch = wave_s; ch < nchunks; ch += kSortThreads / 64) {
-#pragma unroll
-		for(int e = 0; e < 4; e++) {
-			const uint32_t j = ch * 256 + e * 64 + lane_s;
-			if(j < m) {
-				const uint4 en = list[j];
-				const uint32_t smp = (uint32_t)__popc(en.z) + (uint32_t)__popc(en.w);
-				s_smp[j] = (uint8_t)smp;
-				mine += smp;
-				// the unsorted baseline: list order (rank 0, the position alone)
-				s_key[j] = unsorted ? j : en.y;
-				lo = min(lo, en.y);
-				hi = max(hi, en.y);
-			}
-		}
-	}
-	lo = wave_min_u32(lo);
-	hi = wave_max_u32(hi);
-	mine = wave_read(wave_inclusive_add(mine), 63);
-	if(lane_s == 0)
-		s_lo[wave_s] = lo, s_hi[wave_s] = hi, s_wsum[1][wave_s] = mine;
-	__syncthreads();
 	uint32_t tot = 0;
 #pragma unroll
 	for(int w = 0; w < kSortThreads / 64; w++)
@@ -1511,11 +1520,30 @@ __device__ __forceinline__ void high_finalize_kernel_body(const FrameConst &c, c
 			s_bound[w] = w == 0 ? 0u : m;
 	}
 	const DepthGrid grid(lo, hi, 32 - pb);
-	// Bitonic sort: levels up to 256 in registers (one 256-key chunk per wave at a time; each
-	// lane reads back only what it wrote in pass 1), then per level the strides >= 256 in LDS
-	// and the rest in registers. A real key never equals the padding ~0u: position P - 1
-	// exists only when nothing is padded.
-	for(uint32_t ch = wave_s; ch < nchunks && !unsorted; ch += kSortThreads / 64) {
+	// Bitonic sort. Up to 256 keys: one per thread, levels up to 64 within the waves, the two strides
+	// across them through LDS (a buffer each, so one barrier each). Longer lists: levels up to 256
+	// in registers (one 256-key chunk per wave at a time), then per level the strides >= 256 in LDS
+	// and the rest in registers. A real key never equals the padding ~0u: position P - 1 exists
+	// only when nothing is padded.
+	if(nchunks == 1 && !unsorted) {
+		static_assert(CAP >= 4 * kSortThreads, "the exchanges' buffers beside the keys");
+		const uint32_t j = threadIdx.x;
+		uint32_t v[1] = {j < m ? (grid.rank(s_key[j]) << pb) | j : ~0u};
+		bitonic_regs<1>(v, (j & 64u) ? ~0u : 0u);
+		auto exchange = [&](uint32_t *buf, uint32_t stride, uint32_t k) {
+			buf[j] = v[0];
+			__syncthreads();
+			const uint32_t o = buf[j ^ stride];
+			v[0] = ((j & k) == 0) == ((j & stride) == 0) ? min(v[0], o) : max(v[0], o);
+		};
+		exchange(s_key + kSortThreads, 64u, 128u);
+		bitonic_merge<1, 32>(v, (j & 128u) ? ~0u : 0u);
+		exchange(s_key + 2 * kSortThreads, 128u, 256u);
+		exchange(s_key + 3 * kSortThreads, 64u, 256u);
+		bitonic_merge<1, 32>(v, 0u);
+		s_key[j] = v[0];
+	}
+	for(uint32_t ch = wave_s; ch < nchunks && nchunks > 1 && !unsorted; ch += kSortThreads / 64) {
 		uint32_t v[4];
 #pragma unroll
 		for(int e = 0; e < 4; e++) {
@@ -2497,24 +2525,17 @@ __device__ __forceinline__ void fallback_kernel_body(const FrameConst &c, const 
 	const uint32_t w = wg.id * (kFallbackThreads / 64) + (threadIdx.x >> 6);
 	for(uint32_t qi = w; qi < nq; qi += waves)
 		fallback_pixel<FP32, TEX>(c, b, s_tex, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
-	// The pixels are counted once per work-group (an atomic each, on two words of the whole frame,
-	// took 130 of the kernel's 157 us for 17 k pixels of 32 fragments); the work-group that
-	// completes the count ends the frame. With an empty queue that is the first one.
-	constexpr uint32_t kItems = kFallbackThreads / 64;
-	if(nq ? wg.id * kItems >= nq : wg.id != 0)
+	// The work-group that empties the queue last ends the frame (with an empty queue, the first one).
+	// Nothing is counted per pixel: two atomics each, on words of the whole frame, took 130 of the
+	// kernel's 157 us for 17 k pixels of 32 fragments.
+	const uint32_t busy = min(wg.count, (nq + kFallbackThreads / 64 - 1) / (kFallbackThreads / 64));
+	if(nq ? wg.id >= busy || !last_work_group(b.ctrl, kDoneFallback, wg.id, busy) : wg.id != 0)
 		return;
-	if(nq) {
-		uint32_t mine = 0;
-		for(uint32_t k = 0; k < kItems; k++) {
-			const uint32_t q0 = wg.id * kItems + k;
-			mine += q0 < nq ? (nq - q0 + waves - 1) / waves : 0u;
-		}
-		if(!last_work_group(&b.ctrl[kCtrlFallbackPixels], mine, nq))
-			return;
+	if(nq && threadIdx.x == 0) {
+		agent_store(&b.ctrl[kCtrlFallbackPixels], nq);
 		// stats[2]: pixels resolved by the exact per-pixel sort (the reference counts the
 		// pixels its 3-deep window gets wrong there, shading.glsl:258-265)
-		if(threadIdx.x == 0)
-			((lucid_info *)b.info)->stats[2] = nq;
+		((lucid_info *)b.info)->stats[2] = nq;
 	}
 	// The control words go to pinned host memory, where the host reads them once the frame's
 	// event has completed (a copy command of 64 bytes: 4 us of the GPU, and its submission).

@@ -3153,7 +3153,10 @@ __device__ void enqueue_block_whole(const FrameConst &c, const FrameBufs &b, uin
 template <bool REUSE>
 __global__ __launch_bounds__(1024) void grad_row_scan_kernel(FrameConst c, FrameBufs b, BwdBufs g) {
 	const uint32_t n = (uint32_t)c.bin_count * 16;
-	__shared__ uint32_t s_wave[2][16];
+	// Four slots per thread and round, whose loads are in flight together: one work-group's chain of
+	// loads and barriers is all this kernel waits for (4096 blocks: 12 -> 9 us).
+	constexpr int kSlots = 4;
+	__shared__ uint32_t s_wave[2][kSlots * 16];
 	__shared__ uint32_t s_carry[2];
 	if constexpr(REUSE) {
 		if(threadIdx.x < (uint32_t)kCtrlWords)
@@ -3162,42 +3165,50 @@ __global__ __launch_bounds__(1024) void grad_row_scan_kernel(FrameConst c, Frame
 	if(threadIdx.x < 2)
 		s_carry[threadIdx.x] = 0;
 	__syncthreads();
-	const int wave = threadIdx.x >> 6;
-	for(uint32_t base = 0; base < n; base += 1024) {
-		const uint32_t slot = base + threadIdx.x;
-		uint32_t v[2] = {0u, 0u};
-		if(slot < n) {
-			const uint32_t flags = b.blk_flags[slot];
-			const uint32_t level = flags & kSlotLevelMask;
-			const uint32_t m = b.blk_slot[slot].y;
-			if(level != LUCID_BIN_LEVEL_EMPTY && !(flags & (kSlotWhole | kSlotPromoted)) && m) {
-				v[0] = m;
-				v[1] = (flags & kSlotPresorted) ? b.sorted_pool[b.blk_sorted[slot]] : 1u;
-			}
-			if(REUSE && (flags & kSlotWhole))
-				enqueue_block_whole(c, b, slot);
+	const int wave = threadIdx.x >> 6, lane = lane_id();
+	for(uint32_t base = 0; base < n; base += kSlots * 1024) {
+		uint32_t flags[kSlots], m[kSlots], at[kSlots], v[2][kSlots], inc[2][kSlots];
+#pragma unroll
+		for(int i = 0; i < kSlots; i++) {
+			const uint32_t slot = base + i * 1024 + threadIdx.x;
+			flags[i] = slot < n ? b.blk_flags[slot] : 0u;
+			m[i] = slot < n ? b.blk_slot[slot].y : 0u;
+			at[i] = slot < n ? b.blk_sorted[slot] : 0u;
 		}
-		uint32_t inc[2];
+#pragma unroll
+		for(int i = 0; i < kSlots; i++) {
+			const uint32_t level = flags[i] & kSlotLevelMask;
+			const bool live = level != LUCID_BIN_LEVEL_EMPTY && !(flags[i] & (kSlotWhole | kSlotPromoted)) && m[i];
+			v[0][i] = live ? m[i] : 0u;
+			v[1][i] = !live ? 0u : (flags[i] & kSlotPresorted) ? b.sorted_pool[at[i]] : 1u;
+			if(REUSE && (flags[i] & kSlotWhole))
+				enqueue_block_whole(c, b, base + i * 1024 + threadIdx.x);
+		}
+#pragma unroll
 		for(int k = 0; k < 2; k++) {
-			inc[k] = wave_inclusive_add(v[k]);
-			if(lane_id() == 63)
-				s_wave[k][wave] = inc[k];
-		}
-		__syncthreads();
-		if(threadIdx.x < 2) {
-			const int k = threadIdx.x;
-			uint32_t run = s_carry[k];
-			for(int w = 0; w < 16; w++) {
-				uint32_t x = s_wave[k][w];
-				s_wave[k][w] = run;
-				run += x;
+#pragma unroll
+			for(int i = 0; i < kSlots; i++) {
+				inc[k][i] = wave_inclusive_add(v[k][i]);
+				if(lane == 63)
+					s_wave[k][i * 16 + wave] = inc[k][i];
 			}
-			s_carry[k] = run;
 		}
 		__syncthreads();
-		if(slot < n) {
-			g.row_base[slot] = s_wave[0][wave] + inc[0] - v[0];
-			g.range_base[slot] = s_wave[1][wave] + inc[1] - v[1];
+		if(wave < 2) { // wave k: the sums before each (slot, wave)
+			static_assert(kSlots * 16 == 64, "a lane per sum");
+			const uint32_t x = s_wave[wave][lane], ex = wave_inclusive_add(x) - x + s_carry[wave];
+			s_wave[wave][lane] = ex;
+			if(lane == 63)
+				s_carry[wave] = ex + x;
+		}
+		__syncthreads();
+#pragma unroll
+		for(int i = 0; i < kSlots; i++) {
+			const uint32_t slot = base + i * 1024 + threadIdx.x;
+			if(slot < n) {
+				g.row_base[slot] = s_wave[0][i * 16 + wave] + inc[0][i] - v[0][i];
+				g.range_base[slot] = s_wave[1][i * 16 + wave] + inc[1][i] - v[1][i];
+			}
 		}
 		__syncthreads();
 	}

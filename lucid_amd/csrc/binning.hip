@@ -328,6 +328,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		b.ctrl[kCtrlTotalBinQuads] = nq;
 		b.ctrl[kCtrlTotalBinTris] = nt;
 		b.ctrl[kCtrlFixedHigh] = nhigh;
+		b.ctrl[kCtrlFixedFit] = fits ? 1u : 0u;
 		// the size the host grows the lists to after an overflow (promoted bins add theirs)
 		b.ctrl[kCtrlListCursor] = (uint32_t)min(16ull * total[4], 0xffffffffull);
 		const uint32_t ovf = (nq > b.bin_quads_cap || nt > b.bin_tris_cap ? kOvfBinLists : 0u) |

@@ -48,6 +48,7 @@ enum CtrlWord : int {
 	// device-only words (not copied to the host) up to kStatStripeBase:
 	kCtrlBigSorts = 16, // blocks queued in big_queue for the long-list sort pass
 	kCtrlFixedHigh = 17, // high bins before row generation adds the promoted ones
+	kCtrlFixedFit = 18,  // 1: the lists of those bins fit (promoted bins may still set kOvfLists)
 };
 
 // Frame statistics summed per block (fragments, list entries) go to kStatStripes counters

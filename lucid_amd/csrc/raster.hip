@@ -1314,14 +1314,14 @@ template <int THREADS>
 __device__ __forceinline__ void rowgen_high_body(const FrameConst &c, const FrameBufs &b, uint32_t id) {
 	constexpr uint32_t kSplits = kRowgenSplitThreads / THREADS;
 	const uint32_t slot = id / kSplits, split = id % kSplits;
-	const uint32_t overflow = b.ctrl[kCtrlOverflow];
-	if((overflow & kOvfBinLists) || slot >= b.ctrl[kCtrlFixedHigh])
+	if((b.ctrl[kCtrlOverflow] & kOvfBinLists) || slot >= b.ctrl[kCtrlFixedHigh])
 		return;
 	const int bin = (int)b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + slot];
 	const BinInfo bi = load_bin(c, b, bin);
 	const uint32_t lst = b.blk_slot[(size_t)bin * 16].x;
-	// (a low bin that is promoted meanwhile may set kOvfLists: such a frame is rendered again)
-	const bool fits = !(overflow & kOvfLists);
+	// Not kOvfLists: a low bin promoted in the same launch may set that while the waves of this
+	// work-group read it, and waves that disagree would miss each other at the barriers below.
+	const bool fits = b.ctrl[kCtrlFixedFit] != 0u;
 	if(split == 0 && threadIdx.x < 16) {
 		if(threadIdx.x > 0)
 			b.blk_slot[(size_t)bin * 16 + threadIdx.x] = make_uint2(lst + threadIdx.x * bi.nlevel, 0u);

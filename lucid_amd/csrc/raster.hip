@@ -1828,13 +1828,15 @@ constexpr bool is_plain(int mode) { return shade_kind(mode) == kShadePlain; }
 constexpr bool is_textured(int mode) { return shade_kind(mode) == kShadeTextured; }
 // Window slots of the register-sorted and the pre-sorted blocks. A pre-sorted pixel's depth ranges
 // are composited apart and then chained, which rounds differently from the exact sort: there the
-// general kinds keep four slots, so that no RGBA8 pixel changes to the exact sort by the tuning.
+// general and plain kinds keep four slots, so that no pixel's bits change by the tuning, or from run
+// to run, with the exact sort that fewer slots would send it to. (Flat ones take one slot there,
+// which costs an RGBA8 byte now and then.)
 constexpr int window_slots(int mode, bool presorted) {
-	return !(mode & kShadeNarrow) ? kWindow
-		   : is_flat(mode)		  ? kNarrowWindow
-		   : is_plain(mode)		  ? kNarrowPlainWindow
-		   : presorted			  ? kWindow
-								  : kNarrowGeneralWindow;
+	return !(mode & kShadeNarrow)		  ? kWindow
+		   : is_flat(mode)				  ? kNarrowWindow
+		   : presorted					  ? kWindow
+		   : is_plain(mode)				  ? kNarrowPlainWindow
+										  : kNarrowGeneralWindow;
 }
 constexpr int rec_quads(int mode) { return is_flat(mode) ? kFlatQuads : kRecQuads; }
 // LDS of one wave's slice of 64 W records

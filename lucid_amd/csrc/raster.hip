@@ -474,19 +474,18 @@ struct OrderWindow {
 	uint64_t k0, k1, k2, k3;
 	P c0, c1, c2, c3;
 	uint32_t n;           // filled slots
-	uint64_t first_key, last; // first and last emitted key (kEmptyKey / 0 before the first)
+	uint64_t first, last; // first and last emitted key (0 before the first)
 	bool bad;
 
-	__device__ __forceinline__ uint32_t first() const { return (uint32_t)(first_key >> 32); }
 	__device__ __forceinline__ void init() {
 		k0 = k1 = k2 = k3 = kEmptyKey;
 		c0.zero(), c1.zero(), c2.zero(), c3.zero();
-		n = 0, first_key = kEmptyKey, last = 0, bad = false;
+		n = 0, first = last = 0, bad = false;
 	}
 
 	template <class F> __device__ __forceinline__ void emit(uint64_t k, const P &col, F &&f) {
 		bad |= k <= last;
-		first_key = first_key == kEmptyKey ? k : first_key;
+		first = last == 0ull ? k : first;
 		last = k;
 		f(col);
 	}
@@ -557,18 +556,22 @@ struct SmallWindow {
 	// recording does not). The keys of one pixel are distinct (one sample per triangle).
 	uint64_t k0, k1;
 	P c0, c1;
-	uint64_t last;
-	uint32_t first_depth; // smallest depth key inserted: for an exact pixel the first one emitted
+	uint64_t first, last; // first and last emitted key (0 before the first)
 	uint32_t bad;         // samples that came after a later one had left
 
 	__device__ __forceinline__ void init() {
 		k0 = k1 = 0ull;
 		c0.zero(), c1.zero();
-		first_depth = ~0u, last = 0, bad = 0;
+		first = last = 0, bad = 0;
 	}
-	__device__ __forceinline__ uint32_t first() const { return first_depth; }
+	template <class F> __device__ __forceinline__ void emit(uint64_t k, const P &col, F &&f) {
+		if(PH || k != 0ull) {
+			first = last == 0ull ? k : first;
+			last = k;
+			f(col);
+		}
+	}
 	template <class F> __device__ __forceinline__ void insert(uint64_t key, const P &col, F &&f) {
-		first_depth = min(first_depth, (uint32_t)(key >> 32));
 		const uint64_t back = N == 1 ? k0 : k1;
 		uint64_t ke = k0, n0 = N == 1 ? key : k1, n1 = key;
 		P ce, m0, m1;
@@ -592,22 +595,12 @@ struct SmallWindow {
 		k0 = n0, c0 = m0;
 		if constexpr(N == 2)
 			k1 = n1, c1 = m1;
-		if(PH || ke != 0ull) {
-			last = ke;
-			f(ce);
-		}
+		emit(ke, ce, f);
 	}
 	template <class F> __device__ __forceinline__ void flush(F &&f) {
-		if(PH || k0 != 0ull) { // the last samples, or placeholders
-			last = k0;
-			f(c0);
-		}
-		if constexpr(N == 2) {
-			if(PH || k1 != 0ull) {
-				last = k1;
-				f(c1);
-			}
-		}
+		emit(k0, c0, f); // the last samples, or placeholders
+		if constexpr(N == 2)
+			emit(k1, c1, f);
 		k0 = k1 = 0ull;
 		c0.zero(), c1.zero();
 	}
@@ -2223,8 +2216,8 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 	// work-groups fit on a CU.
 	struct RangeEnd {
 		float4 part[64]; // the range's partial composite
-		uint32_t first[64], last[64]; // depth keys of the first and the last sample emitted
-		uint32_t cnt[64];             // fragments | 0x80000000 when the range's order is not exact
+		uint64_t first[64], last[64];
+		uint32_t cnt[64]; // fragments | 0x80000000 when the range's order is not exact
 	};
 	static_assert(sizeof(RangeEnd) <= sizeof(s_rec[0]), "a range's end state fits its staging");
 	auto range_end = [&](int w) -> RangeEnd & { return *reinterpret_cast<RangeEnd *>(&s_rec[w][0]); };
@@ -2272,8 +2265,8 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 		wave_sync_lds(); // every lane is done with the staged records (also after an early end)
 		RangeEnd &re = range_end(wave);
 		re.part[lane] = make_float4(ps.acc.cr, ps.acc.cg, ps.acc.cb, ps.acc.tr);
-		re.first[lane] = ps.w.first();
-		re.last[lane] = (uint32_t)(ps.w.last >> 32);
+		re.first[lane] = ps.w.first;
+		re.last[lane] = ps.w.last;
 		re.cnt[lane] = count | (ps.w.bad ? 0x80000000u : 0u);
 	}
 	__syncthreads();
@@ -2281,7 +2274,7 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 		return;
 	Accum acc;
 	acc.init();
-	uint32_t last = 0;
+	uint64_t last = 0;
 	bool bad = false;
 	uint32_t count = 0;
 	for(uint32_t w = 0; w < nw; w++) {
@@ -2289,8 +2282,8 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 		const uint32_t cw = re.cnt[lane];
 		count += cw & 0x7fffffffu;
 		bad |= (cw >> 31) != 0;
-		const uint32_t f = re.first[lane];
-		if(f != ~0u) { // the range has samples here (equal depths in two ranges: not in order)
+		const uint64_t f = re.first[lane];
+		if(f != 0ull) { // the range has samples here
 			bad |= f <= last;
 			last = re.last[lane];
 			const float4 p = re.part[lane];
@@ -2782,8 +2775,8 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 	struct RangeEnd {
 		double pc[4][64]; // C rgb, T (fp64)
 		float4 p32[64];   // fp32 partial composite
-		uint32_t first[64], last[64]; // depth keys
-		uint32_t bad[64], count[64];  // count: RECORD, fragments per pixel
+		uint64_t first[64], last[64];
+		uint32_t bad[64], count[64]; // count: RECORD, fragments per pixel
 	};
 	__shared__ uint4 s_rec[kBigWaves][kSliceEntries * kRecQuads];
 	static_assert(sizeof(RangeEnd) <= sizeof(s_rec[0]), "a range's end state fits its staging");
@@ -2859,7 +2852,7 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 		re.pc[0][lane] = part.cr, re.pc[1][lane] = part.cg;
 		re.pc[2][lane] = part.cb, re.pc[3][lane] = part.t;
 		re.p32[lane] = make_float4(part.acc.cr, part.acc.cg, part.acc.cb, part.acc.tr);
-		re.first[lane] = w.first(), re.last[lane] = (uint32_t)(w.last >> 32);
+		re.first[lane] = w.first, re.last[lane] = w.last;
 		re.bad[lane] = w.bad ? 1u : 0u;
 		re.count[lane] = count;
 	}
@@ -2876,15 +2869,15 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 	double cb4[3] = {0.0, 0.0, 0.0}, tb4 = 1.0; // composite of the ranges before this one
 	Accum a32;
 	a32.init();
-	uint32_t last = 0;
+	uint64_t last = 0;
 	bool bad = false;
 	for(uint32_t v = 0; v < ent.nw; v++) {
 		if(v == (uint32_t)wave)
 			cb4[0] = ct[0], cb4[1] = ct[1], cb4[2] = ct[2], tb4 = tt;
 		const RangeEnd &re = range_end((int)v);
 		bad |= re.bad[lane] != 0;
-		const uint32_t f = re.first[lane];
-		if(f != ~0u) {
+		const uint64_t f = re.first[lane];
+		if(f != 0ull) {
 			bad |= f <= last;
 			last = re.last[lane];
 		}

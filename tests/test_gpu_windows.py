@@ -48,3 +48,33 @@ def test_fp32_presorted_blocks_keep_their_bits(n, slope, blend):
     for g in got:
         for k in ref:
             assert np.array_equal(g[k].view(np.uint32), ref[k].view(np.uint32)), k
+
+
+def _coplanar_pairs(n, w, h):
+    """n parallel tilted layers, each of two triangles in exactly one plane (the second has the
+    first one's corner and edges, one of them doubled, in dyadic coordinates, so that both depth
+    planes have the same bits). In blocks that the first one's edge crosses their pixel masks, and
+    so their centroids' depths, differ, and the first one comes first, as by its id."""
+    p0 = np.stack([np.full(n, -32.0), np.full(n, -32.0), -(16.0 + np.arange(n) / 8.0)], -1)
+    u, v = np.array([64.0, 0.0, -1.0]), np.array([0.0, 64.0, 0.0])
+    pos = np.stack([p0, p0 + u, p0 + v, p0, p0 + 2 * u, p0 + v], 1).reshape(-1, 3)
+    rng = np.random.default_rng(n)
+    sc = scenes.soup_scene(w, h, np.zeros((2 * n, 3, 2)), np.ones(2 * n), rng.uniform(0, 1, (2 * n, 3, 3)),
+                           rng.uniform(0.001, 0.01, 2 * n), name=f"coplanar_{n}")
+    sc.positions = pos.astype(np.float32)
+    assert np.array_equal(sc.positions, pos)
+    return sc
+
+
+@pytest.mark.parametrize("window", [1, 4])
+@pytest.mark.parametrize("opts", [0, _lib.OPT_FP32_SAMPLES])
+def test_equal_depths_in_two_ranges_are_ordered_by_id(oracle_mod, opts, window):
+    """Equal depths on both sides of a depth range's end, in the order of their ids: exact, so no
+    pixel takes the exact sort."""
+    sc = _coplanar_pairs(300, 72, 64)
+    (got,), stats = _render(sc, opts, window)
+    assert stats["block_tris"] > 300 * 16 and stats["fragments"] > 300 * 1024
+    assert stats["fallback_pixels"] == 0
+    ref = oracle_mod.render(sc, opts=oracle_mod.OPT_FP32_SAMPLES if opts else 0)
+    assert np.array_equal(got["frag_counts"].astype(np.uint32), ref["frag_counts"])
+    assert np.abs(got["image"].astype(int) - ref["image"].astype(int)).max() <= 1

@@ -328,16 +328,20 @@ __device__ __forceinline__ uint32_t batch_frame(const StageBatch &sb, uint32_t w
 // kShadeNarrow (a flag): narrow ordering windows (tuning window 1).
 enum ShadeMode : int { kShadeGeneral = 0, kShadeTextured = 1, kShadeFlat = 2, kShadePlain = 3, kShadeNarrow = 4 };
 
+// Whether a frame may take the narrow windows with records of this kind. The alpha threshold looks
+// at the samples that have left the window, so its results depend on the slots: only flat records
+// take it with the narrow ones.
+inline bool narrow_windows(const FrameConst &c, int kind) {
+	return c.window == 1 && (kind == kShadeFlat || !(c.opts & LUCID_OPT_ALPHA_THRESHOLD));
+}
+
 inline int frame_shade_mode(const FrameConst &c) {
 	const bool fp32 = (c.opts & LUCID_OPT_FP32_SAMPLES) != 0;
 	const bool flat_colors = c.color_mode == kColorNone || c.color_mode == kColorF32;
 	const int kind = c.has_textures ? kShadeTextured
 					 : fp32 ? (c.plain_colors ? kShadePlain : kShadeGeneral)
 							: (c.identity_light && flat_colors ? kShadeFlat : kShadeGeneral);
-	// the alpha threshold looks at the samples that have left the window, so its results depend
-	// on the slots: only flat frames take it with the narrow ones
-	const bool threshold = (c.opts & LUCID_OPT_ALPHA_THRESHOLD) != 0;
-	return kind | (c.window == 1 && (kind == kShadeFlat || !threshold) ? kShadeNarrow : 0);
+	return kind | (narrow_windows(c, kind) ? kShadeNarrow : 0);
 }
 
 struct BatchPlan {

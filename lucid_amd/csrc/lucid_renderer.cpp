@@ -1186,7 +1186,7 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 	}
 	const size_t n = bt->rs.size();
 	std::vector<FrameDesc> frames(n);
-	bool tex = false, fast = true, narrow = true; // fast: flat or plain records for every frame
+	bool tex = false, fast = true; // fast: flat or plain records for every frame
 	int fast_mode = kShadeGeneral;
 	for(size_t i = 0; i < n; i++) {
 		lucid_renderer *r = bt->rs[i];
@@ -1204,9 +1204,7 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 		frames[i].c.slice_words = bt->rs[0]->tuning.slice_words;
 		frames[i].b.host_status = bt->status_dev + i * kCtrlWords;
 		tex = tex || frames[i].c.has_textures;
-		const int mode = frame_shade_mode(frames[i].c);
-		narrow = narrow && (mode & kShadeNarrow);
-		fast_mode = mode & ~kShadeNarrow;
+		fast_mode = frame_shade_mode(frames[i].c) & ~kShadeNarrow;
 		fast = fast && (fast_mode == kShadeFlat || fast_mode == kShadePlain);
 		r->last_num_quads = nq;
 		r->last_stream = stream;
@@ -1232,8 +1230,12 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 	plan.bin_lds = bin_lds;
 	plan.fp32 = (bt->rs[0]->opts & LUCID_OPT_FP32_SAMPLES) != 0;
 	// (one sample format: fast frames are all flat or all plain)
-	plan.mode = (tex ? kShadeTextured : fast ? fast_mode : kShadeGeneral) |
-				(narrow ? kShadeNarrow : 0);
+	plan.mode = tex ? kShadeTextured : fast ? fast_mode : kShadeGeneral;
+	// narrow windows if every frame may take them with the records that the batch has in the end
+	// (a flat frame with the alpha threshold may not among general or textured ones)
+	const int kind = plan.mode;
+	if(std::all_of(frames.begin(), frames.end(), [&](const FrameDesc &f) { return narrow_windows(f.c, kind); }))
+		plan.mode |= kShadeNarrow;
 	plan.slice_words = bt->rs[0]->tuning.slice_words;
 	// the launches read the frames' constants and buffers from device memory, so a frame
 	// whose inputs change only needs them uploaded; the graph is recorded again only when a

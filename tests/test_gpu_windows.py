@@ -12,13 +12,15 @@ pytestmark = pytest.mark.gpu
 
 
 def _planes(n, w, h, slope, alpha, seed, color_format="f32"):
-    """n screen-filling quads at even depths, with slopes that make near neighbours cross."""
+    """n screen-filling quads at even depths, with slopes that make near neighbours cross. alpha: a
+    range, or the alphas from the nearest on."""
     rng = np.random.default_rng(seed)
     corners = np.array([[-1.3, -1.2], [1.2, -1.3], [1.3, 1.2], [-1.2, 1.3]])
     ndc = np.repeat(corners[None], n, axis=0)
     k = rng.uniform(-slope, slope, (n, 2))
-    depth = 10.0 + 0.05 * rng.permutation(n)[:, None] + corners[:, 0] * k[:, :1] + corners[:, 1] * k[:, 1:]
-    a = np.broadcast_to(alpha, n) if np.ndim(alpha) == 0 else rng.uniform(*alpha, n)
+    rank = rng.permutation(n)
+    depth = 10.0 + 0.05 * rank[:, None] + corners[:, 0] * k[:, :1] + corners[:, 1] * k[:, 1:]
+    a = alpha[rank] if isinstance(alpha, np.ndarray) else rng.uniform(*alpha, n)
     return scenes.quad_soup_scene(w, h, ndc, depth, rng.uniform(0.0, 1.0, (n, 4, 3)), a,
                                   color_format=color_format, name=f"crossing_{n}")
 
@@ -78,3 +80,34 @@ def test_equal_depths_in_two_ranges_are_ordered_by_id(oracle_mod, opts, window):
     ref = oracle_mod.render(sc, opts=oracle_mod.OPT_FP32_SAMPLES if opts else 0)
     assert np.array_equal(got["frag_counts"].astype(np.uint32), ref["frag_counts"])
     assert np.abs(got["image"].astype(int) - ref["image"].astype(int)).max() <= 1
+
+
+@pytest.mark.parametrize("other", ["bytes", "textured"])
+def test_batch_of_mixed_frames_keeps_the_threshold_wide(other):
+    """A flat frame with the alpha threshold batched with a byte-coloured or textured frame without
+    it: the batch's records are then not flat, and the threshold, which looks at the samples that
+    have left the window, needs the four slots whatever the tuning. After the first 64 of the 100
+    layers the transmittance is below 1/128 with all but two of them blended, and not yet with all
+    but four."""
+    from lucid_amd.batch import LucidBatch
+    from lucid_amd.renderer import GpuScene, LucidRenderer
+    alpha = np.where(np.arange(100) % 2, 19.0, 20.0) / 255.0
+    left = np.cumprod(1.0 - alpha)
+    assert left[59] > 1.0 / 128.0 > left[61]
+    flat = _planes(100, 40, 32, 0.0, alpha, seed=2)
+    if other == "bytes":
+        second = scenes.config0(seed=6, num_tris=500, width=64, height=40, color_format="rgba8")
+    else:
+        second = scenes.textured_planes(64, 40, 5, seed=7)
+    images = {}
+    for window in (4, 1):
+        print(f"\n[case] batch of flat and {other}, window={window}", flush=True)
+        rs = [LucidRenderer((40, 32), opts=_lib.OPT_ALPHA_THRESHOLD), LucidRenderer((64, 40))]
+        for r in rs:
+            r.set_tuning(window=window)
+        outs = [r.alloc_outputs(rgba8=True, rgba32f=True, counts=True) for r in rs]
+        LucidBatch(rs).render([GpuScene(flat), GpuScene(second)], outs)
+        images[window] = [{k: v.cpu().numpy() for k, v in o.items()} for o in outs]
+    for a, b in zip(images[1], images[4]):
+        for k in a:
+            assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k

@@ -295,7 +295,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		}
 	}
 	const uint64_t list0 = (uint64_t)NB * 16 * kRegSortCap;
-	const bool fits = list0 + 16ull * total[4] <= b.blk_lists_cap;
+	const bool fits = lists_fit(list0, 0u, total[4], b.blk_lists_cap);
 	for(int i = b0; i < b1; i += 64 * kAhead) {
 		load(i);
 #pragma unroll
@@ -318,7 +318,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 					counts[LUCID_COUNTS_LOW_BINS * NB + at[2]] = (uint32_t)bin;
 				if(v[3]) {
 					counts[LUCID_COUNTS_HIGH_BINS * NB + at[3]] = (uint32_t)bin;
-					b.blk_slot[(size_t)bin * 16] = make_uint2((uint32_t)(list0 + 16ull * at[4]), 0u);
+					b.blk_slot[(size_t)bin * 16] = make_uint2((uint32_t)list_entry(list0, at[4]), 0u);
 				}
 			}
 		}
@@ -330,7 +330,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		b.ctrl[kCtrlFixedHigh] = nhigh;
 		b.ctrl[kCtrlFixedFit] = fits ? 1u : 0u;
 		// the size the host grows the lists to after an overflow (promoted bins add theirs)
-		b.ctrl[kCtrlListCursor] = (uint32_t)min(16ull * total[4], 0xffffffffull);
+		b.ctrl[kCtrlListCursor] = list_cursor_start(total[4]);
 		const uint32_t ovf = (nq > b.bin_quads_cap || nt > b.bin_tris_cap ? kOvfBinLists : 0u) |
 							 (fits ? 0u : kOvfLists);
 		if(ovf)

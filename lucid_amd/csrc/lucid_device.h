@@ -16,6 +16,7 @@
 
 #include "../../include/lucid_c.h"
 #include "../../include/lucid_structs.h"
+#include "list_space.h"
 
 namespace lucid {
 
@@ -36,7 +37,7 @@ enum CtrlWord : int {
 	kCtrlTotalBinQuads = 5,
 	kCtrlTotalBinTris = 6,
 	kCtrlFallbackPixels = 7,
-	kCtrlListCursor = 8,    // high-bin block-list space the frame needs (entries)
+	kCtrlListCursor = 8,    // list positions of high bins (list_space.h): the space the frame needs
 	kCtrlOverflowCarry = 9, // overflow bits of earlier frames not yet seen by the host
 	kCtrlSortedCursor = 10, // pre-sorted pool size a frame needed, after an overflow (u32 units)
 	kCtrlBwdRows = 11,      // gradient rows of the block kernel (set by the row scan)

@@ -236,10 +236,11 @@ int grow_after_overflow(lucid_renderer *r) {
 	}
 	if(flags & kOvfLists) {
 		uint64_t low = (uint64_t)r->bin_count * 16 * kRegSortCap;
-		uint64_t need = std::max<uint64_t>(low + (uint64_t)r->status[kCtrlListCursor],
-										   r->blk_lists_cap * 5 / 4);
-		LUCID_CHECK(r->blk_lists.reserve(need * 16));
-		r->blk_lists_cap = need;
+		const uint64_t cap = grown_list_cap(low, r->status[kCtrlListCursor], r->blk_lists_cap);
+		if(!cap)
+			return LUCID_ERR_OUT_OF_MEMORY;
+		LUCID_CHECK(r->blk_lists.reserve(cap * 16));
+		r->blk_lists_cap = cap;
 	}
 	if(flags & kOvfSorted) {
 		uint64_t need = std::max<uint64_t>((uint64_t)r->status[kCtrlSortedCursor], r->sorted_cap * 2);

@@ -1284,12 +1284,12 @@ __device__ __forceinline__ void rowgen_low_bin(const FrameConst &c, const FrameB
 		lucid_info *info = (lucid_info *)b.info;
 		uint32_t id = atomicAdd((uint32_t *)&info->bin_level_counts[LUCID_BIN_LEVEL_HIGH], 1u);
 		b.info[LUCID_INFO_U32_SIZE + LUCID_COUNTS_HIGH_BINS * c.bin_count + id] = (uint32_t)bin;
-		const uint32_t off = atomicAdd(&b.ctrl[kCtrlListCursor], 16u * bi.nlevel);
-		const uint64_t lst = (uint64_t)c.bin_count * 16 * kRegSortCap + off;
-		const bool ok = lst + 16ull * bi.nlevel <= b.blk_lists_cap;
+		const uint64_t list0 = (uint64_t)c.bin_count * 16 * kRegSortCap;
+		const uint32_t cursor = atomicAdd(&b.ctrl[kCtrlListCursor], bi.nlevel);
+		const bool ok = lists_fit(list0, cursor, bi.nlevel, b.blk_lists_cap);
 		if(!ok)
 			atomicOr(&b.ctrl[kCtrlOverflow], kOvfLists);
-		sh.blk_n[0] = (uint32_t)lst, sh.blk_n[1] = ok ? 1u : 0u;
+		sh.blk_n[0] = (uint32_t)list_entry(list0, cursor), sh.blk_n[1] = ok ? 1u : 0u;
 	}
 	__syncthreads();
 	const uint32_t lst = sh.blk_n[0];

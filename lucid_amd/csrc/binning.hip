@@ -242,7 +242,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 	lucid_info *info = (lucid_info *)b.info;
 	const uint32_t *qcs = counts + LUCID_COUNTS_QUAD_COUNTS * NB, *tcs = counts + LUCID_COUNTS_TRI_COUNTS * NB;
 	constexpr int kWaves = kScanThreads / 64;
-	__shared__ uint32_t s_wave[kWaves][5];
+	__shared__ uint32_t s_wave[kWaves][5], s_refs[kWaves][2];
 	const int wave = threadIdx.x >> 6, lane = lane_id();
 	const int run = (NB + 64 * kWaves - 1) / (64 * kWaves) * 64;
 	const int b0 = wave * run, b1 = min(NB, b0 + run);
@@ -267,6 +267,9 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		v[4] = high ? n : 0u;
 	};
 	uint32_t ex[5] = {0u, 0u, 0u, 0u, 0u}, total[5];
+	// every list position in 64 bits (a bin has less than 2^31): where they pass 32 bits, the sums
+	// and offsets above wrap, and the frame must not go on to use them
+	uint64_t refs = 0;
 	for(int i = b0; i < b1; i += 64 * kAhead) {
 		load(i);
 #pragma unroll
@@ -276,6 +279,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 #pragma unroll
 			for(int k = 0; k < 5; k++)
 				ex[k] += v[k];
+			refs += (uint64_t)t[j] + 2ull * q[j];
 		}
 	}
 #pragma unroll
@@ -284,7 +288,16 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		if(lane == 0)
 			s_wave[wave][k] = sum;
 	}
+	const uint32_t refs_lo = wave_read(wave_inclusive_add((uint32_t)refs & 0xfffffu), 63);
+	const uint32_t refs_hi = wave_read(wave_inclusive_add((uint32_t)(refs >> 20)), 63);
+	if(lane == 0)
+		s_refs[wave][0] = refs_lo, s_refs[wave][1] = refs_hi;
 	__syncthreads();
+	refs = 0;
+#pragma unroll
+	for(int w = 0; w < kWaves; w++)
+		refs += s_refs[w][0] + ((uint64_t)s_refs[w][1] << 20);
+	const bool wrapped = refs >= kBinListsWrapped;
 #pragma unroll
 	for(int k = 0; k < 5; k++) {
 		total[k] = ex[k] = 0;
@@ -295,7 +308,7 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 		}
 	}
 	const uint64_t list0 = (uint64_t)NB * 16 * kRegSortCap;
-	const bool fits = lists_fit(list0, 0u, total[4], b.blk_lists_cap);
+	const bool fits = !wrapped && lists_fit(list0, 0u, total[4], b.blk_lists_cap);
 	for(int i = b0; i < b1; i += 64 * kAhead) {
 		load(i);
 #pragma unroll
@@ -326,12 +339,12 @@ __device__ __forceinline__ void categorize_bins(const FrameConst &c, const Frame
 	if(threadIdx.x == 0) {
 		const uint32_t nq = total[0], nt = total[1], nlow = total[2], nhigh = total[3];
 		b.ctrl[kCtrlTotalBinQuads] = nq;
-		b.ctrl[kCtrlTotalBinTris] = nt;
+		b.ctrl[kCtrlTotalBinTris] = wrapped ? kBinListsWrapped : nt;
 		b.ctrl[kCtrlFixedHigh] = nhigh;
 		b.ctrl[kCtrlFixedFit] = fits ? 1u : 0u;
 		// the size the host grows the lists to after an overflow (promoted bins add theirs)
 		b.ctrl[kCtrlListCursor] = list_cursor_start(total[4]);
-		const uint32_t ovf = (nq > b.bin_quads_cap || nt > b.bin_tris_cap ? kOvfBinLists : 0u) |
+		const uint32_t ovf = (wrapped || nq > b.bin_quads_cap || nt > b.bin_tris_cap ? kOvfBinLists : 0u) |
 							 (fits ? 0u : kOvfLists);
 		if(ovf)
 			atomicOr(&b.ctrl[kCtrlOverflow], ovf);

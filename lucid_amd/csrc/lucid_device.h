@@ -35,7 +35,7 @@ enum CtrlWord : int {
 	kCtrlOverflow = 3,      // kOvf* bits
 	kCtrlSpillCursor = 4,   // bump allocator of the deep-pixel spill pool (u64 units)
 	kCtrlTotalBinQuads = 5,
-	kCtrlTotalBinTris = 6,
+	kCtrlTotalBinTris = 6,  // kBinListsWrapped: more list positions than 32 bits count
 	kCtrlFallbackPixels = 7,
 	kCtrlListCursor = 8,    // list positions of high bins (list_space.h): the space the frame needs
 	kCtrlOverflowCarry = 9, // overflow bits of earlier frames not yet seen by the host
@@ -51,6 +51,8 @@ enum CtrlWord : int {
 	kCtrlFixedHigh = 17, // high bins before row generation adds the promoted ones
 	kCtrlFixedFit = 18,  // 1: the lists of those bins fit (promoted bins may still set kOvfLists)
 };
+
+constexpr uint32_t kBinListsWrapped = 0xffffffffu;
 
 // Frame statistics summed per block (fragments, list entries) go to kStatStripes counters
 // per statistic, one 128-byte line each, after the control words in the same buffer: the

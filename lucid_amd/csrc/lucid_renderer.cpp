@@ -225,6 +225,8 @@ int grow_after_overflow(lucid_renderer *r) {
 	if(!flags)
 		return LUCID_OK;
 	if(flags & kOvfBinLists) {
+		if(r->status[kCtrlTotalBinTris] == kBinListsWrapped)
+			return LUCID_ERR_OUT_OF_MEMORY; // the bins' offsets are 32 bits
 		uint64_t need = std::max<uint64_t>(r->status[kCtrlTotalBinTris], r->bin_tris_cap * 2);
 		LUCID_CHECK(r->bin_tris.reserve(need * 4));
 		r->bin_tris_cap = need;

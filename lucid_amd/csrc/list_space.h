@@ -28,12 +28,13 @@ constexpr bool lists_fit(uint64_t low_entries, uint32_t cursor, uint32_t positio
 }
 
 // Capacity after an overflow of `cap` entries, from the cursor that the frame left; 0 if no
-// capacity will do.
+// capacity will do. Twice the old one, so that a scene that grows a little every frame overflows
+// seldom (the frames of an asynchronous loop that overflow are lost).
 constexpr uint64_t grown_list_cap(uint64_t low_entries, uint32_t cursor, uint64_t cap) {
 	const uint64_t need = list_entry(low_entries, cursor);
 	if(need > kMaxListEntries)
 		return 0;
-	const uint64_t more = cap * 5 / 4;
+	const uint64_t more = cap * 2;
 	return need > more ? need : more < kMaxListEntries ? more : kMaxListEntries;
 }
 

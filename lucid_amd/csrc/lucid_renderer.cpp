@@ -76,18 +76,24 @@ struct DevBuf {
 			(void)hipFree(ptr);
 		ptr = nullptr, bytes = 0;
 	}
-	// Grows (never shrinks); contents are not preserved.
+	// Grows (never shrinks); contents are not preserved. A buffer that cannot grow keeps its size:
+	// its owner's capacity still stands.
 	hipError_t reserve(size_t need) {
 		if(need <= bytes)
 			return hipSuccess;
+		const size_t old = bytes;
 		release();
-		hipError_t e = hipMalloc(&ptr, need);
-		if(e != hipSuccess) {
-			ptr = nullptr;
-			return e;
+		const hipError_t e = hipMalloc(&ptr, need);
+		if(e == hipSuccess) {
+			bytes = need;
+			return hipSuccess;
 		}
-		bytes = need;
-		return hipSuccess;
+		(void)hipGetLastError();
+		if(old && hipMalloc(&ptr, old) == hipSuccess)
+			bytes = old;
+		else
+			ptr = nullptr;
+		return e;
 	}
 	template <class T> T *as() const { return (T *)ptr; }
 };
@@ -241,8 +247,10 @@ int grow_after_overflow(lucid_renderer *r) {
 		const uint64_t cap = grown_list_cap(low, r->status[kCtrlListCursor], r->blk_lists_cap);
 		if(!cap)
 			return LUCID_ERR_OUT_OF_MEMORY;
-		LUCID_CHECK(r->blk_lists.reserve(cap * 16));
-		r->blk_lists_cap = cap;
+		// where twice the space is more than the GPU has left, just what this frame needs
+		if(r->blk_lists.reserve(cap * 16) != hipSuccess)
+			LUCID_CHECK(r->blk_lists.reserve(list_entry(low, r->status[kCtrlListCursor]) * 16));
+		r->blk_lists_cap = r->blk_lists.bytes / 16;
 	}
 	if(flags & kOvfSorted) {
 		uint64_t need = std::max<uint64_t>((uint64_t)r->status[kCtrlSortedCursor], r->sorted_cap * 2);
@@ -631,6 +639,7 @@ int prepare_frame(lucid_renderer *r, const lucid_frame_inputs *in, const lucid_f
 	b.blk_flags = r->blk_flags.as<uint32_t>();
 	b.blk_sorted = r->blk_sorted.as<uint32_t>();
 	b.big_queue = b.blk_sorted + (size_t)r->bin_count * 16;
+	LUCID_CHECK(r->blk_lists.reserve(r->blk_lists_cap * 16)); // (lost if it could not grow back)
 	b.blk_lists = r->blk_lists.as<uint4>();
 	b.blk_lists_cap = r->blk_lists_cap;
 	b.blk_count = r->blk_count.as<uint32_t>();

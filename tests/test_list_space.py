@@ -70,3 +70,32 @@ def compile_and_run(tmp_path_factory):
 def test_cursor_and_offsets(compile_and_run):
     out = compile_and_run(PROGRAM)
     assert out.returncode == 0 and out.stdout == "ok\n", out.stderr
+
+
+GROWING = r"""
+#include "list_space.h"
+#include <stdio.h>
+using namespace lucid;
+
+int main() {
+	// a scene whose lists grow by 5 % a frame, to about 300 times the first space
+	const uint64_t low = 2040ull * 16 * 256;
+	uint64_t cap = low + (1ull << 22);
+	int frames = 0, overflows = 0;
+	for(double p = 200000.0; p < 60e6; p *= 1.05, frames++)
+		if(!lists_fit(low, 0u, (uint32_t)p, cap)) {
+			overflows++;
+			cap = grown_list_cap(low, (uint32_t)p, cap);
+			if(!lists_fit(low, 0u, (uint32_t)p, cap))
+				return 1;
+		}
+	printf("%d %d\n", frames, overflows);
+}
+"""
+
+
+def test_a_growing_scene_overflows_seldom(compile_and_run):
+    """Doubling: at most one overflow for every factor of two, log2(300) of them."""
+    out = compile_and_run(GROWING)
+    frames, overflows = map(int, out.stdout.split())
+    assert out.returncode == 0 and frames > 100 and 0 < overflows <= 9

@@ -3376,15 +3376,19 @@ __global__ __launch_bounds__(kFallbackThreads) void bwd_fallback_kernel(FrameCon
 // Row generation of small frames (kFusedRasterBins) in one launch, where two would each end with
 // a nearly empty chip (767 x 431 particles 33 + gap -> 24 us, 1280 x 720 lit mesh 49 + gap -> 44);
 // larger ones fill it and do better apart, with the high bins' smaller groups (1440p mesh 310 us
-// apart, 350 in one launch).
-static void launch_rowgen(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
+// apart, 350 in one launch). Timed frames take two launches at every size, with `after_low` (if not
+// null) recorded between them.
+static void launch_rowgen(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
+						  hipEvent_t *after_low = nullptr) {
 	constexpr int kHigh = kRowgenSplitThreads / kRowgenThreads, kHighFused = kRowgenSplitThreads / kRowgenLowThreads;
-	if(c.bin_count <= kFusedRasterBins) {
+	if(c.bin_count <= kFusedRasterBins && !after_low) {
 		hipLaunchKernelGGL(rowgen_fused_kernel, dim3(c.bin_count * (kHighFused + 1)), dim3(kRowgenLowThreads),
 						   0, stream, c, b);
 		return;
 	}
 	hipLaunchKernelGGL(rowgen_low_kernel, dim3(c.bin_count), dim3(kRowgenLowThreads), 0, stream, c, b);
+	if(after_low)
+		(void)hipEventRecord(*after_low, stream);
 	hipLaunchKernelGGL(rowgen_high_kernel, dim3(c.bin_count * kHigh), dim3(kRowgenThreads), 0, stream, c, b);
 }
 
@@ -3454,9 +3458,7 @@ template <bool FP32, int MODE>
 static void launch_raster_t(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 							hipEvent_t *ev) {
 	constexpr bool TEX = is_textured(MODE);
-	launch_rowgen(c, b, stream);
-	if(ev)
-		(void)hipEventRecord(ev[0], stream);
+	launch_rowgen(c, b, stream, ev); // (ev[0] between low and high bins)
 	launch_high_finalize(c, b, stream);
 	if(ev)
 		(void)hipEventRecord(ev[1], stream);
@@ -3508,8 +3510,8 @@ hipError_t launch_raster_batch(const BatchPlan &p, hipStream_t stream) {
 	return hipGetLastError();
 }
 
-// events (optional, 4): after the row generation, after the sorting of long block lists,
-// after block rasterisation, after the fallback kernel.
+// events (optional, 4): after the row generation of low bins, after that of high bins and the
+// sorting of long block lists, after block rasterisation, after the fallback kernel.
 hipError_t launch_raster(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 						 hipEvent_t *events) {
 	// frames with albedo textures take kernels built with the texture path (the others carry
@@ -3564,9 +3566,7 @@ static void launch_pass_a(const FrameConst &c, const FrameBufs &b, const BwdBufs
 // (which then render only what the recording pass does not).
 hipError_t launch_raster_recording(const FrameConst &c, const FrameBufs &b, const BwdBufs &g,
 								   hipStream_t stream, hipEvent_t *ev) {
-	launch_rowgen(c, b, stream);
-	if(ev)
-		(void)hipEventRecord(ev[0], stream);
+	launch_rowgen(c, b, stream, ev); // (ev[0] between low and high bins)
 	launch_high_finalize(c, b, stream);
 	hipLaunchKernelGGL(grad_row_scan_kernel<false>, dim3(1), dim3(1024), 0, stream, c, b, g);
 	hipLaunchKernelGGL(record_gate_kernel, dim3(1), dim3(64), 0, stream, b, g);

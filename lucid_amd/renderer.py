@@ -267,7 +267,6 @@ class LucidRenderer:
                                              aabb.ctypes.data, num_quads), "lucid_read_setup")
         return recs, aabb
 
-    # "rowgen_low" is the row generation of every bin, "rowgen_high_sort" the sort of long lists
     STAGES = ("setup", "binning", "rowgen_low", "rowgen_high_sort", "block_raster", "fallback")
 
     def stage_times(self) -> dict:

@@ -111,3 +111,34 @@ def test_batch_of_mixed_frames_keeps_the_threshold_wide(other):
     for a, b in zip(images[1], images[4]):
         for k in a:
             assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("blend", [0, _lib.OPT_ADDITIVE_BLENDING])
+@pytest.mark.parametrize("kind", ["bytes", "textured"])
+def test_two_slots_send_pixels_to_the_exact_sort(kind, blend):
+    """General and textured records in register-sorted blocks: two slots cannot order every pixel
+    here, four order more of them, and the bits are the same."""
+    if kind == "bytes":
+        sc = _planes(90, 72, 56, 0.25, (0.01, 0.1), seed=8, color_format="rgba8")
+    else:
+        sc = scenes.textured_planes(150, 97, 60, seed=7)
+    (a,), narrow = _render(sc, blend, 1)
+    (b,), wide = _render(sc, blend, 4)
+    assert narrow["fallback_pixels"] > wide["fallback_pixels"]
+    for k in a:
+        assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("kind", ["bytes", "textured"])
+def test_threshold_of_general_records(oracle_mod, kind):
+    """The alpha threshold with the default (narrow) tuning on general and textured records: counts
+    as in the oracle's exact frame, colours within the skipped remainder (below 1/128 per channel)
+    and the 1/255 quantisation."""
+    if kind == "bytes":
+        sc = scenes.config0(num_tris=20000, width=128, height=128, seed=42, color_format="rgba8")
+    else:
+        sc = scenes.textured_planes(150, 97, 90, seed=9)
+    (got,), _ = _render(sc, _lib.OPT_ALPHA_THRESHOLD, 1)
+    ref = oracle_mod.render(sc)
+    assert np.array_equal(got["frag_counts"].astype(np.uint32), ref["frag_counts"])
+    assert np.abs(got["image"].astype(int) - ref["image"].astype(int)).max() <= 3

@@ -36,7 +36,6 @@ enum CtrlWord : int {
 	kCtrlSpillCursor = 4,   // bump allocator of the deep-pixel spill pool (u64 units)
 	kCtrlTotalBinQuads = 5,
 	kCtrlTotalBinTris = 6,  // kBinListsWrapped: more list positions than 32 bits count
-	kCtrlFallbackPixels = 7,
 	kCtrlListCursor = 8,    // list positions of high bins (list_space.h): the space the frame needs
 	kCtrlOverflowCarry = 9, // overflow bits of earlier frames not yet seen by the host
 	kCtrlSortedCursor = 10, // pre-sorted pool size a frame needed, after an overflow (u32 units)

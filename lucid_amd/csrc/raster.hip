@@ -2526,12 +2526,10 @@ __device__ __forceinline__ void fallback_kernel_body(const FrameConst &c, const 
 	const uint32_t busy = min(wg.count, (nq + kFallbackThreads / 64 - 1) / (kFallbackThreads / 64));
 	if(nq ? wg.id >= busy || !last_work_group(b.ctrl, kDoneFallback, wg.id, busy) : wg.id != 0)
 		return;
-	if(nq && threadIdx.x == 0) {
-		agent_store(&b.ctrl[kCtrlFallbackPixels], nq);
-		// stats[2]: pixels resolved by the exact per-pixel sort (the reference counts the
-		// pixels its 3-deep window gets wrong there, shading.glsl:258-265)
+	// stats[2]: pixels resolved by the exact per-pixel sort (the reference counts the pixels its
+	// 3-deep window gets wrong there, shading.glsl:258-265)
+	if(nq && threadIdx.x == 0)
 		((lucid_info *)b.info)->stats[2] = nq;
-	}
 	// The control words go to pinned host memory, where the host reads them once the frame's
 	// event has completed (a copy command of 64 bytes: 4 us of the GPU, and its submission).
 	if(b.host_status && threadIdx.x < (uint32_t)kCtrlWords)

@@ -75,13 +75,12 @@ typedef struct lucid_tuning {
 	int slice_words;      /* entries staged in LDS per step: 64 * slice_words (1 or 2) */
 	int presort_min;      /* high-bin blocks with more entries are pre-sorted (64..256) */
 	int samples_per_wave; /* target samples per wave of a pre-sorted block (256..65536) */
-	int window;           /* per-pixel ordering window of the block rasterisers and of the
-						   * backward's first pass: 1 (one slot; two for lit, textured or
-						   * byte-coloured samples and in the backward) for lists whose block
-						   * order is nearly every pixel's depth order, 4 for more disorder
-						   * (and, whatever this says, for such samples with the alpha
-						   * threshold). A pixel the window cannot order takes the exact
-						   * per-pixel sort either way. */
+	int window;           /* per-pixel ordering window of the block rasterisers in frames of
+						   * RGBA8 samples with unit lighting and flat colours, and of the
+						   * backward's first pass: 1 (one slot; two in the backward) for
+						   * lists whose block order is nearly every
+						   * pixel's depth order, 4 for more disorder. A pixel the window
+						   * cannot order takes the exact per-pixel sort either way. */
 } lucid_tuning;
 
 typedef struct lucid_create_info {

@@ -164,7 +164,7 @@ struct FrameConst {
 	uint32_t presort_min;      // high-bin blocks with more entries are pre-sorted (<= kRegSortCap)
 	uint32_t samples_per_wave; // target samples per wave of a pre-sorted block
 	int slice_words;           // block rasteriser slice width: 1 or 2 words of 64 entries
-	int window;                // ordering window (tuning): 1 (narrow) or 4
+	int window;                // ordering window (tuning) of flat-colour frames and pass A: 1 or 4
 	int color_mode;
 	int has_normals;
 	// 1 when an earlier frame of the renderer may still be running: the clear kernel then
@@ -327,23 +327,17 @@ __device__ __forceinline__ uint32_t batch_frame(const StageBatch &sb, uint32_t w
 // of the pixel divided by the inverse depth).
 // kShadePlain: the same frames with fp32 samples whose instances all have fp32 vertex colours
 // and no instance colour (the general shading's values, without its tests).
-// kShadeNarrow (a flag): narrow ordering windows (tuning window 1).
+// kShadeNarrow (a flag): flat records with the narrow ordering window (tuning window 1).
 enum ShadeMode : int { kShadeGeneral = 0, kShadeTextured = 1, kShadeFlat = 2, kShadePlain = 3, kShadeNarrow = 4 };
 
-// Whether a frame may take the narrow windows with records of this kind. The alpha threshold looks
-// at the samples that have left the window, so its results depend on the slots: only flat records
-// take it with the narrow ones.
-inline bool narrow_windows(const FrameConst &c, int kind) {
-	return c.window == 1 && (kind == kShadeFlat || !(c.opts & LUCID_OPT_ALPHA_THRESHOLD));
-}
-
 inline int frame_shade_mode(const FrameConst &c) {
-	const bool fp32 = (c.opts & LUCID_OPT_FP32_SAMPLES) != 0;
-	const bool flat_colors = c.color_mode == kColorNone || c.color_mode == kColorF32;
-	const int kind = c.has_textures ? kShadeTextured
-					 : fp32 ? (c.plain_colors ? kShadePlain : kShadeGeneral)
-							: (c.identity_light && flat_colors ? kShadeFlat : kShadeGeneral);
-	return kind | (narrow_windows(c, kind) ? kShadeNarrow : 0);
+	if(c.has_textures)
+		return kShadeTextured;
+	if(c.opts & LUCID_OPT_FP32_SAMPLES)
+		return c.plain_colors ? kShadePlain : kShadeGeneral;
+	if(!c.identity_light || !(c.color_mode == kColorNone || c.color_mode == kColorF32))
+		return kShadeGeneral;
+	return kShadeFlat | (c.window == 1 ? kShadeNarrow : 0);
 }
 
 struct BatchPlan {

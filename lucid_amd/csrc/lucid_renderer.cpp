@@ -1241,12 +1241,10 @@ int lucid_batch_render(lucid_batch *bt, const lucid_frame_inputs *ins,
 	plan.num_frames = (uint32_t)n;
 	plan.bin_lds = bin_lds;
 	plan.fp32 = (bt->rs[0]->opts & LUCID_OPT_FP32_SAMPLES) != 0;
-	// (one sample format: fast frames are all flat or all plain)
+	// one sample format: fast frames are all flat, with the first renderer's window (a tuning
+	// knob), or all plain. A flat frame among others takes their records and their four slots.
 	plan.mode = tex ? kShadeTextured : fast ? fast_mode : kShadeGeneral;
-	// narrow windows if every frame may take them with the records that the batch has in the end
-	// (a flat frame with the alpha threshold may not among general or textured ones)
-	const int kind = plan.mode;
-	if(std::all_of(frames.begin(), frames.end(), [&](const FrameDesc &f) { return narrow_windows(f.c, kind); }))
+	if(plan.mode == kShadeFlat && bt->rs[0]->tuning.window == 1)
 		plan.mode |= kShadeNarrow;
 	plan.slice_words = bt->rs[0]->tuning.slice_words;
 	// the launches read the frames' constants and buffers from device memory, so a frame

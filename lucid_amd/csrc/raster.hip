@@ -29,12 +29,12 @@ namespace lucid {
 constexpr int kSortThreads = 256;
 constexpr int kFallbackThreads = 256;
 constexpr int kWindow = 4;
-// Narrow ordering windows (tuning window 1): one slot for flat and plain records, in the
-// register-sorted blocks and in the pre-sorted ones (whose depth ranks keep 32 - log2 of the padded
-// list length bits); two for the general records of register-sorted blocks, where a pixel sent to
-// the exact sort costs more (4 -> 2 slots: 1280 x 720 lit mesh 98 -> 83 us, textured planes 254 ->
-// 237). The fp32 soup of 41 M fragments at 512 x 512: four slots 178 us, two 138, one 121.
-constexpr int kNarrowWindow = 1, kNarrowPlainWindow = 1, kNarrowGeneralWindow = 2;
+// The narrow ordering window (tuning window 1) of flat records: one slot, in the register-sorted
+// blocks and in the pre-sorted ones (whose depth ranks keep 32 - log2 of the padded list length
+// bits). Other records keep four: where surfaces cross, fewer send too many pixels to the exact sort,
+// which costs them more (640 x 360, 250 crossing planes, four slots against one with plain records
+// and two with general ones: 465 against 2275 us a frame, 486 against 665).
+constexpr int kNarrowWindow = 1;
 constexpr int kFallbackCap = 512; // fragments per pixel sorted in LDS by the fallback kernel
 
 // ------------------------------------------------------------------ shading
@@ -544,16 +544,17 @@ struct OrderWindow {
 // window is a queue: k0 leaves, no key is compared with the last emitted one and nothing is
 // selected; the wave tests for that with one comparison. (A pending key is never before `last`: a
 // new key before k0 leaves at once, as the smallest.) Otherwise the wave takes the selects. The
-// walks are bound by VALU issue (75 -> 60 instructions
-// per flat sample): both block kernels of 1 M soup triangles at 1080p 203 -> 190 us, of the 32-frame
-// batch 1800 -> 1667, the fp32 soup's 121 -> 112.
-template <class P, int N, bool PH = (N == 1)>
+// walks are bound by VALU issue (75 -> 60 instructions per flat sample): both block kernels of 1 M
+// soup triangles at 1080p 203 -> 190 us, of the 32-frame batch 1800 -> 1650, pass A of the fp32
+// soup (41 M fragments at 512 x 512) 178 -> 160.
+template <class P, int N>
 struct SmallWindow {
 	static_assert(N == 1 || N == 2, "one or two slots");
+	static constexpr bool PH = N == 1;
 	// Free slots hold placeholders (key 0, below every sample key; a zero payload), which the first
-	// samples push out, so no fill count is kept. PH: they are emitted like samples, and the emit
-	// callback treats the zero payload as nothing (the forward blend does; the backward's order
-	// recording does not). The keys of one pixel are distinct (one sample per triangle).
+	// samples push out, so no fill count is kept. PH (the forward's one slot): they are emitted like
+	// samples, and the blend treats the zero payload as nothing; the backward's order recording (two
+	// slots) does not. The keys of one pixel are distinct (one sample per triangle).
 	uint64_t k0, k1;
 	P c0, c1;
 	uint64_t first, last; // first and last emitted key (0 before the first)
@@ -609,7 +610,7 @@ struct SmallWindow {
 // Forward per-pixel state: the ordering window (N slots) feeding the front-to-back blend.
 template <bool FP32, int N = kWindow>
 struct PixelState {
-	std::conditional_t<N == kWindow, OrderWindow<SampleColor<FP32>>, SmallWindow<SampleColor<FP32>, N, true>> w;
+	std::conditional_t<N == kWindow, OrderWindow<SampleColor<FP32>>, SmallWindow<SampleColor<FP32>, N>> w;
 	Accum acc;
 
 	__device__ __forceinline__ void init() {
@@ -1819,18 +1820,7 @@ constexpr int shade_kind(int mode) { return mode & ~kShadeNarrow; }
 constexpr bool is_flat(int mode) { return shade_kind(mode) == kShadeFlat; }
 constexpr bool is_plain(int mode) { return shade_kind(mode) == kShadePlain; }
 constexpr bool is_textured(int mode) { return shade_kind(mode) == kShadeTextured; }
-// Window slots of the register-sorted and the pre-sorted blocks. A pre-sorted pixel's depth ranges
-// are composited apart and then chained, which rounds differently from the exact sort: there the
-// general and plain kinds keep four slots, so that no pixel's bits change by the tuning, or from run
-// to run, with the exact sort that fewer slots would send it to. (Flat ones take one slot there,
-// which costs an RGBA8 byte now and then.)
-constexpr int window_slots(int mode, bool presorted) {
-	return !(mode & kShadeNarrow)		  ? kWindow
-		   : is_flat(mode)				  ? kNarrowWindow
-		   : presorted					  ? kWindow
-		   : is_plain(mode)				  ? kNarrowPlainWindow
-										  : kNarrowGeneralWindow;
-}
+constexpr int window_slots(int mode) { return mode & kShadeNarrow ? kNarrowWindow : kWindow; }
 constexpr int rec_quads(int mode) { return is_flat(mode) ? kFlatQuads : kRecQuads; }
 // LDS of one wave's slice of 64 W records
 template <int W, int MODE> constexpr int slice_quads() { return 64 * W * rec_quads(MODE); }
@@ -1896,9 +1886,8 @@ __device__ __forceinline__ SampleColor<false> shade_flat(const uint4 *f, float p
 // quads, the triangle id in place of the flags; still kRecQuads apart, as six quads would put
 // twice as many entries on one LDS bank) and evaluate the general shading without its tests of
 // instance flags and frame options: the same operations on the same values, bit for bit. These
-// kernels are bound by VALU issue: 41 M fragments at 512 x 512, forward raster 204 -> 121 us (with
-// the one-slot window), pass A 214 -> 179, pass B 534 -> 441 (with its eight rotated orders and
-// 12.5 KB of LDS instead of 15.5).
+// kernels are bound by VALU issue: 41 M fragments at 512 x 512, forward raster 204 -> 175 us, pass A
+// 214 -> 179, pass B 534 -> 441 (with its eight rotated orders and 12.5 KB of LDS instead of 15.5).
 constexpr int kPlainQuads = 6; // depth plane | triangle id; two barycentric planes; c0 | alpha; c1; c2
 
 struct PlainShade {
@@ -2157,7 +2146,7 @@ __device__ __forceinline__ void raster_sorted_block(const FrameConst &c, const F
 	}
 	const bool additive = (c.opts & (1u << 5)) != 0;
 	const bool threshold = alpha_threshold_on(c);
-	PixelState<FP32, window_slots(MODE, false)> ps;
+	PixelState<FP32, window_slots(MODE)> ps;
 	ps.init();
 	uint32_t count = 0;
 	bool opaque = false; // every pixel of the block is nearly opaque (alpha threshold)
@@ -2233,7 +2222,7 @@ __device__ __forceinline__ void raster_presorted_block(const FrameConst &c, cons
 	const bool additive = (c.opts & (1u << 5)) != 0;
 	if((uint32_t)wave < nw) {
 		const uint32_t e0 = hdr[1 + wave], e1 = hdr[2 + wave];
-		PixelState<FP32, window_slots(MODE, true)> ps;
+		PixelState<FP32, window_slots(MODE)> ps;
 		ps.init();
 		uint32_t count = 0;
 		const bool threshold = alpha_threshold_on(c);
@@ -2802,7 +2791,7 @@ __global__ __launch_bounds__(kBigWaves * 64) void bwd_pass_a_kernel(FrameConst c
 	const uint32_t row0 = g.row_base[slot];
 
 	if((uint32_t)wave < ent.nw) {
-		std::conditional_t<WIN == kWindow, OrderWindow<BwdColor>, SmallWindow<BwdColor, WIN, false>> w;
+		std::conditional_t<WIN == kWindow, OrderWindow<BwdColor>, SmallWindow<BwdColor, WIN>> w;
 		w.init();
 		BwdTotals part;
 		part.init();
@@ -3400,27 +3389,19 @@ static void launch_high_finalize(const FrameConst &c, const FrameBufs &b, hipStr
 
 // Calls f with the sample format and shading mode as compile-time constants.
 template <class F> static void with_shade_mode(bool fp32, int mode, F &&f) {
-	auto pick = [&](auto fmt, auto kind) {
-		if(mode & kShadeNarrow)
-			f(fmt, std::integral_constant<int, decltype(kind)::value | kShadeNarrow>{});
-		else
-			f(fmt, kind);
-	};
 	const std::integral_constant<int, kShadeGeneral> general;
 	const std::integral_constant<int, kShadeTextured> textured;
-	if(fp32) {
-		if(shade_kind(mode) == kShadePlain)
-			pick(std::true_type{}, std::integral_constant<int, kShadePlain>{});
-		else if(is_textured(mode))
-			pick(std::true_type{}, textured);
-		else
-			pick(std::true_type{}, general);
-	} else if(is_flat(mode))
-		pick(std::false_type{}, std::integral_constant<int, kShadeFlat>{});
-	else if(is_textured(mode))
-		pick(std::false_type{}, textured);
+	const std::integral_constant<int, kShadePlain> plain;
+	const std::integral_constant<int, kShadeFlat> flat;
+	const std::integral_constant<int, kShadeFlat | kShadeNarrow> flat_narrow;
+	const std::true_type f32;
+	const std::false_type bytes;
+	if(fp32)
+		mode == kShadePlain ? f(f32, plain) : is_textured(mode) ? f(f32, textured) : f(f32, general);
+	else if(is_flat(mode))
+		mode & kShadeNarrow ? f(bytes, flat_narrow) : f(bytes, flat);
 	else
-		pick(std::false_type{}, general);
+		is_textured(mode) ? f(bytes, textured) : f(bytes, general);
 }
 
 template <bool FP32, int W, int MODE>

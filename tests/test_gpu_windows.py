@@ -1,7 +1,6 @@
 """The ordering windows decide only which pixels take the exact sort, never a result: fp32 frames
-whose blocks are pre-sorted (their depth ranges are composited apart and chained), narrow windows
-of general and textured records where pixels do reach the exact sort, and batches that mix frames
-with and without the alpha threshold."""
+whose blocks are pre-sorted (their depth ranges are composited apart and chained), the window knob
+on records that are not flat, and batches that mix frames with and without the alpha threshold."""
 
 import numpy as np
 import pytest
@@ -114,17 +113,20 @@ def test_batch_of_mixed_frames_keeps_the_threshold_wide(other):
 
 
 @pytest.mark.parametrize("blend", [0, _lib.OPT_ADDITIVE_BLENDING])
-@pytest.mark.parametrize("kind", ["bytes", "textured"])
-def test_two_slots_send_pixels_to_the_exact_sort(kind, blend):
-    """General and textured records in register-sorted blocks: two slots cannot order every pixel
-    here, four order more of them, and the bits are the same."""
-    if kind == "bytes":
-        sc = _planes(90, 72, 56, 0.25, (0.01, 0.1), seed=8, color_format="rgba8")
-    else:
+@pytest.mark.parametrize("kind", ["bytes", "textured", "fp32"])
+def test_the_window_knob_is_for_flat_records(kind, blend):
+    """Byte-coloured, textured and fp32 frames, whose surfaces cross: the narrow tuning sends no
+    more of their pixels to the exact sort, and none when four slots can order them."""
+    opts = blend
+    if kind == "textured":
         sc = scenes.textured_planes(150, 97, 60, seed=7)
-    (a,), narrow = _render(sc, blend, 1)
-    (b,), wide = _render(sc, blend, 4)
-    assert narrow["fallback_pixels"] > wide["fallback_pixels"]
+    else:
+        sc = _planes(90, 72, 56, 0.25, (0.01, 0.1), seed=8, color_format="rgba8" if kind == "bytes" else "f32")
+        opts |= _lib.OPT_FP32_SAMPLES if kind == "fp32" else 0
+    (a,), narrow = _render(sc, opts, 1)
+    (b,), wide = _render(sc, opts, 4)
+    assert narrow["fallback_pixels"] == wide["fallback_pixels"]
+    assert kind == "textured" or wide["fallback_pixels"] == 0
     for k in a:
         assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), k
 

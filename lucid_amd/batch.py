@@ -2,9 +2,9 @@
 recorded into one hipGraph and launched at once (lucid_batch_* in include/lucid_c.h).
 
 The reference renders one scene per frame (src/lucid_renderer.cpp:319-350); this is the
-batch extension of the same forward. Frames are spread over forked streams inside the
-graph so that small scenes run side by side; the graph is recorded again only when a
-frame's constants or buffers change.
+batch extension of the same forward. Every pipeline stage is one launch for all frames, so
+that small scenes run side by side; the launches read the frames' constants and buffers from
+device memory, and the graph is recorded again only when a grid or a choice of kernels changes.
 """
 
 from __future__ import annotations

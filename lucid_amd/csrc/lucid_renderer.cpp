@@ -64,7 +64,7 @@ namespace {
 constexpr int kMaxWidth = 2560, kMaxHeight = 2048;   // src/lucid_renderer.h:27
 constexpr int kMaxInstances = 64 * 1024;            // src/lucid_renderer.h:28
 constexpr int64_t kMaxQuads = (int64_t)1 << 28;     // quad ids share a word with 4 flag bits
-constexpr uint64_t kAsideTris = 1u << 16; // triangles from which the backward uses the helper stream
+constexpr uint64_t kAsideTris = 1u << 16; // the backward uses the helper stream beyond so many triangles
 constexpr int kNumBinWgs = 256; // bin_wg_scan_kernel assumes at most 256 (16 rows per part)
 
 struct DevBuf {
@@ -903,7 +903,10 @@ int lucid_backward_ex(lucid_renderer *r, const lucid_frame_inputs *in, const flo
 	// check beside pass A, then the row grouping beside pass B (which needs the scale). Pass A is
 	// submitted first: the GPU would otherwise wait for the host to submit the helper stream's work
 	// before it. Small ones take one stream: what could overlap is shorter than the events are to
-	// submit (10 k triangles at 200 x 136: 317 -> 299 us a step).
+	// submit (4 k triangles at 200 x 200: the backward 185 -> 107 us, 32 k 179 -> 144). The line is a
+	// compromise, as pass B's share grows with the pixels: at 200 x 200 one stream is the better one
+	// up to 96 k triangles (189 -> 171 us; 140 k: 187 -> 206), at 512 x 512 up to 4 k (16 k to 66 k:
+	// 3 to 5 % slower, 337 -> 349 us at 48 k; 400 k: 727 -> 786).
 	const bool aside = ntri > kAsideTris;
 	const hipStream_t aux = aside ? r->aux : stream;
 	if(aside)

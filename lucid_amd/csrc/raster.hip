@@ -4,15 +4,18 @@
 // Kernels (wave64; an 8x8 block of pixels is one wave, one lane per pixel):
 //   rowgen_low   one work-group per bin with fewer than 1024 triangles: block lists with the
 //                reference's 8-row scanline rule; promotes the bin to the high path when an 8x8
-//                block holds more than 256 triangles (raster_low.glsl:39-106,229-237).
-//   rowgen_high  eight work-groups per high bin: block lists with the 4-row rule of
-//                raster_high.glsl:54-90.
-//   high_prep / high_finalize  allocation for high bins; long block lists are sorted by
-//                centroid depth (LDS bitonic, whole work-group) and split into depth ranges so
-//                that several waves share a dense block.
+//                block holds more than 256 triangles (raster_low.glsl:39-106,229-237), and
+//                generates it again as a high bin.
+//   rowgen_high  kRowgenSplitThreads threads per high bin (eight work-groups, or four larger ones
+//                in the launch that takes low and high bins, rowgen_fused): block lists with the
+//                4-row rule of raster_high.glsl:54-90. (Their space is the bin categories' work.)
+//   high_finalize  long block lists of high bins are sorted by centroid depth (bitonic, in
+//                registers and LDS, whole work-group) and split into depth ranges so that several
+//                waves share a dense block; lists beyond 2048 entries in high_finalize_long.
 //   block_raster one wave per block: sorts short lists itself in registers, turns the coverage
 //                masks into per-pixel entry bitmaps, shades and blends front to back; pre-sorted
-//                blocks take one wave per depth range.
+//                blocks take one wave per depth range (block_raster_big; both kinds in one launch:
+//                block_raster_fused).
 //   fallback     exact per-pixel sort for pixels whose speculative order was violated.
 //
 // Exact ordering: triangles of a block are pre-sorted by the depth at their covered-pixel
@@ -1382,8 +1385,8 @@ __device__ __forceinline__ uint32_t sorted_mask_offset(uint32_t m) {
 
 // Finalises every block of the high bins: copies the list lengths into the slot table and
 // pre-sorts long lists. A long list is sorted once by centroid depth (LDS bitonic by the
-// whole work-group) and split into `parts` pixel-row groups, each a compacted list of the
-// entries that cover it, so that several waves can rasterise a dense block.
+// whole work-group) and split into contiguous depth ranges of about equal sample counts, so that
+// several waves can rasterise a dense block.
 // A work-group is a chain of memory and LDS latencies (VALU busy 0.4), so the loads that decide its
 // early exits are made together, the pool is asked for while the entries load, and a list of up to
 // 256 keys is sorted by all four waves: 32-frame batch 506 -> 471 us, 5.2 M mesh triangles 192 ->
@@ -2337,11 +2340,10 @@ __global__ __launch_bounds__(kBigWaves * 64) void block_raster_big_kernel_batch(
 	block_raster_big_body<FP32, W, MODE>(d.c, d.b, wg - sb.pre[f]);
 }
 
-// Both kinds in one launch, for frames of few blocks (kFusedRasterBins): the first 16 work-groups
+// Both kinds in one launch, for frames of few blocks (launch_block_raster): the first 16 work-groups
 // per bin take the pre-sorted blocks, the others four register-sorted blocks each (one wave a
 // block, on its own quarter of the LDS), which fill the CUs that run out of the long ones. As two
 // launches each ends with a nearly empty chip. fp32 samples: four waves per SIMD, as apart.
-constexpr int kFusedRasterBins = 1024;
 static_assert(kBigWaves == 4, "a bin's 16 blocks are four work-groups of register-sorted blocks");
 template <bool FP32, int MODE>
 __global__ __launch_bounds__(kBigWaves * 64, FP32 ? 4 : 1) void block_raster_fused_kernel(FrameConst c, FrameBufs b) {
@@ -3360,15 +3362,24 @@ __global__ __launch_bounds__(kFallbackThreads) void bwd_fallback_kernel(FrameCon
 		bwd_fallback_pixel(c, b, g, b.fallback_queue[qi], s_keys[threadIdx.x >> 6]);
 }
 
-// Row generation of small frames (kFusedRasterBins) in one launch, where two would each end with
-// a nearly empty chip (767 x 431 particles 33 + gap -> 24 us, 1280 x 720 lit mesh 49 + gap -> 44);
-// larger ones fill it and do better apart, with the high bins' smaller groups (1440p mesh 310 us
-// apart, 350 in one launch). Timed frames take two launches at every size, with `after_low` (if not
-// null) recorded between them.
+// Row generation of small frames in one launch, where two would each end with a nearly empty chip
+// (767 x 431 particles 33 + gap -> 24 us, 1280 x 720 lit mesh 49 + gap -> 44); large ones fill it
+// and do better apart, with the high bins' smaller groups (1440p mesh 310 us apart, 350 in one
+// launch). The line: whole frames of the same scene kinds at ten sizes, one launch against two, us.
+//   bins                    520   1024   1435   2040   2800   3600
+//   clustered triangles    +4.6   -3.7   -3.3  -13.7  -24.5  +14.6
+//   byte-coloured ones     -7.6  -11.4   -6.4   -3.8   +3.7   +8.4
+//   fp32 samples           -6.7  -11.2   -7.7   -3.2   +2.7   +8.7
+//   384 spheres            -5.3   -3.5   -2.0   -1.6   -0.6   +1.8
+//   20 k small triangles   -1.5   -0.3   +1.3   -0.1   +1.0   +1.6
+// So the kinds part between 1400 and 3600 bins; up to 1024 one launch is not worse but for +5 of
+// 300 us at one size. Timed frames take two launches at every size, with `after_low` (if not null)
+// recorded between them.
+constexpr int kFusedRowgenBins = 1024;
 static void launch_rowgen(const FrameConst &c, const FrameBufs &b, hipStream_t stream,
 						  hipEvent_t *after_low = nullptr) {
 	constexpr int kHigh = kRowgenSplitThreads / kRowgenThreads, kHighFused = kRowgenSplitThreads / kRowgenLowThreads;
-	if(c.bin_count <= kFusedRasterBins && !after_low) {
+	if(c.bin_count <= kFusedRowgenBins && !after_low) {
 		hipLaunchKernelGGL(rowgen_fused_kernel, dim3(c.bin_count * (kHighFused + 1)), dim3(kRowgenLowThreads),
 						   0, stream, c, b);
 		return;
@@ -3412,11 +3423,19 @@ static void launch_block_raster_apart(const FrameConst &c, const FrameBufs &b, h
 					   dim3(kBigWaves * 64), 0, stream, c, b);
 }
 
-// Frames of up to kFusedRasterBins bins take one launch (two -> one: 767 x 431 particles 336
-// bins, 79 -> 64 us; 1280 x 720 lit mesh, 920 bins, 104 -> 99 us; 512 x 512 preview, 18 -> 15 us).
-// Larger ones fill the chip either way, and the register-sorted blocks are better off as
-// work-groups of their own (1080p soup, 2040 bins, 198 -> 199 us; 1440p mesh, 3600 bins, 336 ->
-// 365 us), as are textured ones, whose blocks differ most in length (768 bins, 261 -> 269 us).
+// Small frames take one launch (two -> one: 767 x 431 particles, 336 bins, 79 -> 64 us; 1280 x 720
+// lit mesh, 920 bins, 104 -> 99 us; 512 x 512 preview, 18 -> 15 us). Large ones fill the chip either
+// way, and the register-sorted blocks are better off as work-groups of their own (1440p mesh, 3600
+// bins, 336 -> 365 us), as are textured ones, whose blocks differ most in length (768 bins, 261 ->
+// 269 us). The line: whole frames as above, one launch against two, us.
+//   bins                    520   1024   1435   1750   2040   2800
+//   clustered triangles   -25.4  -29.5  -25.5  -15.9  -11.0   -5.6
+//   byte-coloured ones    -28.2  -17.0   -1.4   +4.9  +14.1  +24.7
+//   fp32 samples          -23.3  -12.8   -4.0   -0.3   +2.7   +9.9
+//   384 spheres            -7.1   -5.5   -4.1   -2.3   -0.6   +2.4
+//   20 k small triangles   -1.0   -0.5   -0.9   -0.6   -0.6   -0.1
+// The first kind turns between 1435 and 1750 bins, the last beyond 2800; up to 1024 all gain.
+constexpr int kFusedRasterBins = 1024;
 template <bool FP32, int MODE>
 static void launch_block_raster(const FrameConst &c, const FrameBufs &b, hipStream_t stream) {
 	if constexpr(!is_textured(MODE)) {
